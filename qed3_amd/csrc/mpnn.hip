@@ -309,23 +309,37 @@ __global__ __launch_bounds__(256) void k_net_out(NetGeo g, const bf16* __restric
 }
 
 // ---------------------------------------------------------------- backward kernels
-// loss pieces: per pair |e|^2 and |out - e|^2
+// Loss pieces of each pair, |e|^2 and |out - e|^2: nbp blocks stride over each pair's points
+// and leave one FP64 partial each, k_net_loss_sum adds a pair's partials.  (One atomicAdd
+// pair per point into two doubles serialised the whole field there: 7.9 ms for 4 fields of
+// 81,920 points, now 0.01 ms.)
 __global__ __launch_bounds__(256) void k_net_loss(const Spin<float>* __restrict__ out,
-                                                  const Spin<float>* __restrict__ e, size_t np,
-                                                  size_t per, double* acc) {
-  const size_t P = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  double en = 0, dn = 0;
-  int b = -1;
-  if (P < np) {
-    const Spin<float> o = out[P], t = e[P];
-    en = double(t.a.x) * t.a.x + double(t.a.y) * t.a.y + double(t.b.x) * t.b.x + double(t.b.y) * t.b.y;
+                                                  const Spin<float>* __restrict__ e, size_t per, unsigned nbp,
+                                                  double2* __restrict__ partials) {
+  const unsigned b = blockIdx.x / nbp, k = blockIdx.x - b * nbp;
+  const size_t P0 = size_t(b) * per;
+  double2 acc = {0.0, 0.0};
+  for (size_t i = size_t(k) * blockDim.x + threadIdx.x; i < per; i += size_t(nbp) * blockDim.x) {
+    const Spin<float> o = out[P0 + i], t = e[P0 + i];
+    acc.x += double(t.a.x) * t.a.x + double(t.a.y) * t.a.y + double(t.b.x) * t.b.x + double(t.b.y) * t.b.y;
     const double d0 = o.a.x - t.a.x, d1 = o.a.y - t.a.y, d2 = o.b.x - t.b.x, d3 = o.b.y - t.b.y;
-    dn = d0 * d0 + d1 * d1 + d2 * d2 + d3 * d3;
-    b = int(P / per);
+    acc.y += d0 * d0 + d1 * d1 + d2 * d2 + d3 * d3;
   }
-  if (b >= 0) {
-    atomicAdd(acc + 2 * b, en);
-    atomicAdd(acc + 2 * b + 1, dn);
+  store_partial(acc, partials, blockIdx.x);
+}
+
+__global__ __launch_bounds__(256) void k_net_loss_sum(const double2* __restrict__ partials, unsigned n,
+                                                      double* __restrict__ acc) {
+  double2 s = {0.0, 0.0};
+  for (unsigned i = threadIdx.x; i < n; i += blockDim.x) {
+    const double2 p = partials[size_t(blockIdx.x) * n + i];
+    s.x += p.x;
+    s.y += p.y;
+  }
+  const double2 t = block_sum2(s);
+  if (threadIdx.x == 0) {
+    acc[2 * blockIdx.x] = t.x;
+    acc[2 * blockIdx.x + 1] = t.y;
   }
 }
 
@@ -344,60 +358,72 @@ __global__ __launch_bounds__(256) void k_net_gout(const Spin<float>* __restrict_
   gout[P] = gg;
 }
 
-// Output head backward: A_k = F_k^dagger gout.  Input spin a of F_k feeds output spin
-// o_k(a) = a (k != 2) or 1 - a (k = 2, the gamma map), so dh[c,a] = sum_k conj(u[o_k(a)][k][c])
-// A_k,a and du[o][k][c] = A_k,a conj(h_c,a) with o = o_k(a) (per-point contributions,
-// summed by k_colsum).
-__global__ __launch_bounds__(256) void k_net_out_bwd(NetGeo g, const Spin<float>* __restrict__ gout,
-                                                     const bf16* __restrict__ h,
-                                                     const float2* __restrict__ u,
-                                                     float* __restrict__ dh, float* __restrict__ contrib) {
-  const size_t P = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (P >= g.np) return;
-  float2 A[5][2];
-  feat1<true>(g, gout, P, A);
-  for (int c = 0; c < C; c++) {
-    for (int a = 0; a < 2; a++) {
-      float2 z = {0.f, 0.f};
-      for (int k = 0; k < 5; k++) cadd_(z, cmc(u[((k == 2 ? 1 - a : a) * 5 + k) * C + c], A[k][a]));
-      dh[(P * 2 + a) * RW + 2 * c] = z.x;
-      dh[(P * 2 + a) * RW + 2 * c + 1] = z.y;
+// Gradient of a head: sums over points of the products of the ten feature components of a
+// single-channel field with the 32 channel components of a C-channel one,
+//   output head (OUT): du[o][k][c] = sum_P A_k,a conj(h_c,a), A_k = F_k^dagger gout, input spin
+//     a of F_k feeding output spin o = a (k != 2) or 1 - a (k = 2, the gamma map);
+//   input head: dv[a][k][c] = sum_P dh_c,a conj(F_k(r)_a);
+// and, for the output head, dh[c,a] = sum_k conj(u[o_k(a)][k][c]) A_k,a.
+// A block walks groups of 256 points: one thread per point forms the features and leaves them
+// in LDS; then the threads turn into (spin, channel) columns for dh, whose rows they write
+// whole, and into the 160 (spin, map, channel) sums, each an FP64 accumulator kept over the
+// block's groups and stored once (partial[block][160]).  The form before wrote all 160
+// products of every point (1.25 KB) and summed them column by column in another kernel:
+// 0.83 (output head) and 0.39 ms (input head) plus 0.9 ms a sum at 4 x 81,920 points; this
+// takes 0.067 and 0.054 ms plus 0.008 ms.
+constexpr int kHeadCols = 10 * C;  // complex sums of a head gradient
+template <bool OUT>
+__global__ __launch_bounds__(256) void k_net_head_bwd(NetGeo g, const Spin<float>* __restrict__ f,
+                                                      const bf16* __restrict__ h, const float2* __restrict__ u,
+                                                      float* __restrict__ dh, double2* __restrict__ partial) {
+  __shared__ float2 Fs[10][256 + 1];  // [2 k + a][point]; the pad spreads the columns' writes
+  const int t = threadIdx.x;
+  const int c = t & (C - 1), ka = t >> 4;  // the sum this thread keeps (t < kHeadCols)
+  const int sk = ka >> 1, sa = ka & 1;
+  double2 acc = {0.0, 0.0};
+  for (size_t P0 = size_t(blockIdx.x) * 256; P0 < g.np; P0 += size_t(gridDim.x) * 256) {
+    const int cnt = int(g.np - P0 < 256 ? g.np - P0 : 256);
+    if (t < cnt) {
+      float2 F[5][2];
+      feat1<OUT>(g, f, P0 + t, F);
+#pragma unroll
+      for (int k = 0; k < 5; k++)
+#pragma unroll
+        for (int a = 0; a < 2; a++) Fs[2 * k + a][t] = F[k][a];
     }
-    if (!contrib) continue;  // adjoint apply: no weight gradient
-    float* cdst = contrib + P * (20 * C);
-    float2 hc[2];
-    for (int a = 0; a < 2; a++) {
-      const bf16* src = h + (P * 2 + a) * RW + 2 * c;
-      hc[a] = {float(src[0]), float(src[1])};
-    }
-    for (int a = 0; a < 2; a++)
-      for (int k = 0; k < 5; k++) {
-        const int o = k == 2 ? 1 - a : a;
-        const float2 z = cmc(hc[a], A[k][a]);
-        cdst[2 * ((o * 5 + k) * C + c)] = z.x;
-        cdst[2 * ((o * 5 + k) * C + c) + 1] = z.y;
+    __syncthreads();
+    if constexpr (OUT) {
+      const int a = (t >> 4) & 1;
+      float2 uk[5];
+#pragma unroll
+      for (int k = 0; k < 5; k++) uk[k] = u[((k == 2 ? 1 - a : a) * 5 + k) * C + c];
+      float2* row = reinterpret_cast<float2*>(dh) + P0 * RW + (t & (RW - 1));
+      for (int p = t >> 5; p < cnt; p += 8) {
+        float2 z = {0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 5; k++) cadd_(z, cmc(uk[k], Fs[2 * k + a][p]));
+        row[size_t(p) * RW] = z;
       }
+    }
+    if (t < kHeadCols) {
+      for (int p = 0; p < cnt; p++) {
+        const float2 x = Fs[ka][p];
+        float2 z;
+        if constexpr (OUT) {
+          const bf16* src = h + ((P0 + p) * 2 + sa) * RW + 2 * c;
+          z = cmc(float2{float(src[0]), float(src[1])}, x);
+        } else {
+          const float2 y = reinterpret_cast<const float2*>(dh)[((P0 + p) * 2 + sa) * C + c];
+          z = cmc(x, y);
+        }
+        acc.x += double(z.x);
+        acc.y += double(z.y);
+      }
+    }
+    __syncthreads();
   }
-}
-
-// Input head backward: contributions to dv[a][k][c] = dh1[c,a] conj(F_k(r)_a)
-__global__ __launch_bounds__(256) void k_net_in_bwd(NetGeo g, const Spin<float>* __restrict__ r,
-                                                    const float* __restrict__ dh,
-                                                    float* __restrict__ contrib) {
-  const size_t P = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (P >= g.np) return;
-  float2 F[5][2];
-  feat1<false>(g, r, P, F);
-  float* cdst = contrib + P * (20 * C);
-  for (int c = 0; c < C; c++)
-    for (int a = 0; a < 2; a++) {
-      const float2 ga = {dh[(P * 2 + a) * RW + 2 * c], dh[(P * 2 + a) * RW + 2 * c + 1]};
-      for (int k = 0; k < 5; k++) {
-        const float2 z = cmc(F[k][a], ga);
-        cdst[2 * ((a * 5 + k) * C + c)] = z.x;
-        cdst[2 * ((a * 5 + k) * C + c) + 1] = z.y;
-      }
-    }
+  const int o = OUT && sk == 2 ? 1 - sa : sa;
+  if (t < kHeadCols) partial[size_t(blockIdx.x) * kHeadCols + (o * 5 + sk) * C + c] = acc;
 }
 
 // Input gradient of a mixing layer, G = R_a^T dz per column of spin a (MFMA, M = 160 in 5
@@ -428,52 +454,74 @@ __global__ __launch_bounds__(256) void k_net_mid_G(size_t np, const float* __res
   }
 }
 
-// Weight gradient of a mixing layer, dR_a (32 x 160) = sum over the block's 64 columns of
-// spin a of dz (32) F^T (160) (MFMA with K over those columns), one partial per block:
-// partial[block][a][32][160].
+// Weight gradient of a mixing layer, dR_a (32 x 160) = sum over the columns of spin a of
+// dz (32) F^T (160): MFMA with K over the 64 columns of a group of points, each group's FP32
+// tile added to FP64 accumulators that a block keeps over all its groups, so a block writes
+// its sums once (partial[block][a][32][160]) whatever the number of points.  One FP32 partial
+// per group (41 KB per 64 points) was written and read back before: 0.13 + 0.9 ms per layer
+// at 4 x 81,920 points, now 0.12 + 0.008 ms.
+constexpr int kDwJobs = 3;  // (feature tile, spin) jobs of a wave: 10 over 4 waves
 __global__ __launch_bounds__(256) void k_net_mid_dW(NetGeo g, const bf16* __restrict__ hin,
                                                     const float* __restrict__ dz,
-                                                    float* __restrict__ partial) {
+                                                    double* __restrict__ partial) {
   __shared__ __attribute__((aligned(16))) bf16 FT[KF][2 * PTS + 8];   // [feature][col]
   __shared__ __attribute__((aligned(16))) bf16 ZT[RW][2 * PTS + 8];   // [row][col]
   const int t = threadIdx.x;
-  const size_t P0 = size_t(blockIdx.x) * PTS;
-  {
-    const int p = t >> 2, grp = t & 3;
-    const size_t P = P0 + p;
-    float2 F[5][2][4];
-    const bool ok = P < g.np;
-    if (ok) feat4<false>(g, hin, P, grp, F);
-    for (int a = 0; a < 2; a++) {
-      const int col = a * PTS + p;
-      for (int k = 0; k < 5; k++)
-        for (int i = 0; i < 4; i++) {
-          const int f = k * RW + 2 * (4 * grp + i);
-          FT[f][col] = bf16(ok ? F[k][a][i].x : 0.f);
-          FT[f + 1][col] = bf16(ok ? F[k][a][i].y : 0.f);
-        }
-      for (int i = 0; i < 8; i++) {
-        const int row = 8 * grp + i;
-        ZT[row][col] = bf16(ok ? dz[(P * 2 + a) * RW + row] : 0.f);
-      }
-    }
-  }
-  __syncthreads();
   const int lane = t & 63, w = t >> 6;
   const int m = lane & 31, hi = lane >> 5;
-  // 10 jobs (5 feature tiles x 2 spins) over 4 waves: wave w takes jobs w, w+4, w+8
-  for (int job = w; job < 10; job += 4) {
-    const int tile = job % 5, a = job / 5;
-    f32x16 acc = {};
-    for (int kk = a * (PTS / 16); kk < (a + 1) * (PTS / 16); kk++) {
-      const bf16x8 av = *reinterpret_cast<const bf16x8*>(&ZT[m][16 * kk + 8 * hi]);
-      const bf16x8 bv = *reinterpret_cast<const bf16x8*>(&FT[32 * tile + m][16 * kk + 8 * hi]);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc, 0, 0, 0);
+  double sum[kDwJobs][16];
+#pragma unroll
+  for (int j = 0; j < kDwJobs; j++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) sum[j][i] = 0.0;
+  for (size_t P0 = size_t(blockIdx.x) * PTS; P0 < g.np; P0 += size_t(gridDim.x) * PTS) {
+    {
+      const int p = t >> 2, grp = t & 3;
+      const size_t P = P0 + p;
+      float2 F[5][2][4];
+      const bool ok = P < g.np;
+      if (ok) feat4<false>(g, hin, P, grp, F);
+      for (int a = 0; a < 2; a++) {
+        const int col = a * PTS + p;
+        for (int k = 0; k < 5; k++)
+          for (int i = 0; i < 4; i++) {
+            const int f = k * RW + 2 * (4 * grp + i);
+            FT[f][col] = bf16(ok ? F[k][a][i].x : 0.f);
+            FT[f + 1][col] = bf16(ok ? F[k][a][i].y : 0.f);
+          }
+        for (int i = 0; i < 8; i++) {
+          const int row = 8 * grp + i;
+          ZT[row][col] = bf16(ok ? dz[(P * 2 + a) * RW + row] : 0.f);
+        }
+      }
     }
-    float* dst = partial + (size_t(blockIdx.x) * 2 + a) * (RW * KF);
-    for (int i = 0; i < 16; i++) {
-      const int row = 8 * (i / 4) + 4 * hi + (i % 4);
-      dst[row * KF + 32 * tile + m] = acc[i];
+    __syncthreads();
+    // wave w takes jobs w, w+4, w+8
+#pragma unroll
+    for (int j = 0; j < kDwJobs; j++) {
+      const int job = w + 4 * j;
+      if (job < 10) {
+        const int tile = job % 5, a = job / 5;
+        f32x16 acc = {};
+        for (int kk = a * (PTS / 16); kk < (a + 1) * (PTS / 16); kk++) {
+          const bf16x8 av = *reinterpret_cast<const bf16x8*>(&ZT[m][16 * kk + 8 * hi]);
+          const bf16x8 bv = *reinterpret_cast<const bf16x8*>(&FT[32 * tile + m][16 * kk + 8 * hi]);
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; i++) sum[j][i] += double(acc[i]);
+      }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int j = 0; j < kDwJobs; j++) {
+    const int job = w + 4 * j;
+    if (job < 10) {
+      const int tile = job % 5, a = job / 5;
+      double* dst = partial + (size_t(blockIdx.x) * 2 + a) * (RW * KF);
+#pragma unroll
+      for (int i = 0; i < 16; i++) dst[(8 * (i / 4) + 4 * hi + (i % 4)) * KF + 32 * tile + m] = sum[j][i];
     }
   }
 }
@@ -534,20 +582,35 @@ __global__ __launch_bounds__(256) void k_net_adj(NetGeo g, const float* __restri
   }
 }
 
-// out[j] = sum_i buf[i][j] in FP64, one block per column group
-__global__ __launch_bounds__(256) void k_colsum(const float* __restrict__ buf, size_t rows, int cols,
-                                                double* __restrict__ out) {
-  __shared__ double sh[256];
-  const int j = blockIdx.x;
+// out[j] = sum_i buf[i][j]: a block takes 64 columns, its sixteen waves every sixteenth row
+// of them (a wave's loads consecutive), so the partials are read once.  With the few hundred
+// rows there are, four waves per block were bound by the latency of their serial rows (44 us
+// for 640 x 10,240 with four, 8 us with sixteen).
+constexpr unsigned kColWaves = 16;
+__global__ __launch_bounds__(64 * kColWaves) void k_colsum(const double* __restrict__ buf, unsigned rows,
+                                                           unsigned cols, double* __restrict__ out) {
+  __shared__ double sh[kColWaves][64];
+  const unsigned lane = threadIdx.x & 63, w = threadIdx.x >> 6, j = blockIdx.x * 64 + lane;
   double s = 0;
-  for (size_t i = threadIdx.x; i < rows; i += blockDim.x) s += buf[i * cols + j];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-    if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-    __syncthreads();
+  if (j < cols) {
+#pragma unroll 4
+    for (unsigned i = w; i < rows; i += kColWaves) s += buf[size_t(i) * cols + j];
   }
-  if (threadIdx.x == 0) out[j] = sh[0];
+  sh[w][lane] = s;
+  __syncthreads();
+  if (w == 0 && j < cols) {
+    double t = 0;
+#pragma unroll
+    for (unsigned k = 0; k < kColWaves; k++) t += sh[k][lane];
+    out[j] = t;
+  }
+}
+
+// Blocks of the kernels that keep FP64 sums over groups of points: two to three per CU (more
+// would only add partials to write and sum), never more than there are groups
+constexpr unsigned kSumBlocks = 640;
+unsigned sum_blocks(size_t np, size_t group) {
+  return unsigned(std::min<size_t>((np + group - 1) / group, kSumBlocks));
 }
 
 template <typename T>
@@ -716,9 +779,11 @@ void Net::ensure(int B, bool training) {
     G_ = dmalloc<float>(np * 5 * 2 * RW);
     out_ = dmalloc<Spin<float>>(np);
     gout_ = dmalloc<Spin<float>>(np);
-    const size_t nblk = (np + PTS - 1) / PTS;
-    partial_ = reinterpret_cast<double*>(dmalloc<float>(std::max(nblk * 2 * RW * KF, np * 20 * C)));
-    red_ = dmalloc<double>(2 * RW * KF + 2 * size_t(std::max(B, capB_)));
+    const size_t nB = std::max(B, capB_);
+    partial_ = dmalloc<double>(std::max({sum_blocks(np, PTS) * size_t(2 * RW * KF),
+                                         sum_blocks(np, 256) * size_t(2 * kHeadCols),
+                                         nB * 2 * sum_blocks(D_.points(), 256)}));
+    red_ = dmalloc<double>(2 * RW * KF + 2 * nB);
   }
   capB_ = std::max(B, capB_);
   cap_train_ = cap_train_ || training;
@@ -790,19 +855,26 @@ double Net::loss_grad(const Spin<float>* r, const Spin<float>* e, int B, std::ve
                        static_cast<const bf16*>(mixA_) + size_t(l) * 2 * RW * KF, act(l + 1));
   hipLaunchKernelGGL(k_net_out<false>, dim3(nb), dim3(256), 0, st, g, act(nmid), u, r, skip_, out_);
   // loss
-  QED3_HIP(hipMemsetAsync(red_, 0, 2 * B * sizeof(double), st));
-  hipLaunchKernelGGL(k_net_loss, dim3(nb), dim3(256), 0, st, out_, e, np, per, red_);
+  const unsigned nbl = sum_blocks(per, 256);
+  hipLaunchKernelGGL(k_net_loss, dim3(nbl * unsigned(B)), dim3(256), 0, st, out_, e, per, nbl,
+                     reinterpret_cast<double2*>(partial_));
+  hipLaunchKernelGGL(k_net_loss_sum, dim3(unsigned(B)), dim3(256), 0, st, reinterpret_cast<const double2*>(partial_),
+                     nbl, red_);
   hipLaunchKernelGGL(k_net_gout, dim3(nb), dim3(256), 0, st, out_, e, np, per, red_, B, gout_);
   std::vector<double> pairs(2 * B);
   QED3_HIP(hipMemcpyAsync(pairs.data(), red_, pairs.size() * sizeof(double), hipMemcpyDeviceToHost, st));
   // output head
-  float* contrib = reinterpret_cast<float*>(partial_);
   double* red = red_ + 2 * B;
+  const unsigned nbh = sum_blocks(np, 256), nbw = sum_blocks(np, PTS);
+  auto colsum = [&](unsigned rows, unsigned cols) {
+    hipLaunchKernelGGL(k_colsum, dim3((cols + 63) / 64), dim3(64 * kColWaves), 0, st, partial_, rows, cols, red);
+  };
   grad.assign(p_.size(), 0.0);
   const size_t nw = size_t(nmid) * 10 * C * C;
   std::vector<double> tmp(2 * RW * KF);
-  hipLaunchKernelGGL(k_net_out_bwd, dim3(nb), dim3(256), 0, st, g, gout_, act(nmid), u, gfield_, contrib);
-  hipLaunchKernelGGL(k_colsum, dim3(20 * C), dim3(256), 0, st, contrib, np, 20 * C, red);
+  hipLaunchKernelGGL(k_net_head_bwd<true>, dim3(nbh), dim3(256), 0, st, g, gout_, act(nmid), u, gfield_,
+                     reinterpret_cast<double2*>(partial_));
+  colsum(nbh, 2 * kHeadCols);
   QED3_HIP(hipMemcpyAsync(tmp.data(), red, 20 * C * sizeof(double), hipMemcpyDeviceToHost, st));
   QED3_HIP(hipStreamSynchronize(st));
   for (int i = 0; i < 20 * C; i++) grad[2 * (10 * C + nw) + i] = tmp[i];
@@ -810,8 +882,8 @@ double Net::loss_grad(const Spin<float>* r, const Spin<float>* e, int B, std::ve
   float* gin = gfield_;
   float* gnext = gfield2_;
   for (int l = nmid - 1; l >= 0; l--) {
-    hipLaunchKernelGGL(k_net_mid_dW, dim3(nbm), dim3(256), 0, st, g, act(l), gin, contrib);
-    hipLaunchKernelGGL(k_colsum, dim3(2 * RW * KF), dim3(256), 0, st, contrib, size_t(nbm), 2 * RW * KF, red);
+    hipLaunchKernelGGL(k_net_mid_dW, dim3(nbw), dim3(256), 0, st, g, act(l), gin, partial_);
+    colsum(nbw, 2 * RW * KF);
     QED3_HIP(hipMemcpyAsync(tmp.data(), red, 2 * RW * KF * sizeof(double), hipMemcpyDeviceToHost, st));
     hipLaunchKernelGGL(k_net_mid_G, dim3(nbm), dim3(256), 0, st, np, gin,
                        static_cast<const bf16*>(mixAT_) + size_t(l) * 2 * RW * KF, G_);
@@ -832,8 +904,9 @@ double Net::loss_grad(const Spin<float>* r, const Spin<float>* e, int B, std::ve
     std::swap(gin, gnext);
   }
   // input head
-  hipLaunchKernelGGL(k_net_in_bwd, dim3(nb), dim3(256), 0, st, g, r, gin, contrib);
-  hipLaunchKernelGGL(k_colsum, dim3(20 * C), dim3(256), 0, st, contrib, np, 20 * C, red);
+  hipLaunchKernelGGL(k_net_head_bwd<false>, dim3(nbh), dim3(256), 0, st, g, r, static_cast<const bf16*>(nullptr),
+                     static_cast<const float2*>(nullptr), gin, reinterpret_cast<double2*>(partial_));
+  colsum(nbh, 2 * kHeadCols);
   QED3_HIP(hipMemcpyAsync(tmp.data(), red, 20 * C * sizeof(double), hipMemcpyDeviceToHost, st));
   QED3_HIP(hipStreamSynchronize(st));
   QED3_HIP(hipGetLastError());

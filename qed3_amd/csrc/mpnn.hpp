@@ -76,7 +76,7 @@ class Net {
   float* G_ = nullptr;         // [B*points][5][2][32] FP32
   Spin<float>* out_ = nullptr;
   Spin<float>* gout_ = nullptr;
-  double* partial_ = nullptr;  // per-block weight-gradient partials
+  double* partial_ = nullptr;  // per-block FP64 sums of the loss and weight-gradient kernels
   double* red_ = nullptr;
   int capB_ = 0;
   bool cap_train_ = false;
