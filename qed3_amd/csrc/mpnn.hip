@@ -371,11 +371,19 @@ __global__ __launch_bounds__(256) void k_net_gout(const Spin<float>* __restrict_
 // products of every point (1.25 KB) and summed them column by column in another kernel:
 // 0.83 (output head) and 0.39 ms (input head) plus 0.9 ms a sum at 4 x 81,920 points; this
 // takes 0.067 and 0.054 ms plus 0.008 ms.
+//
+// The gradient field between layers is BF16 where a mixing layer consumes it (its products
+// round it to BF16 in any case) and FP32 where the input head does.
+__device__ __forceinline__ void put_grad(float* p, float2 z) { *reinterpret_cast<float2*>(p) = z; }
+__device__ __forceinline__ void put_grad(bf16* p, float2 z) {
+  typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
+  *reinterpret_cast<bf16x2*>(p) = bf16x2{bf16(z.x), bf16(z.y)};
+}
 constexpr int kHeadCols = 10 * C;  // complex sums of a head gradient
-template <bool OUT>
+template <bool OUT, typename Z>
 __global__ __launch_bounds__(256) void k_net_head_bwd(NetGeo g, const Spin<float>* __restrict__ f,
                                                       const bf16* __restrict__ h, const float2* __restrict__ u,
-                                                      float* __restrict__ dh, double2* __restrict__ partial) {
+                                                      Z* __restrict__ dh, double2* __restrict__ partial) {
   __shared__ float2 Fs[10][256 + 1];  // [2 k + a][point]; the pad spreads the columns' writes
   const int t = threadIdx.x;
   const int c = t & (C - 1), ka = t >> 4;  // the sum this thread keeps (t < kHeadCols)
@@ -397,12 +405,12 @@ __global__ __launch_bounds__(256) void k_net_head_bwd(NetGeo g, const Spin<float
       float2 uk[5];
 #pragma unroll
       for (int k = 0; k < 5; k++) uk[k] = u[((k == 2 ? 1 - a : a) * 5 + k) * C + c];
-      float2* row = reinterpret_cast<float2*>(dh) + P0 * RW + (t & (RW - 1));
+      Z* row = dh + (P0 * RW + (t & (RW - 1))) * 2;
       for (int p = t >> 5; p < cnt; p += 8) {
         float2 z = {0.f, 0.f};
 #pragma unroll
         for (int k = 0; k < 5; k++) cadd_(z, cmc(uk[k], Fs[2 * k + a][p]));
-        row[size_t(p) * RW] = z;
+        put_grad(row + size_t(p) * 2 * RW, z);
       }
     }
     if (t < kHeadCols) {
@@ -413,7 +421,7 @@ __global__ __launch_bounds__(256) void k_net_head_bwd(NetGeo g, const Spin<float
           const bf16* src = h + ((P0 + p) * 2 + sa) * RW + 2 * c;
           z = cmc(float2{float(src[0]), float(src[1])}, x);
         } else {
-          const float2 y = reinterpret_cast<const float2*>(dh)[((P0 + p) * 2 + sa) * C + c];
+          const float2 y = *reinterpret_cast<const float2*>(dh + ((P0 + p) * 2 + sa) * RW + 2 * c);
           z = cmc(x, y);
         }
         acc.x += double(z.x);
@@ -426,34 +434,6 @@ __global__ __launch_bounds__(256) void k_net_head_bwd(NetGeo g, const Spin<float
   if (t < kHeadCols) partial[size_t(blockIdx.x) * kHeadCols + (o * 5 + sk) * C + c] = acc;
 }
 
-// Input gradient of a mixing layer, G = R_a^T dz per column of spin a (MFMA, M = 160 in 5
-// tiles, K = 32): G[P][k][a][32] FP32.  Columns ordered (spin, point) as in k_net_mid.
-__global__ __launch_bounds__(256) void k_net_mid_G(size_t np, const float* __restrict__ dz,
-                                                   const bf16* __restrict__ AT /*[2][160][32]*/,
-                                                   float* __restrict__ G) {
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int m = lane & 31, hi = lane >> 5;
-  const int n = 32 * w + m;
-  const size_t P = size_t(blockIdx.x) * PTS + (n % PTS);
-  const int a = n / PTS;
-  const bf16* ATa = AT + size_t(w >> 1) * KF * RW;
-  bf16x8 b[2];
-  for (int kk = 0; kk < 2; kk++)
-    for (int i = 0; i < 8; i++)
-      b[kk][i] = bf16(P < np ? dz[(P * 2 + a) * RW + 16 * kk + 8 * hi + i] : 0.f);
-  for (int tile = 0; tile < 5; tile++) {
-    f32x16 acc = {};
-    for (int kk = 0; kk < 2; kk++) {
-      const bf16x8 av = *reinterpret_cast<const bf16x8*>(ATa + (32 * tile + m) * RW + 16 * kk + 8 * hi);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, b[kk], acc, 0, 0, 0);
-    }
-    if (P < np) {
-      float* dst = G + ((P * 5 + tile) * 2 + a) * RW;
-      for (int i = 0; i < 16; i++) dst[8 * (i / 4) + 4 * hi + (i % 4)] = acc[i];
-    }
-  }
-}
-
 // Weight gradient of a mixing layer, dR_a (32 x 160) = sum over the columns of spin a of
 // dz (32) F^T (160): MFMA with K over the 64 columns of a group of points, each group's FP32
 // tile added to FP64 accumulators that a block keeps over all its groups, so a block writes
@@ -462,7 +442,7 @@ __global__ __launch_bounds__(256) void k_net_mid_G(size_t np, const float* __res
 // at 4 x 81,920 points, now 0.12 + 0.008 ms.
 constexpr int kDwJobs = 3;  // (feature tile, spin) jobs of a wave: 10 over 4 waves
 __global__ __launch_bounds__(256) void k_net_mid_dW(NetGeo g, const bf16* __restrict__ hin,
-                                                    const float* __restrict__ dz,
+                                                    const bf16* __restrict__ dz,
                                                     double* __restrict__ partial) {
   __shared__ __attribute__((aligned(16))) bf16 FT[KF][2 * PTS + 8];   // [feature][col]
   __shared__ __attribute__((aligned(16))) bf16 ZT[RW][2 * PTS + 8];   // [row][col]
@@ -489,10 +469,9 @@ __global__ __launch_bounds__(256) void k_net_mid_dW(NetGeo g, const bf16* __rest
             FT[f][col] = bf16(ok ? F[k][a][i].x : 0.f);
             FT[f + 1][col] = bf16(ok ? F[k][a][i].y : 0.f);
           }
-        for (int i = 0; i < 8; i++) {
-          const int row = 8 * grp + i;
-          ZT[row][col] = bf16(ok ? dz[(P * 2 + a) * RW + row] : 0.f);
-        }
+        bf16x8 z = {};
+        if (ok) z = *reinterpret_cast<const bf16x8*>(dz + (P * 2 + a) * RW + 8 * grp);
+        for (int i = 0; i < 8; i++) ZT[8 * grp + i][col] = z[i];
       }
     }
     __syncthreads();
@@ -526,59 +505,90 @@ __global__ __launch_bounds__(256) void k_net_mid_dW(NetGeo g, const bf16* __rest
   }
 }
 
-// dh_in(y) = sum_k F_k^dagger G_k  (gather form; thread per point and 4-channel group)
-__global__ __launch_bounds__(256) void k_net_adj(NetGeo g, const float* __restrict__ G,
-                                                 float* __restrict__ dh) {
-  const size_t T = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const size_t P = T >> 2;
-  const int grp = int(T & 3);
-  if (P >= g.np) return;
-  const PointIdx q = point_of(g, P);
-  auto ld = [&](size_t Q, int k, int a, float2 o[4]) {
-    const float4* src = reinterpret_cast<const float4*>(G + ((Q * 5 + k) * 2 + a) * RW + 8 * grp);
-    const float4 v0 = src[0], v1 = src[1];
-    o[0] = {v0.x, v0.y};
-    o[1] = {v0.z, v0.w};
-    o[2] = {v1.x, v1.y};
-    o[3] = {v1.z, v1.w};
+// Input gradient of a mixing layer, dh_in = sum_k F_k^dagger G_k with G_k = R_k^T dz, the maps'
+// neighbour sums gathering dz (128 B a point) and multiplying by the weights at the gathering
+// point: MFMA is idle enough to redo the products for every neighbour, and G (1.25 KB a point
+// in FP32, written once and read four times over) never exists.  Columns are ordered (spin,
+// point) as in k_net_mid, a wave holding 32 points of one output spin; a lane's accumulator
+// rows come in (re, im) pairs, so the transports act on the MFMA result where it is.  Bound by
+// the latency of its gathers: every column's loads are issued before the first product (8
+// VGPRs a column; the weights' five tiles in 40 more).  0.10 ms per layer at 4 x 81,920 points;
+// the two kernels this replaces took 0.13 + 0.13 ms, bound by G's bytes, and this form 0.37 ms
+// with one load at a time and FP32 dz.
+template <int NS, typename Z>
+__global__ __launch_bounds__(256) void k_net_mid_adj(NetGeo g, const bf16* __restrict__ dz,
+                                                     const bf16* __restrict__ AT /*[2][160][32]*/,
+                                                     Z* __restrict__ dh) {
+  struct Col {
+    bf16x8 b[2];
   };
-  float2 r0[4], r1[4], t[4], t2[4];
-  ld(P, 0, 0, r0);
-  ld(P, 0, 1, r1);
-  for (int j = 0; j < g.M; j++) {
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int m = lane & 31, hi = lane >> 5;
+  const int n = 32 * w + m;
+  const size_t P = size_t(blockIdx.x) * PTS + (n % PTS);
+  const int a = w >> 1;  // output spin of the wave
+  const bool ok = P < g.np;
+  // lanes beyond the last point work on the first (every lane takes part in the MFMAs)
+  const size_t Pc = ok ? P : 0;
+  const PointIdx q = point_of(g, Pc);
+  auto load = [&](size_t Q, int sa) {
+    const bf16x8* src = reinterpret_cast<const bf16x8*>(dz + (Q * 2 + sa) * RW + 8 * hi);
+    return Col{{src[0], src[2]}};
+  };
+  size_t Q[NS];
+#pragma unroll
+  for (int j = 0; j < NS; j++) Q[j] = q.base + g.nbr[size_t(j) * g.V + q.x];
+  const Col c0 = load(Pc, a), cm_ = load(q.Pm, a), cp = load(q.Pp, a);
+  Col c1[NS], c2[NS];
+#pragma unroll
+  for (int j = 0; j < NS; j++) {
+    c1[j] = load(Q[j], a);
+    c2[j] = load(Q[j], 1 - a);
+  }
+  Col A[5];  // the weight tiles: the gamma map's (k = 2) takes the other spin's dz
+#pragma unroll
+  for (int k = 0; k < 5; k++) {
+    const bf16x8* src =
+        reinterpret_cast<const bf16x8*>(AT + (size_t(k == 2 ? 1 - a : a) * KF + 32 * k + m) * RW + 8 * hi);
+    A[k] = Col{{src[0], src[2]}};
+  }
+  auto mul = [&](const Col& b, int k) {
+    f32x16 acc = {};
+#pragma unroll
+    for (int kk = 0; kk < 2; kk++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[k].b[kk], b.b[kk], acc, 0, 0, 0);
+    return acc;
+  };
+  float2 r[8];
+  auto add = [&](float2 f, const f32x16& G) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) cadd_(r[i], cm(f, float2{G[2 * i], G[2 * i + 1]}));
+  };
+  {
+    const f32x16 G = mul(c0, 0);
+#pragma unroll
+    for (int i = 0; i < 8; i++) r[i] = {G[2 * i], G[2 * i + 1]};
+  }
+#pragma unroll
+  for (int j = 0; j < NS; j++) {
     const SlotT s = slot_t(g, j, q.x, q.s, true);
-    const size_t Q = q.base + s.y;
     // spin 0: tau_yx,0 G1_0 + e^{-i a_xy} tau_yx,0 G2_1 ; spin 1: tau_yx,1 G1_1 + e^{i a_xy} tau_yx,1 G2_0
-    ld(Q, 1, 0, t);
-    ld(Q, 2, 1, t2);
-    const float2 k0 = cm(s.ea, s.t0), k1 = cm(s.eb, s.t1);
-    for (int i = 0; i < 4; i++) {
-      cadd_(r0[i], cm(s.t0, t[i]));
-      cadd_(r0[i], cm(k0, t2[i]));
-    }
-    ld(Q, 1, 1, t);
-    ld(Q, 2, 0, t2);
-    for (int i = 0; i < 4; i++) {
-      cadd_(r1[i], cm(s.t1, t[i]));
-      cadd_(r1[i], cm(k1, t2[i]));
-    }
+    const float2 t0 = a == 0 ? s.t0 : s.t1, k0 = a == 0 ? cm(s.ea, s.t0) : cm(s.eb, s.t1);
+    add(t0, mul(c1[j], 1));
+    add(k0, mul(c2[j], 2));
   }
   // adjoint of F3 from s-1: bm conj(U_{s-1}) G3(s-1);  adjoint of F4 from s+1: bp U_s G4(s+1)
   const float2 up = g.uT[size_t(q.s) * g.V + q.x];
   const float2 um = cj(g.uT[size_t(q.s == 0 ? g.Lt - 1 : q.s - 1) * g.V + q.x]);
   const float2 wm = {q.bm * um.x, q.bm * um.y}, wp = {q.bp * up.x, q.bp * up.y};
-  for (int a = 0; a < 2; a++) {
-    float2* acc = a == 0 ? r0 : r1;
-    ld(q.Pm, 3, a, t);
-    for (int i = 0; i < 4; i++) cadd_(acc[i], cm(wm, t[i]));
-    ld(q.Pp, 4, a, t);
-    for (int i = 0; i < 4; i++) cadd_(acc[i], cm(wp, t[i]));
-  }
-  for (int a = 0; a < 2; a++) {
-    const float2* acc = a == 0 ? r0 : r1;
-    float4* dst = reinterpret_cast<float4*>(dh + (P * 2 + a) * RW + 8 * grp);
-    dst[0] = float4{acc[0].x, acc[0].y, acc[1].x, acc[1].y};
-    dst[1] = float4{acc[2].x, acc[2].y, acc[3].x, acc[3].y};
+  add(wm, mul(cm_, 3));
+  add(wp, mul(cp, 4));
+  if (ok) {
+    Z* dst = dh + (P * 2 + a) * RW + 4 * hi;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      put_grad(dst + 8 * j, r[2 * j]);
+      put_grad(dst + 8 * j + 2, r[2 * j + 1]);
+    }
   }
 }
 
@@ -684,7 +694,7 @@ Net::Net(Dirac& D, int layers, int seed) : D_(D), L_(layers) {
 
 Net::~Net() {
   for (void* p : {(void*)slot_, (void*)slot_nb_, (void*)kt_, (void*)heads_, mixA_, mixAT_, mixAH_, act_, (void*)gfield_,
-                  (void*)gfield2_, (void*)G_, (void*)out_, (void*)gout_, (void*)partial_, (void*)red_})
+                  (void*)gfield2_, (void*)out_, (void*)gout_, (void*)partial_, (void*)red_})
     if (p) (void)hipFree(p);
 }
 
@@ -764,11 +774,11 @@ void Net::upload_params() {
 void Net::ensure(int B, bool training) {
   if (B <= capB_ && (!training || cap_train_)) return;
   const size_t np = size_t(std::max(B, capB_)) * D_.points();
-  for (void* p : {act_, (void*)gfield_, (void*)gfield2_, (void*)G_, (void*)out_, (void*)gout_,
+  for (void* p : {act_, (void*)gfield_, (void*)gfield2_, (void*)out_, (void*)gout_,
                   (void*)partial_, (void*)red_})
     if (p) (void)hipFree(p);
   act_ = nullptr;
-  gfield_ = gfield2_ = G_ = nullptr;
+  gfield_ = gfield2_ = nullptr;
   out_ = gout_ = nullptr;
   partial_ = red_ = nullptr;
   const int nact = training ? std::max(L_ - 1, 2) : 2;
@@ -776,7 +786,6 @@ void Net::ensure(int B, bool training) {
   if (training) {
     gfield_ = dmalloc<float>(np * 2 * RW);
     gfield2_ = dmalloc<float>(np * 2 * RW);
-    G_ = dmalloc<float>(np * 5 * 2 * RW);
     out_ = dmalloc<Spin<float>>(np);
     gout_ = dmalloc<Spin<float>>(np);
     const size_t nB = std::max(B, capB_);
@@ -872,8 +881,12 @@ double Net::loss_grad(const Spin<float>* r, const Spin<float>* e, int B, std::ve
   grad.assign(p_.size(), 0.0);
   const size_t nw = size_t(nmid) * 10 * C * C;
   std::vector<double> tmp(2 * RW * KF);
-  hipLaunchKernelGGL(k_net_head_bwd<true>, dim3(nbh), dim3(256), 0, st, g, gout_, act(nmid), u, gfield_,
-                     reinterpret_cast<double2*>(partial_));
+  if (nmid > 0)
+    hipLaunchKernelGGL((k_net_head_bwd<true, bf16>), dim3(nbh), dim3(256), 0, st, g, gout_, act(nmid), u,
+                       reinterpret_cast<bf16*>(gfield_), reinterpret_cast<double2*>(partial_));
+  else
+    hipLaunchKernelGGL((k_net_head_bwd<true, float>), dim3(nbh), dim3(256), 0, st, g, gout_, act(nmid), u, gfield_,
+                       reinterpret_cast<double2*>(partial_));
   colsum(nbh, 2 * kHeadCols);
   QED3_HIP(hipMemcpyAsync(tmp.data(), red, 20 * C * sizeof(double), hipMemcpyDeviceToHost, st));
   QED3_HIP(hipStreamSynchronize(st));
@@ -882,12 +895,27 @@ double Net::loss_grad(const Spin<float>* r, const Spin<float>* e, int B, std::ve
   float* gin = gfield_;
   float* gnext = gfield2_;
   for (int l = nmid - 1; l >= 0; l--) {
-    hipLaunchKernelGGL(k_net_mid_dW, dim3(nbw), dim3(256), 0, st, g, act(l), gin, partial_);
+    hipLaunchKernelGGL(k_net_mid_dW, dim3(nbw), dim3(256), 0, st, g, act(l), reinterpret_cast<const bf16*>(gin),
+                       partial_);
     colsum(nbw, 2 * RW * KF);
     QED3_HIP(hipMemcpyAsync(tmp.data(), red, 2 * RW * KF * sizeof(double), hipMemcpyDeviceToHost, st));
-    hipLaunchKernelGGL(k_net_mid_G, dim3(nbm), dim3(256), 0, st, np, gin,
-                       static_cast<const bf16*>(mixAT_) + size_t(l) * 2 * RW * KF, G_);
-    hipLaunchKernelGGL(k_net_adj, dim3(unsigned((4 * np + 255) / 256)), dim3(256), 0, st, g, G_, gnext);
+    const bf16* AT = static_cast<const bf16*>(mixAT_) + size_t(l) * 2 * RW * KF;
+    auto input_grad = [&](auto ns, auto* dst) {
+      constexpr int NS = decltype(ns)::value;
+      using Z = std::remove_pointer_t<decltype(dst)>;
+      hipLaunchKernelGGL((k_net_mid_adj<NS, Z>), dim3(nbm), dim3(256), 0, st, g, reinterpret_cast<const bf16*>(gin), AT,
+                         dst);
+    };
+    auto input_grad_ns = [&](auto* dst) {
+      if (g.M == 6)
+        input_grad(std::integral_constant<int, 6>{}, dst);
+      else
+        input_grad(std::integral_constant<int, 3>{}, dst);
+    };
+    if (l > 0)
+      input_grad_ns(reinterpret_cast<bf16*>(gnext));
+    else
+      input_grad_ns(gnext);
     QED3_HIP(hipStreamSynchronize(st));
     for (int sa = 0; sa < 2; sa++)
     for (int k = 0; k < 5; k++)
@@ -904,8 +932,9 @@ double Net::loss_grad(const Spin<float>* r, const Spin<float>* e, int B, std::ve
     std::swap(gin, gnext);
   }
   // input head
-  hipLaunchKernelGGL(k_net_head_bwd<false>, dim3(nbh), dim3(256), 0, st, g, r, static_cast<const bf16*>(nullptr),
-                     static_cast<const float2*>(nullptr), gin, reinterpret_cast<double2*>(partial_));
+  hipLaunchKernelGGL((k_net_head_bwd<false, float>), dim3(nbh), dim3(256), 0, st, g, r,
+                     static_cast<const bf16*>(nullptr), static_cast<const float2*>(nullptr), gin,
+                     reinterpret_cast<double2*>(partial_));
   colsum(nbh, 2 * kHeadCols);
   QED3_HIP(hipMemcpyAsync(tmp.data(), red, 20 * C * sizeof(double), hipMemcpyDeviceToHost, st));
   QED3_HIP(hipStreamSynchronize(st));

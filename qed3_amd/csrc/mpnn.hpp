@@ -71,9 +71,8 @@ class Net {
   void* mixAT_ = nullptr;      // per middle layer and output spin: R^T (160 x 32) bf16
   void* mixAH_ = nullptr;      // adjoint network: per layer and output spin (32 x 160) bf16
   void* act_ = nullptr;        // activations h1..h^{L-1}: [L-1][B*points][2][32] bf16
-  float* gfield_ = nullptr;    // gradient field [B*points][2][32] FP32 (two buffers)
+  float* gfield_ = nullptr;    // gradient field [B*points][2][32], FP32 or BF16 (two buffers)
   float* gfield2_ = nullptr;
-  float* G_ = nullptr;         // [B*points][5][2][32] FP32
   Spin<float>* out_ = nullptr;
   Spin<float>* gout_ = nullptr;
   double* partial_ = nullptr;  // per-block FP64 sums of the loss and weight-gradient kernels
