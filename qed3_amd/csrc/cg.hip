@@ -54,8 +54,12 @@ struct FinStart {
   CGScalars* sc;
   double tol2, delta2;
   int maxiter;
+  Spin<double>* x;
+  const Spin<double>* b;
   __device__ bool skip() const { return false; }
   __device__ void operator()(double2 t) const {
+    sc->x = x;
+    sc->b = b;
     sc->mu = t.x;
     sc->bnorm2 = t.x;
     sc->maxr2 = t.x;
@@ -75,10 +79,11 @@ struct FinStart {
   }
 };
 
+// x64 += x_inner, x_inner = 0 (x64 the solve's x of the scalars)
 template <typename T>
-__global__ __launch_bounds__(256) void k_flush(Spin<double>* x64, Spin<T>* xin, size_t n,
-                                               const CGScalars* sc, int always) {
+__global__ __launch_bounds__(256) void k_flush(Spin<T>* xin, size_t n, const CGScalars* sc, int always) {
   if (!always && (sc->done != 0 || sc->need_ru == 0)) return;
+  Spin<double>* x64 = sc->x;
   const double s = sc->scale;  // 1 unless the inner fields are stored scaled
   for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
        i += size_t(gridDim.x) * blockDim.x) {
@@ -101,8 +106,14 @@ struct FinStartH {
   CGScalars* sc;
   double ncomp, tol2, delta2;
   int maxiter;
+  Spin<double>* x;
+  const Spin<double>* b;
   __device__ bool skip() const { return false; }
-  __device__ void operator()(double2 t) const { half_start(sc, t.x, ncomp, tol2, delta2, maxiter); }
+  __device__ void operator()(double2 t) const {
+    sc->x = x;
+    sc->b = b;
+    half_start(sc, t.x, ncomp, tol2, delta2, maxiter);
+  }
 };
 
 // r = b / scale in half (FP64 arithmetic, so any finite b is representable)
@@ -185,8 +196,7 @@ CGResult run_cg(Dirac& D, Spin<double>* x, const Spin<double>* b, const CGOption
     W.xin = static_cast<Spin<T>*>(D.scratch(4, fb));
     W.t = static_cast<Spin<double>*>(D.scratch(5, n * sizeof(Spin<double>)));
   } else {
-    W.xin = reinterpret_cast<Spin<T>*>(x);
-    W.t = reinterpret_cast<Spin<double>*>(W.w);
+    W.t = reinterpret_cast<Spin<double>*>(W.w);  // x_inner is x itself
   }
   CGScalars* sc = static_cast<CGScalars*>(D.scratch(7, sizeof(CGScalars)));
   CGScalars* hsc = D.host_scalars();
@@ -196,9 +206,10 @@ CGResult run_cg(Dirac& D, Spin<double>* x, const Spin<double>* b, const CGOption
   const int ngate = int(gated_blocks(n));
   const double tol2 = o.tol * o.tol;
   const double delta2 = kMixed ? o.delta * o.delta : 0.0;
-  hipLaunchKernelGGL(k_init<T>, dim3(nbk), dim3(256), 0, st, b, x, W.xin, W.r, W.p, n, gr);
+  hipLaunchKernelGGL(k_init<T>, dim3(nbk), dim3(256), 0, st, b, x, kMixed ? W.xin : reinterpret_cast<Spin<T>*>(x), W.r,
+                     W.p, n, gr);
   hipLaunchKernelGGL(k_finalize<FinStart>, dim3(1), dim3(256), 0, st, gr.partials, unsigned(nbk),
-                     FinStart{sc, tol2, delta2, o.maxiter});
+                     FinStart{sc, tol2, delta2, o.maxiter, x, b});
   QED3_HIP(hipGetLastError());
 
   const DiracView<T> vin = D.view<T>();
@@ -210,6 +221,8 @@ CGResult run_cg(Dirac& D, Spin<double>* x, const Spin<double>* b, const CGOption
   // start; after a reliable update r and beta are the true residual's), stores that p in
   // the other buffer and applies D to it; K2 reads the new p.  p_old is read at halo points
   // of other blocks while the new p is written, hence two buffers alternating by parity.
+  // No kernel is given x or b: they take them from the scalars, so that the captured chunk
+  // serves every solve on this context.
   Spin<T>* P[2] = {W.p, W.p2};
   EventTimer timer(o.times);
   auto one_iter = [&](int i, int k) {
@@ -225,15 +238,20 @@ CGResult run_cg(Dirac& D, Spin<double>* x, const Spin<double>* b, const CGOption
     launch_stencil_src<T, true>(vin, nn, SrcPlain<T>{W.w}, EpiK2<T>{W.xin, W.r, pnew, sc, T(0)},
                                 D.tile<T>(true), gr, st, hvt, timer.pair(1, k));
     if (kMixed)
-      hipLaunchKernelGGL(k_flush<T>, dim3(ngate), dim3(256), 0, st, x, W.xin, n, sc, 0);
-    launch_stencil<double, false>(v64, nn, x, EpiStoreIfRU{W.t, sc}, D.tile<double>(false), gr, st, hv64f);
-    launch_stencil<double, true>(v64, nn, W.t, EpiResid<T>{b, W.r, sc}, D.tile<double>(true), gr, st, hv64t);
+      hipLaunchKernelGGL(k_flush<T>, dim3(ngate), dim3(256), 0, st, W.xin, n, sc, 0);
+    launch_stencil_src<double, false>(v64, nn, SrcSolX{sc}, EpiStoreIfRU{W.t, sc}, D.tile<double>(false), gr, st,
+                                      hv64f);
+    launch_stencil<double, true>(v64, nn, W.t, EpiResid<T>{nullptr, W.r, sc}, D.tile<double>(true), gr, st, hv64t);
   };
 
-  drive_chunks(one_iter, [] {}, o, n, st, sc, hsc);
+  GraphKey key;
+  key.add(vin).add(v64).add(hvf).add(hvt).add(hv64f).add(hv64t).add(D.tile<T>(false)).add(D.tile<T>(true));
+  key.add(D.tile<double>(false)).add(D.tile<double>(true)).add(W.r).add(W.p).add(W.p2).add(W.w).add(W.xin).add(W.t);
+  key.add(sc).add(gr.partials).add(n).add(nn);
+  drive_chunks(one_iter, [] {}, o, n, st, sc, hsc, &D.graph_slot(kMixed ? 1 : 0), key);
   timer.finish(hsc->iter);
   if (o.times) o.times->ms[2] = o.times->ms[1], o.times->count[2] = o.times->count[1];
-  if (kMixed) hipLaunchKernelGGL(k_flush<T>, dim3(nbk), dim3(256), 0, st, x, W.xin, n, sc, 1);
+  if (kMixed) hipLaunchKernelGGL(k_flush<T>, dim3(nbk), dim3(256), 0, st, W.xin, n, sc, 1);
   QED3_HIP(hipMemcpyAsync(hsc, sc, sizeof(CGScalars), hipMemcpyDeviceToHost, st));
   QED3_HIP(hipStreamSynchronize(st));
   CGResult res;
@@ -276,7 +294,7 @@ class HalfCG {
     ngate_ = int(gated_blocks(n_));
     hipLaunchKernelGGL(k_init_h, dim3(nbk_), dim3(256), 0, st_, b, x, xin_, ring_[kXGroup - 1], n_, gr_);
     hipLaunchKernelGGL(k_finalize<FinStartH>, dim3(1), dim3(256), 0, st_, gr_.partials, unsigned(nbk_),
-                       FinStartH{sc_, 4.0 * double(n_), o.tol * o.tol, o.delta * o.delta, o.maxiter});
+                       FinStartH{sc_, 4.0 * double(n_), o.tol * o.tol, o.delta * o.delta, o.maxiter, x, b});
     // the inner fields live in the temporal gauge (exp(i phi) at every point): b is rotated
     // into it here, the true residual at every reliable update, and x out of it at each flush
     vin_ = D.view_half_temporal_gauge();
@@ -302,12 +320,20 @@ class HalfCG {
     ru_each_ = o.times != nullptr;
     std::function<void()> tail = [] {};
     if (!ru_each_) tail = [this] { reliable_update(1); };
-    loop_ = std::make_unique<ChunkLoop>([this](int i, int k) { one_iter(i, k); }, tail, o, n_, st_, sc_, hsc_);
+    // (x and b are read from the scalars, so that the captured chunk serves every solve)
+    GraphKey key;
+    key.add(vin_).add(v64_).add(hvf_).add(hvt_).add(hv64f_).add(hv64t_).add(D.tile<float>(false));
+    key.add(D.tile<float>(true)).add(D.tile<double>(false)).add(D.tile<double>(true)).add(r_).add(w_).add(xin_);
+    for (SpinH* p : ring_) key.add(p);
+    key.add(t_).add(rt_).add(sc_).add(gr_.partials).add(rot_).add(n_).add(nn_);
+    loop_ = std::make_unique<ChunkLoop>([this](int i, int k) { one_iter(i, k); }, tail, o, n_, st_, sc_, hsc_,
+                                        &D.graph_slot(2), key);
   }
   ChunkLoop& loop() { return *loop_; }
   CGResult finish() {
     timer_.finish(hsc_->iter);
-    hipLaunchKernelGGL(k_flush_h, dim3(nbk_), dim3(256), 0, st_, x_, xin_, pend_, n_, sc_, 1, rot_);
+    hipLaunchKernelGGL(k_flush_h, dim3(nbk_), dim3(256), 0, st_, static_cast<Spin<double>*>(nullptr), xin_, pend_, n_,
+                       sc_, 1, rot_);
     QED3_HIP(hipMemcpyAsync(hsc_, sc_, sizeof(CGScalars), hipMemcpyDeviceToHost, st_));
     QED3_HIP(hipStreamSynchronize(st_));
     CGResult res;
@@ -332,10 +358,12 @@ class HalfCG {
                                     timer_.pair(EpiK2H<POS>::kUpdateX ? 2 : 1, k));
   }
   void reliable_update(int copy_last) {
-    hipLaunchKernelGGL(k_flush_h, dim3(ngate_), dim3(256), 0, st_, x_, xin_, pend_, n_, sc_, 0, rot_);
-    launch_stencil<double, false>(v64_, nn_, x_, EpiStoreIfRU{t_, sc_}, D_.tile<double>(false), gr_, st_, hv64f_);
-    launch_stencil<double, true>(v64_, nn_, t_, EpiResidH{b_, rt_, sc_, inv_ncomp_, 1.0}, D_.tile<double>(true), gr_,
-                                 st_, hv64t_);
+    hipLaunchKernelGGL(k_flush_h, dim3(ngate_), dim3(256), 0, st_, static_cast<Spin<double>*>(nullptr), xin_, pend_, n_,
+                       sc_, 0, rot_);
+    launch_stencil_src<double, false>(v64_, nn_, SrcSolX{sc_}, EpiStoreIfRU{t_, sc_}, D_.tile<double>(false), gr_, st_,
+                                      hv64f_);
+    launch_stencil<double, true>(v64_, nn_, t_, EpiResidH{nullptr, rt_, sc_, inv_ncomp_, 1.0}, D_.tile<double>(true),
+                                 gr_, st_, hv64t_);
     hipLaunchKernelGGL(k_rescale, dim3(ngate_), dim3(256), 0, st_, rt_, r_, ring_all_, copy_last, n_, sc_, rot_);
   }
   void one_iter(int i, int k) {
@@ -446,7 +474,7 @@ CGResult cg_solve_f64_workspace(Dirac& D, Spin<double>* x, const Spin<double>* b
   const int nbk = int(stream_blocks(n));
   hipLaunchKernelGGL(k_init<double>, dim3(nbk), dim3(256), 0, st, b, x, x, r, P[0], n, gr);
   hipLaunchKernelGGL(k_finalize<FinStart>, dim3(1), dim3(256), 0, st, gr.partials, unsigned(nbk),
-                     FinStart{sc, o.tol * o.tol, 0.0, o.maxiter});
+                     FinStart{sc, o.tol * o.tol, 0.0, o.maxiter, x, b});
   QED3_HIP(hipGetLastError());
   const DiracView<double> v64 = D.view<double>();
   const int nn = D.tables().max_nn;

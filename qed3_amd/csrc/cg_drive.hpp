@@ -77,8 +77,10 @@ class EventTimer {
 // Several loops on different streams can be launched before any host wait.
 class ChunkLoop {
  public:
+  // slot: where the captured chunk is kept from one solve to the next (with key, everything
+  // its kernels' arguments were made from); null: captured for this loop alone
   ChunkLoop(std::function<void(int, int)> one_iter, std::function<void()> tail, const CGOptions& o, size_t n,
-            hipStream_t st, const CGScalars* sc, CGScalars* hsc)
+            hipStream_t st, const CGScalars* sc, CGScalars* hsc, GraphSlot* slot = nullptr, GraphKey key = {})
       : one_iter_(std::move(one_iter)), tail_(std::move(tail)), st_(st), sc_(sc), hsc_(hsc) {
     chunk_ = o.chunk > 0 ? o.chunk : (n > (1u << 20) ? 8 : 16);
     chunk_ = (chunk_ + cgepi::kXGroup - 1) / cgepi::kXGroup * cgepi::kXGroup;  // every replay starts a new group
@@ -86,16 +88,26 @@ class ChunkLoop {
     // device's iteration cap ends the solve within this many chunks
     max_chunks_ = o.maxiter + 4;
     if (o.use_graph && !o.times && std::getenv("QED3_NO_GRAPH") == nullptr) {
-      QED3_HIP(hipStreamBeginCapture(st_, hipStreamCaptureModeThreadLocal));
-      for (int i = 0; i < chunk_; i++) one_iter_(i, -1);
-      tail_();
-      QED3_HIP(hipStreamEndCapture(st_, &graph_));
-      QED3_HIP(hipGraphInstantiate(&exec_, graph_, nullptr, nullptr, 0));
+      GraphSlot& g = slot ? *slot : own_;
+      key.add(chunk_);
+      if (!g.exec || g.key != key.words) {
+        g.clear();
+        QED3_HIP(hipStreamBeginCapture(st_, hipStreamCaptureModeThreadLocal));
+        try {
+          for (int i = 0; i < chunk_; i++) one_iter_(i, -1);
+          tail_();
+        } catch (...) {
+          hipGraph_t dead = nullptr;  // end the capture, or the stream stays in it
+          (void)hipStreamEndCapture(st_, &dead);
+          if (dead) (void)hipGraphDestroy(dead);
+          throw;
+        }
+        QED3_HIP(hipStreamEndCapture(st_, &g.graph));
+        QED3_HIP(hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0));
+        g.key = key.words;
+      }
+      exec_ = g.exec;
     }
-  }
-  ~ChunkLoop() {
-    if (exec_) (void)hipGraphExecDestroy(exec_);
-    if (graph_) (void)hipGraphDestroy(graph_);
   }
   ChunkLoop(const ChunkLoop&) = delete;
   ChunkLoop& operator=(const ChunkLoop&) = delete;
@@ -120,16 +132,16 @@ class ChunkLoop {
   const CGScalars* sc_;
   CGScalars* hsc_;
   int chunk_ = 8, max_chunks_ = 1, launched_ = 0;
-  hipGraphExec_t exec_ = nullptr;
-  hipGraph_t graph_ = nullptr;
+  hipGraphExec_t exec_ = nullptr;  // the slot's
+  GraphSlot own_;
 };
 
 // One solve's chunks with one host poll per chunk, until the device marks the solve done.
 // On return hsc holds the final scalars.
 template <class Iter, class Tail>
 void drive_chunks(const Iter& one_iter, const Tail& tail, const CGOptions& o, size_t n, hipStream_t st,
-                  const CGScalars* sc, CGScalars* hsc) {
-  ChunkLoop loop(one_iter, tail, o, n, st, sc, hsc);
+                  const CGScalars* sc, CGScalars* hsc, GraphSlot* slot = nullptr, const GraphKey& key = {}) {
+  ChunkLoop loop(one_iter, tail, o, n, st, sc, hsc, slot, key);
   do {
     loop.launch();
     QED3_HIP(hipStreamSynchronize(st));
@@ -165,11 +177,13 @@ __global__ __launch_bounds__(256) void k_init_h(const Spin<double>* __restrict__
 }
 
 // Half-storage flush: x64 += scale (x_inner + sum_j alpha_pend[j] ring[j]), x_inner = 0,
-// taking the x terms the current group's iterations left pending (alpha_pend[j] = 0 if none)
+// taking the x terms the current group's iterations left pending (alpha_pend[j] = 0 if none);
+// x64 = null: the solve's x of the scalars
 __global__ __launch_bounds__(256) void k_flush_h(Spin<double>* x64, Spin<float>* xin, PendRing ring,
                                                  size_t n, const CGScalars* sc, int always,
                                                  const phase16_t* rot) {
   if (!always && (sc->done != 0 || sc->need_ru == 0)) return;
+  if (!x64) x64 = sc->x;
   const double s = sc->scale;
   float ap[kXGroup - 1];
   for (int j = 0; j < kXGroup - 1; j++) ap[j] = float(sc->alpha_pend[j]);

@@ -41,7 +41,8 @@ struct EpiK1P : EpiK1<T> {
   __device__ void center(size_t i, const Spin<T>& v) const { st(pnew + i, v); }
 };
 
-// K2: q = D^dag w; x += alpha p; r -= alpha q; |r|^2 and the reliable-update decision
+// K2: q = D^dag w; x += alpha p; r -= alpha q; |r|^2 and the reliable-update decision.
+// x = null: the solve's x of the scalars (FP64)
 template <typename T>
 struct EpiK2 {
   static constexpr bool kReduce = true;
@@ -51,7 +52,12 @@ struct EpiK2 {
   CGScalars* sc;
   T alpha;
   __device__ bool skip() const { return sc->done != 0; }
-  __device__ void begin() { alpha = T(sc->alpha); }
+  __device__ void begin() {
+    alpha = T(sc->alpha);
+    if constexpr (std::is_same<T, double>::value) {
+      if (!x) x = sc->x;
+    }
+  }
   __device__ void operator()(size_t i, const Spin<T>& q, double2& acc) const {
     const Spin<T> pp = ld(p + i);
     Spin<T> xx = ld(x + i), rr = ld(r + i);
@@ -96,7 +102,14 @@ struct EpiStoreIfRU {
   __device__ void operator()(double2) const {}
 };
 
-// U3: r64 = b - D^dag t; r_inner = r64; |r64|^2 decides convergence and beta
+// U2's source: the solve's x of the scalars
+struct SrcSolX {
+  const CGScalars* sc;
+  __device__ SrcPlain<double> bind() const { return SrcPlain<double>{sc->x}; }
+};
+
+// U3: r64 = b - D^dag t; r_inner = r64; |r64|^2 decides convergence and beta (b = null, here
+// and in EpiResidH: the solve's b of the scalars)
 template <typename T>
 struct EpiResid {
   static constexpr bool kReduce = true;
@@ -104,7 +117,9 @@ struct EpiResid {
   Spin<T>* r;
   CGScalars* sc;
   __device__ bool skip() const { return sc->done != 0 || sc->need_ru == 0; }
-  __device__ void begin() {}
+  __device__ void begin() {
+    if (!b) b = sc->b;
+  }
   __device__ void operator()(size_t i, const Spin<double>& v, double2& acc) const {
     const Spin<double> bb = ld(b + i);
     Spin<double> rr;
@@ -260,7 +275,10 @@ struct EpiResidH {
   double inv_ncomp;  // 1 / (4 * points)
   double inv_so;
   __device__ bool skip() const { return sc->done != 0 || sc->need_ru == 0; }
-  __device__ void begin() { inv_so = 1.0 / sc->scale; }
+  __device__ void begin() {
+    inv_so = 1.0 / sc->scale;
+    if (!b) b = sc->b;
+  }
   __device__ void operator()(size_t i, const Spin<double>& v, double2& acc) const {
     const Spin<double> bb = ld(b + i);
     Spin<double> rr;

@@ -95,6 +95,8 @@ class Horner {
   // ---- building blocks of the preconditioned CG (pcg.hip) ----
   // Planar FP32 / binary16 work fields for n points (slot-owned, grown on demand)
   void* work(int slot, size_t bytes);
+  // the kept chunk graph of the preconditioned CG with this network
+  GraphSlot& graph_slot() { return graph_; }
 
  private:
   void upload_tables();
@@ -109,6 +111,7 @@ class Horner {
   size_t work_bytes_[kWorkSlots] = {};
   double* red_ = nullptr;  // reduction partials of the gradient kernels
   size_t red_n_ = 0;
+  GraphSlot graph_;
 };
 
 // Flexible CG (Notay's FCG(1)) on D^dagger D preconditioned by M = K K^dagger with the

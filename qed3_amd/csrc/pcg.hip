@@ -93,10 +93,12 @@ struct PendRing8 {
 // x64 += scale exp(-i phi) (x_inner + sum_j alpha_pend[j] ring[j]) (before a reliable
 // update, or always at the end).  Neither x64 nor x_inner is cleared at the start: each is
 // read only once it holds a value (sc->x_set, sc->xin_set), and x_inner counts as cleared
-// again after the update (its flag is reset by the update's last kernel).
-__global__ __launch_bounds__(256) void k_flush_f(Spin<double>* x64, Spin<float>* xin, PendRing8 ring, size_t n,
-                                                 const CGScalars* sc, int always, const phase16_t* rot) {
+// again after the update (its flag is reset by the update's last kernel).  x64 is the solve's
+// x of the scalars.
+__global__ __launch_bounds__(256) void k_flush_f(Spin<float>* xin, PendRing8 ring, size_t n, const CGScalars* sc,
+                                                 int always, const phase16_t* rot) {
   if (!always && (sc->done != 0 || sc->need_ru == 0)) return;
+  Spin<double>* x64 = sc->x;
   float ap[kFGroup];
 #pragma unroll
   for (int j = 0; j < kFGroup; j++) ap[j] = float(sc->alpha_pend[j]);
@@ -234,8 +236,12 @@ struct FinStartF {
   CGScalars* sc;
   double ncomp, tol2, delta2;
   int maxiter;
+  Spin<double>* x;
+  const Spin<double>* b;
   __device__ bool skip() const { return false; }
   __device__ void operator()(double2 t) const {
+    sc->x = x;
+    sc->b = b;
     half_start(sc, t.x, ncomp, tol2, delta2, maxiter);
     sc->fresh = 1;
     sc->rpend = 1.0;
@@ -266,14 +272,17 @@ __global__ __launch_bounds__(256) void k_store_b0_f(const Spin<double>* __restri
 // re-stored it); |r|^2 decides convergence, the new scale and beta as for the half-storage CG
 struct EpiResidF {
   static constexpr bool kReduce = true;
-  const Spin<double>* b;
   SpinH* r;
   CGScalars* sc;
   const phase16_t* rot;
   double inv_ncomp;
   double inv_so;
+  const Spin<double>* b;  // the solve's, from the scalars
   __device__ bool skip() const { return sc->done != 0 || sc->need_ru == 0; }
-  __device__ void begin() { inv_so = 1.0 / sc->scale; }
+  __device__ void begin() {
+    inv_so = 1.0 / sc->scale;
+    b = sc->b;
+  }
   __device__ void operator()(size_t i, const Spin<double>& v, double2& acc) const {
     const Spin<double> bb = ld(b + i);
     Spin<double> rr;
@@ -289,7 +298,7 @@ struct EpiResidF {
   __device__ void operator()(double2 t) const {
     sc->x_set = 1;    // the update's flush has written x
     sc->xin_set = 0;  // ... and taken x_inner
-    EpiResidH{b, nullptr, sc, inv_ncomp, 1.0}(t);
+    EpiResidH{nullptr, nullptr, sc, inv_ncomp, 1.0}(t);
     if (sc->done == 0) sc->rpend = sc->rfac;
   }
 };
@@ -451,7 +460,7 @@ CGResult pcg_solve(Horner& K, Spin<double>* x, const Spin<double>* b, const CGOp
   const int ngate = int(gated_blocks(n));
   hipLaunchKernelGGL(k_init_f, dim3(nbk), dim3(256), 0, st, b, ring[kFGroup - 1], n, gr);
   hipLaunchKernelGGL(k_finalize<FinStartF>, dim3(1), dim3(256), 0, st, gr.partials, unsigned(nbk),
-                     FinStartF{sc, 4.0 * double(n), o.tol * o.tol, o.delta * o.delta, o.maxiter});
+                     FinStartF{sc, 4.0 * double(n), o.tol * o.tol, o.delta * o.delta, o.maxiter, x, b});
   const DiracView<float, phase16_t> vin = D.view_half_temporal_gauge();
   const DiracView<float, phasepair_t> vpairs = D.view_half_tg_pairs();
   const phase16_t* rot = D.half_gauge_rotation();
@@ -490,10 +499,10 @@ CGResult pcg_solve(Horner& K, Spin<double>* x, const Spin<double>* b, const CGOp
   // one: with an update every three to four iterations (delta = 0.001), waiting for a
   // chunk's end would leave the rest of the chunk's iterations idle.
   auto reliable_update = [&] {
-    hipLaunchKernelGGL(k_flush_f, dim3(ngate), dim3(256), 0, st, x, xin, pend, n, sc, 0, rot);
-    launch_stencil<double, false>(v64, nn, x, EpiStoreIfRU{t, sc}, D.tile<double>(false), gr, st, hv64f);
-    launch_stencil<double, true>(v64, nn, t, EpiResidF{b, R, sc, rot, inv_ncomp, 1.0}, D.tile<double>(true), gr, st,
-                                 hv64t);
+    hipLaunchKernelGGL(k_flush_f, dim3(ngate), dim3(256), 0, st, xin, pend, n, sc, 0, rot);
+    launch_stencil_src<double, false>(v64, nn, SrcSolX{sc}, EpiStoreIfRU{t, sc}, D.tile<double>(false), gr, st, hv64f);
+    launch_stencil<double, true>(v64, nn, t, EpiResidF{R, sc, rot, inv_ncomp, 1.0, nullptr}, D.tile<double>(true), gr,
+                                 st, hv64t);
   };
   auto one_iter = [&](int i, int k) {
     const int pos = i % kFGroup;
@@ -512,10 +521,18 @@ CGResult pcg_solve(Horner& K, Spin<double>* x, const Spin<double>* b, const CGOp
   // ring positions run 0 .. kFGroup-1 within every chunk
   CGOptions oc = o;
   oc.chunk = ((o.chunk > 0 ? o.chunk : kFGroup) + kFGroup - 1) / kFGroup * kFGroup;
-  drive_chunks(one_iter, [] {}, oc, n, st, sc, hsc);
+  // (x and b are read from the scalars, so that the captured chunk serves every solve)
+  GraphKey key;
+  key.add(vin).add(vpairs).add(v64).add(hvf).add(hvt).add(hv64f).add(hv64t).add(halo).add(rot).add(sc).add(gr.partials);
+  key.add(D.tile<float>(false)).add(D.tile<float>(true)).add(D.tile<double>(false)).add(D.tile<double>(true));
+  key.add(hv.hrow16).add(hv.invc).add(hv.kt).add(hv.nslot).add(L).add(n).add(nn);
+  for (const std::complex<double>& c : K.params().c) key.add(c.real()).add(c.imag());
+  for (SpinH* p : ring) key.add(p);
+  key.add(w).add(xin).add(t).add(R).add(G[0]).add(G[1]).add(H[0]).add(H[1]).add(Z);
+  drive_chunks(one_iter, [] {}, oc, n, st, sc, hsc, &K.graph_slot(), key);
   timer.finish(hsc->iter);
   ltimer.finish(hsc->iter);
-  hipLaunchKernelGGL(k_flush_f, dim3(nbk), dim3(256), 0, st, x, xin, pend, n, sc, 1, rot);
+  hipLaunchKernelGGL(k_flush_f, dim3(nbk), dim3(256), 0, st, xin, pend, n, sc, 1, rot);
   QED3_HIP(hipMemcpyAsync(hsc, sc, sizeof(CGScalars), hipMemcpyDeviceToHost, st));
   QED3_HIP(hipStreamSynchronize(st));
   CGResult res;
