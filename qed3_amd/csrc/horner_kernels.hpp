@@ -380,10 +380,10 @@ inline void launch_horner_layer(const HornerView& hv, const DiracView<float, P>&
 // binary16 (cos, sin) pairs with the hardware sine and cosine.  The rounding (at most
 // pi/1024 rad) is of the order of the binary16 arithmetic's and only enters the
 // preconditioner.
-constexpr int kTcChunk = 16;   // slices per lane
 constexpr int kTcDepth = 2;    // steps whose loads are in flight ahead of the one computed
-constexpr int kTcBlock = 256;  // most threads per block (S sites x C lanes)
-constexpr int kTcSites = 256;  // most sites per block
+// most threads per block (S sites x C lanes) with T slices per lane: the short chunks leave the
+// registers for twice the lanes
+constexpr int tc_block(int T) { return T == 16 ? 256 : 512; }
 
 // LDS written by threads of a wave and read back by other threads of the same wave: the wave
 // executes its LDS instructions in order, so only the compiler must keep them in order
@@ -400,7 +400,7 @@ __device__ __forceinline__ void wave_sync() {
 // whole halo) and alone reads it, so the per-step staging needs no block barrier.
 template <int NS, bool ADJ, bool FIRST, int T, class Src, class Epi, bool FUSE = false, bool UL = false,
           bool H2 = false, bool WS = false>
-__global__ __launch_bounds__(kTcBlock, (NS == 3 ? 4 : 2)) void k_horner_layer_tc(HornerView hv, DiracView<float, phasepair_t> d,
+__global__ __launch_bounds__(tc_block(T), (NS == 3 ? 4 : 2)) void k_horner_layer_tc(HornerView hv, DiracView<float, phasepair_t> d,
                                                          HaloView halo, Src src, const SpinH* __restrict__ gin,
                                                          SpinH* __restrict__ gout, float2 cj, TileMap tm, Epi epi,
                                                          GridReduce gr, int C, SpinH* __restrict__ gout2,
@@ -419,8 +419,8 @@ __global__ __launch_bounds__(kTcBlock, (NS == 3 ? 4 : 2)) void k_horner_layer_tc
   const int sl = int(threadIdx.x) - lane * S;
   SpinH* tile = reinterpret_cast<SpinH*>(hk_tile_raw);         // [2][C][S + hmax]
   const int row = S + halo.hmax;
-  float2* carry = reinterpret_cast<float2*>(tile + (FIRST ? 0 : 2 * C * row));  // [2][kTcBlock]
-  HopRow16* hqs = reinterpret_cast<HopRow16*>(carry + 2 * kTcBlock);  // [S][2 rows][NS], the sites' hop rows
+  float2* carry = reinterpret_cast<float2*>(tile + (FIRST ? 0 : 2 * C * row));  // [2][blockDim]
+  HopRow16* hqs = reinterpret_cast<HopRow16*>(carry + 2 * blockDim.x);  // [S][2 rows][NS], the sites' hop rows
   int xr, st_;
   tile_of(tm, blockIdx.x, xr, st_);
   (void)st_;
@@ -707,26 +707,54 @@ __global__ __launch_bounds__(kTcBlock, (NS == 3 ? 4 : 2)) void k_horner_layer_tc
   }
 }
 
-// Lanes per site of the parallel-in-time layer: C = ceil(Lt / T) rounded up to a power of
-// two (C * S <= kTcBlock threads, S <= kTcSites sites); at most 64.
-inline int tc_lanes(int Lt) {
-  const int c = (Lt + kTcChunk - 1) / kTcChunk;
-  int p = 1;
-  while (p < c) p <<= 1;
-  if (p > 64) throw std::invalid_argument("time extent too long for the parallel-in-time layer");
-  return p;
+// Shape of the parallel-in-time layer: T slices per lane, C = ceil(Lt / T) lanes per site, S
+// sites per block.  Up to 64 slices a lane is one wave (S = 64), which stages its own tile
+// without block barriers; longer columns split a block of 256 threads over more lanes (C a
+// power of two, at most 64) and synchronise per step.
+constexpr long kTcSimds = 1024;
+struct TcShape {
+  int T, C, S;
+};
+inline int tc_sites(int Lt) {
+  if (Lt <= 64) return 64;
+  int c = 8;
+  while (c * 16 < Lt) c <<= 1;
+  if (c > 64) throw std::invalid_argument("time extent too long for the parallel-in-time layer");
+  return 256 / c;
 }
-inline int tc_sites(int Lt) { return std::min(kTcSites, kTcBlock / tc_lanes(Lt)); }
+// A lane's steps are a serial chain of loads, so the fewer waves there are the shorter its
+// chunk should be; the longer one spends less on carries and on the wrap terms once the GPU is
+// full.  Learned solves, T = 4 / 8 / 16 in us (waves with T = 8): simplicial n=16, Lt=16: 1001 /
+// 1135 / 1484 (82); dual n=24, Lt=20: 1347 / 1436 / 1755 (540); simplicial n=64, Lt=32: 2742 /
+// 2605 / 2871 (2,564); dual n=64, Lt=32: 4064 / 3808 / 3957 (5,120); simplicial n=128, Lt=64:
+// - / 13242 / 13102 (20,488).  So: 4 while chunks of 8 would leave some of the 1,024 SIMDs
+// without a wave, 16 from ten waves a SIMD on; and 16 where more lanes' tiles would not fit in
+// LDS (halos of several times the range, as of randomly numbered tables).
+constexpr size_t kTcLds = 64 * 1024;
+inline size_t tc_smem(int C, int S, int nslot, bool first, int hmax) {
+  return (first ? 0 : size_t(2) * C * (S + hmax) * sizeof(SpinH) + size_t(S) * 2 * nslot * sizeof(HopRow16)) +
+         size_t(2) * C * S * sizeof(float2);
+}
+inline TcShape tc_shape(int V, int Lt, int nslot, bool first, int hmax) {
+  const int S = tc_sites(Lt);
+  if (S != 64) return {16, 256 / S, S};
+  auto lanes = [&](int T) { return (Lt + T - 1) / T; };
+  auto waves = [&](int T) { return long((V + S - 1) / S) * lanes(T); };
+  int T = waves(16) > 10 * kTcSimds ? 16 : (waves(8) <= kTcSimds && lanes(4) * S <= tc_block(4) ? 4 : 8);
+  if (tc_smem(lanes(T), S, nslot, first, hmax) > kTcLds) T = 16;
+  return {T, lanes(T), S};
+}
 
 // gout2 != nullptr (ADJ only): also K's first layer with coefficient cj2 into gout2 (FUSE).
 template <bool ADJ, bool FIRST, class Src, class Epi>
-inline void launch_horner_layer_tc(const HornerView& hv, const DiracView<float, phasepair_t>& tables,
+void launch_horner_layer_tc(const HornerView& hv, const DiracView<float, phasepair_t>& tables,
                                    const HaloView& halo, const Src& src, const SpinH* gin, SpinH* gout, float2 cj,
                                    const Epi& epi, GridReduce gr, hipStream_t st, const hipEvent_t* bracket = nullptr,
                                    SpinH* gout2 = nullptr, float2 cj2 = {0.f, 0.f}) {
   if (gout2 && !ADJ) throw std::logic_error("only a K^dagger layer carries K's first layer");
   if (gout2 && (gout2 == gout || gout2 == gin)) throw std::logic_error("fused output aliases an operand");
-  const int C = tc_lanes(hv.Lt), S = tc_sites(hv.Lt);
+  const TcShape sh = tc_shape(hv.V, hv.Lt, hv.nslot, FIRST, FIRST ? 0 : halo.hmax);
+  const int C = sh.C, S = sh.S;
   if (!tables.uPoly || !tables.uSite10)
     throw std::logic_error("parallel-in-time layer needs the temporal gauge");
   if (!FIRST && !halo.nbl) throw std::logic_error("parallel-in-time layer launched without halo tables");
@@ -737,48 +765,48 @@ inline void launch_horner_layer_tc(const HornerView& hv, const DiracView<float, 
   tm.remap = 1;
   const unsigned nblk = unsigned(tm.nxr_pad);
   if (Epi::kReduce && nblk > kReduceCapacity) throw std::invalid_argument("layer grid exceeds the reduction scratch");
-  const size_t smem =
-      (FIRST ? 0 : size_t(2) * C * (S + halo.hmax) * sizeof(SpinH)) + size_t(2) * kTcBlock * sizeof(float2) +
-      (FIRST ? 0 : size_t(S) * 2 * hv.nslot * sizeof(HopRow16));
-  if (smem > 64 * 1024) throw std::invalid_argument("parallel-in-time layer: halo too large for LDS");
+  const size_t smem = tc_smem(C, S, hv.nslot, FIRST, FIRST ? 0 : halo.hmax);
+  if (smem > kTcLds) throw std::invalid_argument("parallel-in-time layer: halo too large for LDS");
   if (size_t(hv.V) * size_t(hv.Lt) * sizeof(SpinH) > 0xffffffffull ||
       size_t(hv.V) * size_t((hv.nslot + 2) / 3) * size_t(hv.Lt) * sizeof(unsigned) > 0xffffffffull)
     throw std::invalid_argument("parallel-in-time layer: fields beyond 32-bit offsets");
   if (bracket) QED3_HIP(hipEventRecord(bracket[0], st));
-  auto go = [&](auto fuse, auto ul, auto h2, auto ws) {
+  auto go = [&](auto fuse, auto t, auto ws, auto h2) {
     constexpr bool F = decltype(fuse)::value && ADJ;
-    constexpr bool U = decltype(ul)::value;
+    constexpr bool U = decltype(ws)::value;
     constexpr bool H = decltype(h2)::value && !FIRST;
-    constexpr bool W = decltype(ws)::value && U && !FIRST;
+    constexpr bool W = U && !FIRST;
+    constexpr int T = decltype(t)::value;
     if (hv.nslot == 6)
-      hipLaunchKernelGGL((k_horner_layer_tc<6, ADJ, FIRST, kTcChunk, Src, Epi, F, U, H, W>), dim3(nblk),
-                         dim3(C * S), smem, st, hv, tables, halo, src, gin, gout, cj, tm, epi, gr, C, gout2, cj2);
+      hipLaunchKernelGGL((k_horner_layer_tc<6, ADJ, FIRST, T, Src, Epi, F, U, H, W>), dim3(nblk), dim3(C * S), smem, st,
+                         hv, tables, halo, src, gin, gout, cj, tm, epi, gr, C, gout2, cj2);
     else
-      hipLaunchKernelGGL((k_horner_layer_tc<3, ADJ, FIRST, kTcChunk, Src, Epi, F, U, H, W>), dim3(nblk),
-                         dim3(C * S), smem, st, hv, tables, halo, src, gin, gout, cj, tm, epi, gr, C, gout2, cj2);
+      hipLaunchKernelGGL((k_horner_layer_tc<3, ADJ, FIRST, T, Src, Epi, F, U, H, W>), dim3(nblk), dim3(C * S), smem, st,
+                         hv, tables, halo, src, gin, gout, cj, tm, epi, gr, C, gout2, cj2);
   };
-  // the wave-uniform form where a wave's 64 threads belong to one lane (S a multiple of 64),
-  // wave-synchronous where a lane is exactly one wave (S = 64); the second halo load only
-  // where some block's halo is longer than its range
-  const bool ul = S % 64 == 0, ws = S == 64, h2 = !FIRST && halo.hmax > S;
-  auto go2 = [&](auto fuse) {
-    if (ws && h2)
-      go(fuse, std::true_type{}, std::true_type{}, std::true_type{});
-    else if (ws)
-      go(fuse, std::true_type{}, std::false_type{}, std::true_type{});
-    else if (ul && h2)
-      go(fuse, std::true_type{}, std::true_type{}, std::false_type{});
-    else if (ul)
-      go(fuse, std::true_type{}, std::false_type{}, std::false_type{});
-    else if (h2)
-      go(fuse, std::false_type{}, std::true_type{}, std::false_type{});
+  // wave-uniform and wave-synchronous where a lane is one wave (S = 64); the second halo load
+  // only where some block's halo is longer than its range
+  const bool h2 = !FIRST && halo.hmax > S;
+  auto go2 = [&](auto fuse, auto t, auto ws) {
+    if (h2)
+      go(fuse, t, ws, std::true_type{});
     else
-      go(fuse, std::false_type{}, std::false_type{}, std::false_type{});
+      go(fuse, t, ws, std::false_type{});
+  };
+  auto go3 = [&](auto fuse) {
+    if (S != 64)
+      go2(fuse, std::integral_constant<int, 16>{}, std::false_type{});
+    else if (sh.T == 16)
+      go2(fuse, std::integral_constant<int, 16>{}, std::true_type{});
+    else if (sh.T == 8)
+      go2(fuse, std::integral_constant<int, 8>{}, std::true_type{});
+    else
+      go2(fuse, std::integral_constant<int, 4>{}, std::true_type{});
   };
   if (gout2)
-    go2(std::true_type{});
+    go3(std::true_type{});
   else
-    go2(std::false_type{});
+    go3(std::false_type{});
   if (bracket) QED3_HIP(hipEventRecord(bracket[1], st));
   if constexpr (Epi::kReduce)
     hipLaunchKernelGGL((k_finalize<Epi>), dim3(1), dim3(256), 0, st, gr.partials, nblk, epi);

@@ -23,14 +23,21 @@
 #include "cg_drive.hpp"
 #include "cg_epi.hpp"
 #include "horner.hpp"
-#include "horner_kernels.hpp"
+#include "pcg_layers.hpp"
 #include "stencil.hpp"
 
 namespace qed3 {
+#define QED3_TC_EXTERN(...) extern QED3_TC_LAUNCH(__VA_ARGS__)
+QED3_TC_KDAG(QED3_TC_EXTERN)
+QED3_TC_K(QED3_TC_EXTERN)
+QED3_TC_CHECK(QED3_TC_EXTERN)
+
 namespace {
 
 using namespace cgepi;
 using namespace cgdrive;
+using pcgl::EpiFcg;
+using pcgl::EpiSkip;
 
 
 // The directions of the last kFGroup iterations stay in a ring of buffers and their x terms
@@ -195,42 +202,6 @@ __global__ __launch_bounds__(256) void k_init_f(const Spin<double>* __restrict__
   }
   store_partial(acc, gr.partials, blockIdx.x);
 }
-
-// the network's layers wait, like K1 and K2, for a pending reliable update
-struct EpiSkip {
-  static constexpr bool kReduce = false;
-  const CGScalars* sc;
-  __device__ bool skip() const { return sc->done != 0 || sc->need_ru != 0; }
-  __device__ void operator()(size_t, const Spin<float>&, double2&) const {}
-  __device__ void operator()(double2) const {}
-};
-
-// Last layer of K, injecting H = K^dagger r as stored beside H_old (hk::SrcDots), which
-// reduces t = (|H|^2, <H_old, H>) = (<r, z>, <r_old, z>): the FCG scalars.  After a reliable
-// update r is the true residual at the new scale while H_old and p_old are at the old one
-// (rfac = old / new): beta = (|H|^2 - rfac <H_old, H>) / (rfac rho_old).
-struct EpiFcg {
-  static constexpr bool kReduce = true;
-  CGScalars* sc;
-  __device__ bool skip() const { return sc->done != 0 || sc->need_ru != 0; }
-  __device__ void operator()(size_t, const Spin<float>&, double2&) const {}
-  __device__ void operator()(double2 t) const {
-    const double A = t.x, Bv = t.y;
-    if (!(A > 0.0 && A < 1e300) || (!sc->fresh && !(fabs(Bv) < 1e300))) {
-      sc->done = 2;  // M r must be a descent direction: <r, M r> > 0
-      return;
-    }
-    double beta = 0.0;
-    if (!sc->fresh) {
-      const double f = sc->rescale ? sc->rfac : 1.0;
-      beta = (A - f * Bv) / (f * sc->rho);
-    }
-    sc->beta = beta;
-    sc->rho = A;
-    sc->mu = A;  // K1: alpha = mu / |D p|^2
-    sc->fresh = 0;
-  }
-};
 
 struct FinStartF {
   CGScalars* sc;
