@@ -169,6 +169,16 @@ struct FinOut {
   __device__ void operator()(double2 t) const { *out = t; }
 };
 
+// After a reliable update at the end of a chunk the next iteration is a chunk's first, which
+// reads p_old from the buffer `dst`: the last direction is copied there if it is in `src`
+template <typename T>
+__global__ __launch_bounds__(256) void k_keep_p(const Spin<T>* __restrict__ src, Spin<T>* dst, size_t n,
+                                                const CGScalars* sc) {
+  if (sc->done != 0 || sc->rescale == 0 || sc->last_pos == 0) return;
+  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x)
+    dst[i] = src[i];
+}
+
 template <typename T>
 struct Work {
   Spin<T>* r = nullptr;
@@ -224,7 +234,25 @@ CGResult run_cg(Dirac& D, Spin<double>* x, const Spin<double>* b, const CGOption
   // No kernel is given x or b: they take them from the scalars, so that the captured chunk
   // serves every solve on this context.
   Spin<T>* P[2] = {W.p, W.p2};
+  // The reliable update (FP64: the confirmation of the stop test) runs once per chunk: an
+  // iteration that asks for it makes the rest of the chunk's iterations exit at once.  After
+  // every iteration its three kernels and finaliser, idle but for one iteration of a solve
+  // (FP64) or of some thirty (mixed), took a quarter of a small lattice's iteration.  With
+  // kernel timing, whose events must each bracket a real iteration, it follows each.
   EventTimer timer(o.times);
+  const bool ru_each = o.times != nullptr;
+  auto reliable_update = [&] {
+    if (kMixed)
+      hipLaunchKernelGGL(k_flush<T>, dim3(ngate), dim3(256), 0, st, W.xin, n, sc, 0);
+    launch_stencil_src<double, false>(v64, nn, SrcSolX{sc}, EpiStoreIfRU{W.t, sc}, D.tile<double>(false), gr, st,
+                                      hv64f);
+    launch_stencil<double, true>(v64, nn, W.t, EpiResid<T>{nullptr, W.r, sc}, D.tile<double>(true), gr, st, hv64t);
+  };
+  auto tail = [&] {
+    if (ru_each) return;
+    reliable_update();
+    hipLaunchKernelGGL(k_keep_p<T>, dim3(ngate), dim3(256), 0, st, W.p2, W.p, n, sc);
+  };
   auto one_iter = [&](int i, int k) {
     const int par = i & 1;
     Spin<T>* pold = P[par];
@@ -235,20 +263,16 @@ CGResult run_cg(Dirac& D, Spin<double>* x, const Spin<double>* b, const CGOption
     k1.pnew = pnew;
     launch_stencil_src<T, false>(vin, nn, SrcPUpdate<T>{W.r, pold, sc}, k1, D.tile<T>(false), gr, st, hvf,
                                  timer.pair(0, k));
-    launch_stencil_src<T, true>(vin, nn, SrcPlain<T>{W.w}, EpiK2<T>{W.xin, W.r, pnew, sc, T(0)},
+    launch_stencil_src<T, true>(vin, nn, SrcPlain<T>{W.w}, EpiK2<T>{W.xin, W.r, pnew, sc, T(0), par ^ 1},
                                 D.tile<T>(true), gr, st, hvt, timer.pair(1, k));
-    if (kMixed)
-      hipLaunchKernelGGL(k_flush<T>, dim3(ngate), dim3(256), 0, st, W.xin, n, sc, 0);
-    launch_stencil_src<double, false>(v64, nn, SrcSolX{sc}, EpiStoreIfRU{W.t, sc}, D.tile<double>(false), gr, st,
-                                      hv64f);
-    launch_stencil<double, true>(v64, nn, W.t, EpiResid<T>{nullptr, W.r, sc}, D.tile<double>(true), gr, st, hv64t);
+    if (ru_each) reliable_update();
   };
 
   GraphKey key;
   key.add(vin).add(v64).add(hvf).add(hvt).add(hv64f).add(hv64t).add(D.tile<T>(false)).add(D.tile<T>(true));
   key.add(D.tile<double>(false)).add(D.tile<double>(true)).add(W.r).add(W.p).add(W.p2).add(W.w).add(W.xin).add(W.t);
   key.add(sc).add(gr.partials).add(n).add(nn);
-  drive_chunks(one_iter, [] {}, o, n, st, sc, hsc, &D.graph_slot(kMixed ? 1 : 0), key);
+  drive_chunks(one_iter, tail, o, n, st, sc, hsc, &D.graph_slot(kMixed ? 1 : 0), key);
   timer.finish(hsc->iter);
   if (o.times) o.times->ms[2] = o.times->ms[1], o.times->count[2] = o.times->count[1];
   if (kMixed) hipLaunchKernelGGL(k_flush<T>, dim3(nbk), dim3(256), 0, st, W.xin, n, sc, 1);
@@ -486,15 +510,18 @@ CGResult cg_solve_f64_workspace(Dirac& D, Spin<double>* x, const Spin<double>* b
     k1.sc = sc;
     k1.pnew = P[par ^ 1];
     launch_stencil_src<double, false>(v64, nn, SrcPUpdate<double>{r, P[par], sc}, k1, tf, gr, st, hvf);
-    launch_stencil_src<double, true>(v64, nn, SrcPlain<double>{w}, EpiK2<double>{x, r, P[par ^ 1], sc, 0.0}, tt, gr,
-                                     st, hvt);
+    launch_stencil_src<double, true>(v64, nn, SrcPlain<double>{w}, EpiK2<double>{x, r, P[par ^ 1], sc, 0.0, par ^ 1}, tt,
+                                     gr, st, hvt);
+  };
+  auto tail = [&] {
     launch_stencil<double, false>(v64, nn, x, EpiStoreIfRU{w, sc}, tf, gr, st, hvf);
     launch_stencil<double, true>(v64, nn, w, EpiResid<double>{b, r, sc}, tt, gr, st, hvt);
+    hipLaunchKernelGGL(k_keep_p<double>, dim3(unsigned(gated_blocks(n))), dim3(256), 0, st, P[1], P[0], n, sc);
   };
   CGOptions od = o;
   od.use_graph = false;
   od.times = nullptr;
-  drive_chunks(one_iter, [] {}, od, n, st, sc, &hsc);
+  drive_chunks(one_iter, tail, od, n, st, sc, &hsc);
   QED3_HIP(hipMemcpyAsync(&hsc, sc, sizeof(CGScalars), hipMemcpyDeviceToHost, st));
   QED3_HIP(hipStreamSynchronize(st));
   CGResult res;

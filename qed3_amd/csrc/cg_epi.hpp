@@ -24,13 +24,18 @@ struct EpiK1 {
   static constexpr bool kReduce = true;
   Spin<T>* w;
   CGScalars* sc;
-  __device__ bool skip() const { return sc->done != 0; }
+  // an iteration after one that asked for a reliable update waits for it (the update runs once
+  // per chunk of iterations)
+  __device__ bool skip() const { return sc->done != 0 || sc->need_ru != 0; }
   __device__ void begin() {}
   __device__ void operator()(size_t i, const Spin<T>& v, double2& acc) const {
     st(w + i, v);
     acc.x += norm2(v);
   }
-  __device__ void operator()(double2 t) const { k1_finish(sc, t.x); }
+  __device__ void operator()(double2 t) const {
+    sc->rescale = 0;
+    k1_finish(sc, t.x);
+  }
 };
 
 // K1 reading p = r + beta p_old (SrcPUpdate) and storing that p at every point it owns for
@@ -42,7 +47,7 @@ struct EpiK1P : EpiK1<T> {
 };
 
 // K2: q = D^dag w; x += alpha p; r -= alpha q; |r|^2 and the reliable-update decision.
-// x = null: the solve's x of the scalars (FP64)
+// x = null: the solve's x of the scalars (FP64); pos: the buffer that holds this p
 template <typename T>
 struct EpiK2 {
   static constexpr bool kReduce = true;
@@ -51,7 +56,8 @@ struct EpiK2 {
   const Spin<T>* p;
   CGScalars* sc;
   T alpha;
-  __device__ bool skip() const { return sc->done != 0; }
+  int pos;
+  __device__ bool skip() const { return sc->done != 0 || sc->need_ru != 0; }
   __device__ void begin() {
     alpha = T(sc->alpha);
     if constexpr (std::is_same<T, double>::value) {
@@ -75,6 +81,7 @@ struct EpiK2 {
   }
   __device__ void operator()(double2 t) const {
     const double m = t.x;
+    sc->last_pos = pos;
     sc->iter += 1;
     if (!(m >= 0.0 && m < 1e300)) {
       sc->done = 2;
@@ -147,6 +154,7 @@ struct EpiResid {
     sc->beta = m / sc->mu;
     sc->mu = m;
     sc->maxr2 = m;
+    sc->rescale = 1;  // an update has run since the last K1
     if (sc->iter >= sc->maxiter) sc->done = 3;
   }
 };
