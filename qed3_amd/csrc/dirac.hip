@@ -355,6 +355,18 @@ CGScalars* Dirac::host_scalars() {
   return hsc_;
 }
 
+void* Dirac::host_block(size_t bytes) {
+  if (hblock_bytes_ < bytes) {
+    QED3_HIP(hipStreamSynchronize(stream_));
+    if (hblock_) QED3_HIP(hipHostFree(hblock_));
+    hblock_ = nullptr;
+    hblock_bytes_ = 0;
+    QED3_HIP(hipHostMalloc(&hblock_, bytes, hipHostMallocDefault));
+    hblock_bytes_ = bytes;
+  }
+  return hblock_;
+}
+
 Dirac::~Dirac() {
   if (stream_) (void)hipStreamSynchronize(stream_);  // work queued on a caller's stream
   auto f = [](void* p) {
@@ -362,6 +374,7 @@ Dirac::~Dirac() {
   };
   for (void* p : scratch_) f(p);
   if (hsc_) (void)hipHostFree(hsc_);
+  if (hblock_) (void)hipHostFree(hblock_);
   for (void* p : {(void*)d64_.nbr, (void*)d64_.lnk, (void*)d64_.hop, (void*)d64_.hopd,
                   (void*)d64_.diag, (void*)d64_.kth, (void*)d64_.uS, (void*)d64_.uT,
                   (void*)d32_.nbr, (void*)d32_.lnk, (void*)d32_.hop, (void*)d32_.hopd,

@@ -217,15 +217,19 @@ class Dirac {
   GridReduce reducer() const { return {partials_, counter_}; }
   // Device work buffer `slot` of at least `bytes`, kept across calls (grown on demand,
   // freed with the context), so repeated solves allocate nothing; contents are undefined.
-  // Slots are owned by the CG solvers (cg.hip); calls on one context are sequential.
-  static constexpr int kScratchSlots = 14;
+  // Slots are owned by the CG solvers (cg.hip), the last by the multi-shift CG (msolve.hip);
+  // calls on one context are sequential.
+  static constexpr int kScratchSlots = 15;
   void* scratch(int slot, size_t bytes);
   void release_scratch();
-  // the kept chunk graphs of the solvers on this context (0 FP64, 1 mixed, 2 half storage)
-  static constexpr int kGraphSlots = 3;
+  // the kept chunk graphs of the solvers on this context (0 FP64, 1 mixed, 2 half storage,
+  // 3 multi-shift)
+  static constexpr int kGraphSlots = 4;
   GraphSlot& graph_slot(int k) { return graphs_[k]; }
   // pinned host copy of the solver scalars (same lifetime)
   CGScalars* host_scalars();
+  // pinned host memory of at least `bytes` for results read back (kept, grown on demand)
+  void* host_block(size_t bytes);
   // LDS halo tables for ranges of R sites (built on first use)
   HaloView halo(int R);
   bool has_halo(int R) const { return halos_.count(R) != 0; }
@@ -285,6 +289,8 @@ class Dirac {
   void* scratch_[kScratchSlots] = {};
   size_t scratch_bytes_[kScratchSlots] = {};
   CGScalars* hsc_ = nullptr;
+  void* hblock_ = nullptr;
+  size_t hblock_bytes_ = 0;
   GraphSlot graphs_[kGraphSlots];
 };
 

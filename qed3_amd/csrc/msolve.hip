@@ -48,140 +48,235 @@ __global__ __launch_bounds__(256) void k_pair_norms(const Spin<double>* __restri
 }
 
 // ---- device-driven multi-shift CG: every scalar recursion runs in one-block finalisers, so a
-// chunk of iterations is one graph replay and the host polls once per chunk ----------------
+// chunk of iterations is one graph replay and the host polls once per chunk.  An iteration is
+//   w = D p with |w|^2, |p|^2;  alpha, zeta_i, alpha_i
+//   r -= alpha (D^dag w + s0 p) with |r|^2;  beta, beta_i, convergence
+//   x_i += alpha_i p_i, p_i = zeta_i r + beta_i p_i (one read of p_i), p = r + beta p
+// so neither norm nor update has a pass of its own and D^dag w is never stored.  The smallest
+// shift s0 is the one CG runs on (zeta = 1): its p_i is p.  On a small lattice the launches are
+// the cost: five an iteration instead of seven, and the scalars' recursions one lane a shift
+// instead of one thread for all (finalisers 4.8 -> 2.9 us with ten shifts); overlap operator at
+// simplicial n=16, Lt=16, degree 21: 7.4 -> 4.9 ms.
 struct MSScalars {
   double rho, bn2, alpha, beta, a_prev, b_prev, s0, tol2;
   double shift[kMaxShifts], z[kMaxShifts], zo[kMaxShifts], zn[kMaxShifts], ai[kMaxShifts], bi[kMaxShifts];
   int active[kMaxShifts];  // still iterating
-  int now[kMaxShifts];     // active in the current iteration (what K_a and K_b update)
+  int now[kMaxShifts];     // active in the current iteration (what the update pass works on)
   int iters[kMaxShifts];
+  Spin<double>* x[kMaxShifts];  // the caller's solutions (not in the captured arguments)
   int ns, it, maxiter;
   int done;  // 0 running, 1 every shift converged, 3 iteration cap, 4 breakdown
+  int update;  // the update pass of the current iteration is due
 };
 
 struct ShiftPtrs {
-  Spin<double>* x[kMaxShifts];
   Spin<double>* p[kMaxShifts];
-  int n;
+  int n, base;  // base: the smallest shift, whose p_i is p
 };
 
-// D or D^dag into out, skipped once the solve is done
-struct EpiStoreMS {
-  static constexpr bool kReduce = false;
-  Spin<double>* out;
+struct ShiftVals {
+  double s[kMaxShifts];
+  Spin<double>* x[kMaxShifts];
+};
+
+// r = p = p_i = b, x_i = 0, partial |b|^2
+__global__ __launch_bounds__(256) void k_ms_init(const Spin<double>* __restrict__ b, Spin<double>* r, Spin<double>* p,
+                                                 ShiftPtrs S, ShiftVals X, size_t n, double2* partials) {
+  double2 acc = {0.0, 0.0};
+  Spin<double> z;
+  z.a = {0.0, 0.0};
+  z.b = {0.0, 0.0};
+  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x) {
+    const Spin<double> v = b[i];
+    acc.x += nrm2(v);
+    r[i] = v;
+    p[i] = v;
+    for (int k = 0; k < S.n; k++) {
+      X.x[k][i] = z;
+      if (k != S.base) S.p[k][i] = v;
+    }
+  }
+  store_partial(acc, partials, blockIdx.x);
+}
+
+struct FinMSStart {
+  MSScalars* sc;
+  ShiftVals X;
+  int ns, maxiter;
+  double s0, tol2;
+  __device__ bool skip() const { return false; }
+  __device__ void operator()(double2 t) const {
+    const double b2 = t.x;
+    sc->rho = sc->bn2 = b2;
+    sc->alpha = sc->beta = 0.0;
+    sc->a_prev = 1.0;
+    sc->b_prev = 0.0;
+    sc->s0 = s0;
+    sc->tol2 = tol2;
+    sc->ns = ns;
+    sc->it = 0;
+    sc->maxiter = maxiter;
+    sc->update = 0;
+    for (int i = 0; i < ns; i++) {
+      sc->shift[i] = X.s[i];
+      sc->x[i] = X.x[i];
+      sc->z[i] = sc->zo[i] = sc->zn[i] = 1.0;
+      sc->active[i] = b2 > 0 ? 1 : 0;
+      sc->iters[i] = 0;
+    }
+    sc->done = (b2 > 0 && maxiter > 0) ? 0 : (b2 > 0 ? 3 : 1);
+  }
+};
+
+// w = D p, partials of (|w|^2, |p|^2)
+struct EpiMSD {
+  static constexpr bool kReduce = true;
+  static constexpr bool kOwnFinaliser = true;
+  Spin<double>* w;
+  const Spin<double>* p;
   const MSScalars* sc;
   __device__ bool skip() const { return sc->done != 0; }
   __device__ void begin() {}
-  __device__ void operator()(size_t i, const Spin<double>& v, double2&) const { out[i] = v; }
-  __device__ void operator()(double2) const {}
+  __device__ void operator()(size_t i, const Spin<double>& v, double2& acc) const {
+    st(w + i, v);
+    acc.x += nrm2(v);
+    acc.y += nrm2(ld(p + i));
+  }
 };
 
-// partials of (|w|^2, |p|^2)
-__global__ __launch_bounds__(256) void k_msd_norms(const Spin<double>* __restrict__ w,
-                                                   const Spin<double>* __restrict__ p, size_t n,
-                                                   double2* partials, const MSScalars* sc) {
-  if (sc->done != 0) return;
-  double2 acc = {0.0, 0.0};
-  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x) {
-    acc.x += nrm2(w[i]);
-    acc.y += nrm2(p[i]);
-  }
-  store_partial(acc, partials, blockIdx.x);
-}
-
-// alpha = rho / <p, (A + s0) p>; zeta_i and alpha_i of every active shift (Jegerlehner)
-struct FinMSAlpha {
-  MSScalars* sc;
+// r -= alpha (D^dag w + s0 p), partials of |r|^2
+struct EpiMSDdag {
+  static constexpr bool kReduce = true;
+  static constexpr bool kOwnFinaliser = true;
+  Spin<double>* r;
+  const Spin<double>* p;
+  const MSScalars* sc;
+  double alpha, as0;
   __device__ bool skip() const { return sc->done != 0; }
-  __device__ void operator()(double2 t) const {
-    const double pq = t.x + sc->s0 * t.y;
-    if (!(pq > 0.0) || !(pq < 1e300)) {
-      sc->done = 4;
-      return;
-    }
-    const double alpha = sc->rho / pq, ap = sc->a_prev, bp = sc->b_prev;
-    sc->alpha = alpha;
-    for (int i = 0; i < sc->ns; i++) {
-      sc->now[i] = sc->active[i];
-      if (!sc->active[i]) continue;
-      const double ds = sc->shift[i] - sc->s0, z = sc->z[i], zo = sc->zo[i];
-      const double zn = z * zo * ap / (alpha * bp * (zo - z) + zo * ap * (1.0 + ds * alpha));
-      sc->zn[i] = zn;
-      sc->ai[i] = alpha * zn / z;
-    }
+  __device__ void begin() {
+    alpha = sc->alpha;
+    as0 = sc->alpha * sc->s0;
   }
-};
-
-// r -= alpha (q + s0 p); x_i += alpha_i p_i for the shifts active now; partial |r|^2
-__global__ __launch_bounds__(256) void k_msd_a(Spin<double>* r, const Spin<double>* __restrict__ q,
-                                               const Spin<double>* __restrict__ p, ShiftPtrs S, size_t n,
-                                               double2* partials, const MSScalars* sc) {
-  if (sc->done != 0) return;
-  const double alpha = sc->alpha, s0 = sc->s0;
-  double2 acc = {0.0, 0.0};
-  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x) {
-    const Spin<double> pp = p[i], qq = q[i];
-    Spin<double> rr = r[i];
-    axpy_(rr, -alpha, qq);
-    axpy_(rr, -alpha * s0, pp);
-    r[i] = rr;
+  __device__ void operator()(size_t i, const Spin<double>& q, double2& acc) const {
+    Spin<double> rr = ld(r + i);
+    axpy_(rr, -alpha, q);
+    axpy_(rr, -as0, ld(p + i));
+    st(r + i, rr);
     acc.x += nrm2(rr);
-    for (int k = 0; k < S.n; k++) {
-      if (!sc->now[k]) continue;  // uniform
-      Spin<double> xv = S.x[k][i];
-      axpy_(xv, sc->ai[k], S.p[k][i]);
-      S.x[k][i] = xv;
-    }
   }
-  store_partial(acc, partials, blockIdx.x);
-}
+};
 
-// beta, beta_i; then the shifts' zeta history, iteration counts and convergence
-// (|zeta_i| |r| <= tol |b|), the iteration cap
-struct FinMSBeta {
-  MSScalars* sc;
-  __device__ bool skip() const { return sc->done != 0; }
-  __device__ void operator()(double2 t) const {
+// The iteration's two finalisers, one lane a shift (ns <= 32, in the first wave).  BETA = false:
+// alpha = rho / <p, (A + s0) p>, zeta_i and alpha_i of every active shift (Jegerlehner).
+// BETA = true: beta, beta_i, then the shifts' zeta history, iteration counts and convergence
+// (|zeta_i| |r| <= tol |b|), the iteration cap.
+template <bool BETA>
+__global__ __launch_bounds__(256) void k_ms_scalars(const double2* __restrict__ partials, unsigned n, MSScalars* sc) {
+  static_assert(kMaxShifts <= 64, "one lane of the first wave per shift");
+  if (sc->done != 0) {  // uniform
+    if (!BETA && threadIdx.x == 0) sc->update = 0;
+    return;
+  }
+  __shared__ double2 tot_;
+  const int i = threadIdx.x;
+  const bool mine = i < sc->ns;
+  double z = 0, zo = 0, zn = 0, sh = 0;
+  int act = 0;
+  if (mine) {  // in flight with the partials
+    z = sc->z[i];
+    zo = sc->zo[i];
+    zn = sc->zn[i];
+    sh = sc->shift[i];
+    act = sc->active[i];
+  }
+  double2 s = {0.0, 0.0};
+  for (unsigned k = threadIdx.x; k < n; k += blockDim.x) {
+    const double2 v = partials[k];
+    s.x += v.x;
+    s.y += v.y;
+  }
+  s = block_sum2(s);
+  if (threadIdx.x == 0) tot_ = s;
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  const double2 t = tot_;
+  if constexpr (!BETA) {
+    const double pq = t.x + sc->s0 * t.y, ap = sc->a_prev, bp = sc->b_prev;
+    const bool ok = pq > 0.0 && pq < 1e300;
+    const double alpha = sc->rho / pq;
+    if (mine && ok) {
+      sc->now[i] = act;
+      if (act) {
+        const double ds = sh - sc->s0;
+        const double zx = z * zo * ap / (alpha * bp * (zo - z) + zo * ap * (1.0 + ds * alpha));
+        sc->zn[i] = zx;
+        sc->ai[i] = alpha * zx / z;
+      }
+    }
+    if (i == 0) {
+      sc->update = 0;
+      if (ok)
+        sc->alpha = alpha;
+      else
+        sc->done = 4;
+    }
+  } else {
     const double rho_new = t.x, beta = rho_new / sc->rho;
-    sc->beta = beta;
-    sc->it += 1;
-    int any = 0;
-    for (int i = 0; i < sc->ns; i++) {
-      if (!sc->active[i]) continue;
-      const double z = sc->z[i], zn = sc->zn[i];
+    const double stop = sqrt(sc->tol2 * sc->bn2), rn = sqrt(rho_new), alpha = sc->alpha;
+    const int it = sc->it + 1, cap = sc->maxiter;
+    bool on = false;
+    if (mine && act) {
       sc->bi[i] = beta * (zn / z) * (zn / z);
       sc->zo[i] = z;
       sc->z[i] = zn;
-      sc->iters[i] = sc->it;
-      if (fabs(zn) * sqrt(rho_new) <= sqrt(sc->tol2 * sc->bn2))
-        sc->active[i] = 0;
-      else
-        any = 1;
+      sc->iters[i] = it;
+      on = !(fabs(zn) * rn <= stop);
+      if (!on) sc->active[i] = 0;
     }
-    sc->a_prev = sc->alpha;
-    sc->b_prev = beta;
-    sc->rho = rho_new;
-    if (!any)
-      sc->done = 1;
-    else if (sc->it >= sc->maxiter)
-      sc->done = 3;
+    const bool any = __ballot(on) != 0;
+    if (i == 0) {
+      sc->beta = beta;
+      sc->it = it;
+      sc->a_prev = alpha;
+      sc->b_prev = beta;
+      sc->rho = rho_new;
+      sc->update = 1;
+      if (!any)
+        sc->done = 1;
+      else if (it >= cap)
+        sc->done = 3;
+    }
   }
-};
+}
 
-// p = r + beta p; p_i = zeta_i r + beta_i p_i for the shifts active now
-__global__ __launch_bounds__(256) void k_msd_b(const Spin<double>* __restrict__ r, Spin<double>* p, ShiftPtrs S,
-                                               size_t n, const MSScalars* sc) {
-  if (sc->done != 0) return;
+// x_i += alpha_i p_i, p_i = zeta_i r + beta_i p_i for the shifts active in this iteration, and
+// p = r + beta p.  Runs once more after the iteration that ended the solve.  Rows of blocks
+// (blockIdx.y) share the shifts out, row 0 taking the base; one row where the points alone fill
+// the GPU, since every row reads r again.
+__global__ __launch_bounds__(256) void k_ms_update(const Spin<double>* __restrict__ r, Spin<double>* p, ShiftPtrs S,
+                                                   size_t n, const MSScalars* sc) {
+  if (sc->update == 0) return;
   const double beta = sc->beta;
   for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x) {
     const Spin<double> rr = r[i];
-    Spin<double> v = rr;
-    axpy_(v, beta, p[i]);
-    p[i] = v;
-    for (int k = 0; k < S.n; k++) {
-      if (!sc->now[k]) continue;  // uniform
+    if (blockIdx.y == 0) {
+      const Spin<double> pp = p[i];
+      if (sc->now[S.base]) {  // uniform
+        Spin<double> xv = sc->x[S.base][i];
+        axpy_(xv, sc->ai[S.base], pp);
+        sc->x[S.base][i] = xv;
+      }
+      Spin<double> v = rr;
+      axpy_(v, beta, pp);
+      p[i] = v;
+    }
+    for (int k = blockIdx.y; k < S.n; k += gridDim.y) {
+      if (k == S.base || !sc->now[k]) continue;  // uniform
       const double a = sc->zn[k], bb = sc->bi[k];
       const Spin<double> pk = S.p[k][i];
+      Spin<double> xv = sc->x[k][i];
+      axpy_(xv, sc->ai[k], pk);
+      sc->x[k][i] = xv;
       Spin<double> o;
       o.a = {a * rr.a.x + bb * pk.a.x, a * rr.a.y + bb * pk.a.y};
       o.b = {a * rr.b.x + bb * pk.b.x, a * rr.b.y + bb * pk.b.y};
@@ -189,6 +284,24 @@ __global__ __launch_bounds__(256) void k_msd_b(const Spin<double>* __restrict__ 
     }
   }
 }
+
+// |b - D^dag w - s x|^2 into *out, w = D x
+struct EpiShiftResid {
+  static constexpr bool kReduce = true;
+  const Spin<double>* b;
+  const Spin<double>* x;
+  double s;
+  double2* out;
+  __device__ bool skip() const { return false; }
+  __device__ void begin() {}
+  __device__ void operator()(size_t i, const Spin<double>& q, double2& acc) const {
+    Spin<double> v = ld(b + i);
+    axpy_(v, -1.0, q);
+    axpy_(v, -s, ld(x + i));
+    acc.x += nrm2(v);
+  }
+  __device__ void operator()(double2 t) const { *out = t; }
+};
 
 // out = c0 in + c1 (v + sum_k a_k y_k)   (y_k in S.x, a_k in S.a)
 __global__ __launch_bounds__(256) void k_combine(Spin<double>* out, const Spin<double>* __restrict__ in,
@@ -272,111 +385,90 @@ std::vector<CGResult> multishift_cg(Dirac& D, const std::vector<double>& shifts,
   const size_t n = D.points();
   hipStream_t st = D.stream();
   const unsigned nb = unsigned(std::min<size_t>((n + 255) / 256, 4096));
-  const double s0 = *std::min_element(shifts.begin(), shifts.end());
-  Spin<double>* r = dnew<Spin<double>>(n, st);
-  Spin<double>* p = dnew<Spin<double>>(n, st);
-  Spin<double>* w = dnew<Spin<double>>(n, st);
-  Spin<double>* q = dnew<Spin<double>>(n, st);
-  std::vector<Spin<double>*> ps(ns);
-  for (int i = 0; i < ns; i++) ps[i] = dnew<Spin<double>>(n, st);
-  double2* partials = dnew<double2>(nb, st);
-  double2* out = dnew<double2>(1, st);
-  double2* host = nullptr;
-  QED3_HIP(hipHostMalloc((void**)&host, sizeof(double2), hipHostMallocDefault));
-  Reducer red{partials, out, host, nb, st};
-  const size_t bytes = n * sizeof(Spin<double>);
-  QED3_HIP(hipMemcpyAsync(r, b, bytes, hipMemcpyDeviceToDevice, st));
-  QED3_HIP(hipMemcpyAsync(p, b, bytes, hipMemcpyDeviceToDevice, st));
-  for (int i = 0; i < ns; i++) {
-    QED3_HIP(hipMemsetAsync(x[i], 0, bytes, st));
-    QED3_HIP(hipMemcpyAsync(ps[i], b, bytes, hipMemcpyDeviceToDevice, st));
-  }
-  hipLaunchKernelGGL(k_pair_norms, dim3(nb), dim3(256), 0, st, b, b, n, partials);
-  const double bn2 = red.get().x;
-  MSScalars h{};
-  h.rho = bn2;
-  h.bn2 = bn2;
-  h.a_prev = 1.0;
-  h.b_prev = 0.0;
-  h.s0 = s0;
-  h.tol2 = o.tol * o.tol;
-  h.ns = ns;
-  h.maxiter = o.maxiter;
-  for (int i = 0; i < ns; i++) {
-    h.shift[i] = shifts[i];
-    h.z[i] = h.zo[i] = h.zn[i] = 1.0;
-    h.active[i] = bn2 > 0 ? 1 : 0;
-  }
-  h.done = (bn2 > 0 && o.maxiter > 0) ? 0 : (bn2 > 0 ? 3 : 1);
-  MSScalars* sc = dnew<MSScalars>(1, st);
-  MSScalars* hs = nullptr;
-  QED3_HIP(hipHostMalloc((void**)&hs, sizeof(MSScalars), hipHostMallocDefault));
-  *hs = h;
-  QED3_HIP(hipMemcpyAsync(sc, hs, sizeof(MSScalars), hipMemcpyHostToDevice, st));
-  ShiftPtrs S;
+  // work memory: r, p, w, the p_i of every shift but the base (the smallest), the residual
+  // norms and the scalars, each region 256-byte aligned
+  const size_t f = (n * sizeof(Spin<double>) + 255) / 256 * 256;
+  const size_t norms = (size_t(kMaxShifts) * sizeof(double2) + 255) / 256 * 256;
+  unsigned char* base = static_cast<unsigned char*>(D.scratch(14, (ns + 2) * f + norms + sizeof(MSScalars)));
+  auto field = [&](int k) { return reinterpret_cast<Spin<double>*>(base + size_t(k) * f); };
+  Spin<double>*r = field(0), *p = field(1), *w = field(2);
+  double2* out = reinterpret_cast<double2*>(base + (ns + 2) * f);
+  MSScalars* sc = reinterpret_cast<MSScalars*>(base + (ns + 2) * f + norms);
+  // read-back: the norms, then the scalars
+  unsigned char* host = static_cast<unsigned char*>(D.host_block(norms + sizeof(MSScalars)));
+  const double2* hout = reinterpret_cast<const double2*>(host);
+  MSScalars* hs = reinterpret_cast<MSScalars*>(host + norms);
+  ShiftPtrs S{};
+  ShiftVals X{};
   S.n = ns;
-  for (int i = 0; i < ns; i++) {
-    S.x[i] = x[i];
-    S.p[i] = ps[i];
+  S.base = int(std::min_element(shifts.begin(), shifts.end()) - shifts.begin());
+  for (int i = 0, k = 3; i < ns; i++) {
+    S.p[i] = i == S.base ? p : field(k++);
+    X.s[i] = shifts[i];
+    X.x[i] = x[i];
   }
+  const GridReduce gr = D.reducer();
+  hipLaunchKernelGGL(k_ms_init, dim3(nb), dim3(256), 0, st, b, r, p, S, X, n, gr.partials);
+  hipLaunchKernelGGL(k_finalize<FinMSStart>, dim3(1), dim3(256), 0, st, gr.partials, nb,
+                     FinMSStart{sc, X, ns, o.maxiter, shifts[S.base], o.tol * o.tol});
+  QED3_HIP(hipGetLastError());
   const DiracView<double> v64 = D.view<double>();
   const int nn = D.tables().max_nn;
   const HaloView hvf = D.halo_for<double>(false), hvt = D.halo_for<double>(true);
-  const GridReduce gr = D.reducer();
+  const StencilTile tf = D.tile<double>(false), tt = D.tile<double>(true);
+  // rows of the update pass: up to 2,048 blocks over the points and the shifts
+  const unsigned rows = std::max(1u, std::min(unsigned(ns), 2048u / nb));
   auto one_iter = [&] {
-    launch_stencil<double, false>(v64, nn, p, EpiStoreMS{w, sc}, D.tile<double>(false), gr, st, hvf);
-    launch_stencil<double, true>(v64, nn, w, EpiStoreMS{q, sc}, D.tile<double>(true), gr, st, hvt);
-    hipLaunchKernelGGL(k_msd_norms, dim3(nb), dim3(256), 0, st, w, p, n, partials, sc);
-    hipLaunchKernelGGL(k_finalize<FinMSAlpha>, dim3(1), dim3(256), 0, st, partials, nb, FinMSAlpha{sc});
-    hipLaunchKernelGGL(k_msd_a, dim3(nb), dim3(256), 0, st, r, q, p, S, n, partials, sc);
-    hipLaunchKernelGGL(k_finalize<FinMSBeta>, dim3(1), dim3(256), 0, st, partials, nb, FinMSBeta{sc});
-    hipLaunchKernelGGL(k_msd_b, dim3(nb), dim3(256), 0, st, r, p, S, n, sc);
+    const unsigned n1 = launch_stencil<double, false>(v64, nn, p, EpiMSD{w, p, sc}, tf, gr, st, hvf);
+    hipLaunchKernelGGL(k_ms_scalars<false>, dim3(1), dim3(256), 0, st, gr.partials, n1, sc);
+    const unsigned n2 = launch_stencil<double, true>(v64, nn, w, EpiMSDdag{r, p, sc, 0.0, 0.0}, tt, gr, st, hvt);
+    hipLaunchKernelGGL(k_ms_scalars<true>, dim3(1), dim3(256), 0, st, gr.partials, n2, sc);
+    hipLaunchKernelGGL(k_ms_update, dim3(nb, rows), dim3(256), 0, st, r, p, S, n, sc);
   };
-  // chunks of iterations replayed as one graph; the kernels of iterations after the end
-  // exit at once
-  const int chunk = 8;
-  hipGraph_t graph = nullptr;
+  // chunks of iterations replayed as one kept graph (the caller's x_i are read from the
+  // scalars); the kernels of iterations after the end exit at once
+  const int chunk = n > (1u << 20) ? 8 : 16;
   hipGraphExec_t exec = nullptr;
   if (std::getenv("QED3_NO_GRAPH") == nullptr) {
-    QED3_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    for (int c = 0; c < chunk; c++) one_iter();
-    QED3_HIP(hipStreamEndCapture(st, &graph));
-    QED3_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
+    GraphKey key;
+    key.add(v64).add(hvf).add(hvt).add(tf).add(tt).add(base).add(gr.partials).add(n).add(nn).add(ns).add(S.base);
+    GraphSlot& g = D.graph_slot(3);
+    if (!g.exec || g.key != key.words) {
+      g.clear();
+      QED3_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+      for (int c = 0; c < chunk; c++) one_iter();
+      QED3_HIP(hipStreamEndCapture(st, &g.graph));
+      QED3_HIP(hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0));
+      g.key = key.words;
+    }
+    exec = g.exec;
   }
   for (int c = 0; c <= o.maxiter / chunk + 1; c++) {
-    QED3_HIP(hipMemcpyAsync(hs, sc, sizeof(MSScalars), hipMemcpyDeviceToHost, st));
-    QED3_HIP(hipStreamSynchronize(st));
-    if (hs->done != 0) break;
     if (exec)
       QED3_HIP(hipGraphLaunch(exec, st));
     else
       for (int k = 0; k < chunk; k++) one_iter();
     QED3_HIP(hipGetLastError());
+    QED3_HIP(hipMemcpyAsync(hs, sc, sizeof(MSScalars), hipMemcpyDeviceToHost, st));
+    QED3_HIP(hipStreamSynchronize(st));
+    if (hs->done != 0) break;
   }
-  QED3_HIP(hipMemcpyAsync(hs, sc, sizeof(MSScalars), hipMemcpyDeviceToHost, st));
-  QED3_HIP(hipStreamSynchronize(st));
-  if (exec) (void)hipGraphExecDestroy(exec);
-  if (graph) (void)hipGraphDestroy(graph);
-  std::vector<int> iters(hs->iters, hs->iters + ns);
   // FP64 true residual per shift
+  for (int i = 0; i < ns; i++) {
+    launch_stencil<double, false>(v64, nn, x[i], EpiStore<double>{w}, tf, gr, st, hvf);
+    launch_stencil<double, true>(v64, nn, w, EpiShiftResid{b, x[i], shifts[i], out + i}, tt, gr, st, hvt);
+  }
+  QED3_HIP(hipGetLastError());
+  QED3_HIP(hipMemcpyAsync(host, out, ns * sizeof(double2), hipMemcpyDeviceToHost, st));
+  QED3_HIP(hipStreamSynchronize(st));
+  const double sec = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   std::vector<CGResult> res(ns);
   for (int i = 0; i < ns; i++) {
-    D.apply<double>(false, w, x[i], false);
-    D.apply<double>(true, q, w, false);
-    hipLaunchKernelGGL(k_shift_resid, dim3(nb), dim3(256), 0, st, b, q, x[i], shifts[i], n, partials);
-    const double rr = red.get().x;
-    res[i].iterations = iters[i];
-    res[i].true_resid = bn2 > 0 ? std::sqrt(rr / bn2) : 0.0;
+    res[i].iterations = hs->iters[i];
+    res[i].true_resid = hs->bn2 > 0 ? std::sqrt(hout[i].x / hs->bn2) : 0.0;
     res[i].status = res[i].true_resid <= o.tol * 1.0000001 ? 0 : 3;
+    res[i].seconds = sec;
   }
-  for (void* ptr : {(void*)r, (void*)p, (void*)w, (void*)q, (void*)partials, (void*)out, (void*)sc})
-    (void)hipFreeAsync(ptr, st);
-  for (auto* ptr : ps) (void)hipFreeAsync(ptr, st);
-  QED3_HIP(hipStreamSynchronize(st));
-  (void)hipHostFree(host);
-  (void)hipHostFree(hs);
-  const double sec = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-  for (auto& r2 : res) r2.seconds = sec;
   return res;
 }
 

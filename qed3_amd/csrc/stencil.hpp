@@ -449,10 +449,17 @@ __device__ __forceinline__ double norm2(const Spin<T>& v) {
          double(v.b.y) * v.b.y;
 }
 
+// A reducing epilogue whose finaliser the caller launches itself names kOwnFinaliser
+template <class E, class = void>
+struct EpiOwnFinaliser : std::false_type {};
+template <class E>
+struct EpiOwnFinaliser<E, std::void_t<decltype(E::kOwnFinaliser)>> : std::bool_constant<E::kOwnFinaliser> {};
+
 // `bracket` (optional, a pair of events) is recorded just before and just after the
-// stencil kernel itself (not its reduction finaliser), for per-kernel timing.
+// stencil kernel itself (not its reduction finaliser), for per-kernel timing.  Returns the
+// number of blocks, which is that of a reducing epilogue's partials.
 template <typename T, bool DAG, class Epi, class Src, typename P>
-inline void launch_stencil_src(const DiracView<T, P>& v, int max_nn, const Src& in, const Epi& epi,
+inline unsigned launch_stencil_src(const DiracView<T, P>& v, int max_nn, const Src& in, const Epi& epi,
                                StencilTile t, GridReduce gr, hipStream_t st, const HaloView& hv,
                                const hipEvent_t* bracket = nullptr) {
   TileMap tm;
@@ -480,14 +487,15 @@ inline void launch_stencil_src(const DiracView<T, P>& v, int max_nn, const Src& 
     hipLaunchKernelGGL((k_stencil<T, 3, DAG, Epi, Src, P>), grid, dim3(t.block), 0, st, v, in, epi, t.ts, tm, gr);
   }
   if (bracket) QED3_HIP(hipEventRecord(bracket[1], st));
-  if constexpr (Epi::kReduce)
+  if constexpr (Epi::kReduce && !EpiOwnFinaliser<Epi>::value)
     hipLaunchKernelGGL((k_finalize<Epi>), dim3(1), dim3(256), 0, st, gr.partials, unsigned(nblk), epi);
+  return unsigned(nblk);
 }
 
 template <typename T, bool DAG, class Epi, typename P>
-inline void launch_stencil(const DiracView<T, P>& v, int max_nn, const Spin<T>* in, const Epi& epi,
-                           StencilTile t, GridReduce gr, hipStream_t st, const HaloView& hv) {
-  launch_stencil_src<T, DAG>(v, max_nn, SrcPlain<T>{in}, epi, t, gr, st, hv);
+inline unsigned launch_stencil(const DiracView<T, P>& v, int max_nn, const Spin<T>* in, const Epi& epi,
+                               StencilTile t, GridReduce gr, hipStream_t st, const HaloView& hv) {
+  return launch_stencil_src<T, DAG>(v, max_nn, SrcPlain<T>{in}, epi, t, gr, st, hv);
 }
 
 }  // namespace qed3
