@@ -124,69 +124,99 @@ __global__ __launch_bounds__(256) void k_loss_f32(const Spin<float>* __restrict_
   store_partial(acc, gr.partials, blockIdx.x);
 }
 
-// Gradient partials of one Horner step t: per block of (site range, spin row a),
-//   q[0..1] = sum conj(v_a) mu_a                      (-> the step's c)
-//   q[2..3] = sum conj(P_a) mu_a, P_a = sum_j u_j H_aa g_a(nb_j)        (-> A_a, times -1)
-//   q[4..5] = sum conj(Q_a) mu_a, Q_a = sum_j u_j H_a,abar g_abar(nb_j)  (-> B_a, times -1)
-// with g the previous step's output (has_g) and mu = dloss / d conj(y_t).
+// Gradient sums of one Horner step t over the points a block walks, for both spin rows a:
+//   q[a][0..1] = sum conj(v_a) mu_a                      (-> the step's c)
+//   q[a][2..3] = sum conj(P_a) mu_a, P_a = sum_j u_j H_aa g_a(nb_j)        (-> A_a, times -1)
+//   q[a][4..5] = sum conj(Q_a) mu_a, Q_a = sum_j u_j H_a,abar g_abar(nb_j)  (-> B_a, times -1)
+// with g the previous step's output (has_g) and mu = dloss / d conj(y_t).  A thread takes a site
+// and a tile of kGradSlices slices, both rows from the same neighbours and phases; one thread
+// per row walking the whole column (the form before) had 160 blocks at dual n=32, Lt=32 and took
+// 44 us, this takes 14.  Partials [12][blocks], summed by k_grad_sum.
+constexpr int kGradSlices = 4, kGradSums = 12;
 template <int NS>
 __global__ __launch_bounds__(256) void k_horner_grad(HornerView hv, DiracView<float> d, const Spin<float>* __restrict__ v,
                                                      const Spin<float>* __restrict__ mu,
                                                      const Spin<float>* __restrict__ g, int has_g, TileMap tm,
                                                      double* part) {
-  int xr, a;
-  tile_of(tm, blockIdx.x, xr, a);
-  const int V = hv.V, Lt = hv.Lt;
+  int xr, st;
+  tile_of(tm, blockIdx.x, xr, st);
+  const int V = hv.V;
   const int x = xr < tm.nxr ? xr * int(blockDim.x) + int(threadIdx.x) : V;
-  double q[6] = {0, 0, 0, 0, 0, 0};
+  double q[2][6] = {};
   if (x < V) {
     int nb[NS], lk[NS];
-    float4 hr[NS];
-    const float4* rows = hv.hrow + (size_t(2 * 2 + a) * NS) * V;  // mode 2: unit coefficients
+    float4 hr[2][NS];
+    const float4* rows = hv.hrow + size_t(2 * 2) * NS * V;  // mode 2: unit coefficients
+    if (has_g) {
 #pragma unroll
-    for (int j = 0; j < NS; j++) {
-      nb[j] = d.nbr[j * V + x];
-      lk[j] = d.lnk[j * V + x];
-      hr[j] = rows[size_t(j) * V + x];
+      for (int j = 0; j < NS; j++) {
+        nb[j] = d.nbr[size_t(j) * V + x];
+        lk[j] = d.lnk[size_t(j) * V + x];
+        hr[0][j] = rows[size_t(j) * V + x];
+        hr[1][j] = rows[size_t(NS + j) * V + x];
+      }
     }
-    for (int s = 0; s < Lt; s++) {
-      const size_t i = size_t(s) * V + x;
-      const float2 m = hk::comp(mu[i], a);
-      const float2 vv = hk::comp(v[i], a);
-      q[0] += double(vv.x) * m.x + double(vv.y) * m.y;
-      q[1] += double(vv.x) * m.y - double(vv.y) * m.x;
+    const int s1 = min(hv.Lt, (st + 1) * kGradSlices);
+    for (int s = st * kGradSlices; s < s1; s++) {
+      const size_t sV = size_t(s) * V, i = sV + x;
+      const Spin<float> mp = mu[i], vp = v[i];
+      float2 u[NS];
+      Spin<float> gy[NS];
       if (has_g) {
-        float2 P = {0.f, 0.f}, Q = {0.f, 0.f};
         const float2* uS = d.uS + size_t(s) * d.E;
 #pragma unroll
         for (int j = 0; j < NS; j++) {
-          const int l = lk[j];
-          float2 u = ldu(uS + (l >= 0 ? l : ~l));
-          if (l < 0) u.y = -u.y;
-          const size_t iy = size_t(s) * V + nb[j];
-          const Spin<float> gy = g[iy];
-          const float2 ga = hk::comp(gy, a), gb = hk::comp(gy, 1 - a);
-          P = cadd<float>(P, cmul<float>(u, cmul<float>({hr[j].x, hr[j].y}, ga)));
-          Q = cadd<float>(Q, cmul<float>(u, cmul<float>({hr[j].z, hr[j].w}, gb)));
+          u[j] = ldu(uS + (lk[j] >= 0 ? lk[j] : ~lk[j]));
+          gy[j] = g[sV + nb[j]];
         }
-        q[2] += double(P.x) * m.x + double(P.y) * m.y;
-        q[3] += double(P.x) * m.y - double(P.y) * m.x;
-        q[4] += double(Q.x) * m.x + double(Q.y) * m.y;
-        q[5] += double(Q.x) * m.y - double(Q.y) * m.x;
+      }
+#pragma unroll
+      for (int a = 0; a < 2; a++) {
+        const float2 m = hk::comp(mp, a);
+        const float2 vv = hk::comp(vp, a);
+        q[a][0] += double(vv.x) * m.x + double(vv.y) * m.y;
+        q[a][1] += double(vv.x) * m.y - double(vv.y) * m.x;
+        if (has_g) {
+          float2 P = {0.f, 0.f}, Q = {0.f, 0.f};
+#pragma unroll
+          for (int j = 0; j < NS; j++) {
+            float2 uj = u[j];
+            if (lk[j] < 0) uj.y = -uj.y;
+            const float4 h = hr[a][j];
+            P = cadd<float>(P, hk::cmul_phase(uj, hk::cmul_phase({h.x, h.y}, hk::comp(gy[j], a))));
+            Q = cadd<float>(Q, hk::cmul_phase(uj, hk::cmul_phase({h.z, h.w}, hk::comp(gy[j], 1 - a))));
+          }
+          q[a][2] += double(P.x) * m.x + double(P.y) * m.y;
+          q[a][3] += double(P.x) * m.y - double(P.y) * m.x;
+          q[a][4] += double(Q.x) * m.x + double(Q.y) * m.y;
+          q[a][5] += double(Q.x) * m.y - double(Q.y) * m.x;
+        }
       }
     }
   }
-  for (int k = 0; k < 6; k++) {
-    const double2 b = block_sum2({q[k], 0.0});
-    if (threadIdx.x == 0) part[size_t(blockIdx.x) * 6 + k] = b.x;
+#pragma unroll
+  for (int k = 0; k < kGradSums; k += 2) {
+    const double2 b = block_sum2({q[k / 6][k % 6], q[(k + 1) / 6][(k + 1) % 6]});
+    if (threadIdx.x == 0) {
+      part[size_t(k) * gridDim.x + blockIdx.x] = b.x;
+      part[size_t(k + 1) * gridDim.x + blockIdx.x] = b.y;
+    }
   }
 }
 
-TileMap spin_tiles(int V) {
+// out[k] = sum of part[k][0..n), one block per k
+__global__ __launch_bounds__(256) void k_grad_sum(const double* __restrict__ part, unsigned n, double* out) {
+  double s = 0;
+  for (unsigned i = threadIdx.x; i < n; i += blockDim.x) s += part[size_t(blockIdx.x) * n + i];
+  const double2 t = block_sum2({s, 0.0});
+  if (threadIdx.x == 0) out[blockIdx.x] = t.x;
+}
+
+TileMap grad_tiles(int V, int Lt) {
   TileMap tm;
   tm.nxr = (V + 255) / 256;
   tm.nxr_pad = (tm.nxr + 7) / 8 * 8;
-  tm.nst = 2;
+  tm.nst = (Lt + kGradSlices - 1) / kGradSlices;
   tm.remap = 1;
   return tm;
 }
@@ -271,30 +301,21 @@ void run_layers(Horner& K, bool adj, const Spin<float>* in, Spin<float>* const* 
   Dirac& D = K.dirac();
   const HornerView hv = K.view();
   const DiracView<float> tab = D.view<float>();
-  const HaloView halo = D.halo(256);
+  hipStream_t st = D.stream();
   const int L = K.layers();
-  const hk::SrcF<Spin<float>> src{in};
-  const GridReduce gr = D.reducer();
   Spin<float>* prev = nullptr;
   for (int t = 0; t < L; t++) {
     const cd c = K.params().c[L - 1 - t];
     const float2 cj = {float(c.real()), float(adj ? -c.imag() : c.imag())};
     Spin<float>* o = keep ? keep[t] : (t == L - 1 ? out : bufs[t & 1]);
-    if (t == 0) {
-      if (adj)
-        hk::launch_horner_layer<true, true, false>(hv, tab, halo, src, (const Spin<float>*)nullptr, o, cj,
-                                                   hk::EpiNone{}, gr, D.stream());
-      else
-        hk::launch_horner_layer<false, true, false>(hv, tab, halo, src, (const Spin<float>*)nullptr, o, cj,
-                                                    hk::EpiNone{}, gr, D.stream());
-    } else {
-      if (adj)
-        hk::launch_horner_layer<true, false, false>(hv, tab, halo, src, (const Spin<float>*)prev, o, cj,
-                                                    hk::EpiNone{}, gr, D.stream());
-      else
-        hk::launch_horner_layer<false, false, false>(hv, tab, halo, src, (const Spin<float>*)prev, o, cj,
-                                                     hk::EpiNone{}, gr, D.stream());
-    }
+    if (t == 0 && adj)
+      hk::launch_horner_layer<true, true>(hv, tab, in, nullptr, o, cj, st);
+    else if (t == 0)
+      hk::launch_horner_layer<false, true>(hv, tab, in, nullptr, o, cj, st);
+    else if (adj)
+      hk::launch_horner_layer<true, false>(hv, tab, in, prev, o, cj, st);
+    else
+      hk::launch_horner_layer<false, false>(hv, tab, in, prev, o, cj, st);
     prev = o;
   }
   QED3_HIP(hipGetLastError());
@@ -332,64 +353,57 @@ double Horner::loss_grad(const Spin<double>* v, const Spin<double>* e, int batch
   Spin<float>* mu[2] = {static_cast<Spin<float>*>(work(3, fb)), static_cast<Spin<float>*>(work(4, fb))};
   std::vector<Spin<float>*> G(L);
   for (int t = 0; t < L; t++) G[t] = static_cast<Spin<float>*>(work(6 + t, fb));
-  double* dscal = static_cast<double*>(work(5, 2 * sizeof(double)));
-  const TileMap tm = spin_tiles(V);
-  const unsigned nblk = unsigned(tm.nxr_pad) * 2u;
-  if (red_n_ < size_t(nblk) * 6) {
+  // per pair: |e|^2, its loss, then every step's gradient sums; read back once at the end
+  const size_t per = 2 + size_t(L) * kGradSums;
+  double* dscal = static_cast<double*>(work(5, batch * per * sizeof(double)));
+  const TileMap tm = grad_tiles(V, D_.Lt());
+  const unsigned nblk = unsigned(tm.nxr_pad) * unsigned(tm.nst);
+  if (red_n_ < size_t(nblk) * kGradSums) {
     if (red_) QED3_HIP(hipFree(red_));
-    QED3_HIP(hipMalloc((void**)&red_, size_t(nblk) * 6 * sizeof(double)));
-    red_n_ = size_t(nblk) * 6;
+    red_ = nullptr;
+    red_n_ = 0;
+    QED3_HIP(hipMalloc((void**)&red_, size_t(nblk) * kGradSums * sizeof(double)));
+    red_n_ = size_t(nblk) * kGradSums;
   }
   const GridReduce gr = D_.reducer();
   const HornerView hv = view();
   const DiracView<float> tab = D_.view<float>();
-  const HaloView halo = D_.halo(256);
   std::vector<cd> g(p_.count(), cd(0, 0));
-  std::vector<double> part(size_t(nblk) * 6);
-  double loss = 0;
   const unsigned nbk = stream_grid(n);
   for (int b = 0; b < batch; b++) {
+    double* ds = dscal + b * per;
     hipLaunchKernelGGL(k_to_f32, dim3(nbk), dim3(256), 0, st, v + size_t(b) * n, pv, n);
     hipLaunchKernelGGL(k_to_f32, dim3(nbk), dim3(256), 0, st, e + size_t(b) * n, pe, n);
     run_layers(*this, false, pv, nullptr, nullptr, G.data());
     hipLaunchKernelGGL(k_norm_f32, dim3(nbk), dim3(256), 0, st, pe, n, gr);
-    hipLaunchKernelGGL(k_finalize<FinStore>, dim3(1), dim3(256), 0, st, gr.partials, nbk, FinStore{dscal});
-    hipLaunchKernelGGL(k_loss_f32, dim3(nbk), dim3(256), 0, st, G[L - 1], pe, lam, dscal, 1.0 / batch, n, gr);
-    hipLaunchKernelGGL(k_finalize<FinStore>, dim3(1), dim3(256), 0, st, gr.partials, nbk, FinStore{dscal + 1});
-    QED3_HIP(hipGetLastError());
-    double hl[2];
-    QED3_HIP(hipMemcpyAsync(hl, dscal, sizeof(hl), hipMemcpyDeviceToHost, st));
+    hipLaunchKernelGGL(k_finalize<FinStore>, dim3(1), dim3(256), 0, st, gr.partials, nbk, FinStore{ds});
+    hipLaunchKernelGGL(k_loss_f32, dim3(nbk), dim3(256), 0, st, G[L - 1], pe, lam, ds, 1.0 / batch, n, gr);
+    hipLaunchKernelGGL(k_finalize<FinStore>, dim3(1), dim3(256), 0, st, gr.partials, nbk, FinStore{ds + 1});
     // backward: mu_{L-1} = T^-dag lambda; mu_{t-1} = T^-dag (S_th^dag mu_t)
-    const hk::SrcF<Spin<float>> srcl{lam};
     for (int t = L - 1; t >= 0; t--) {
       Spin<float>* mo = mu[t & 1];
       if (t == L - 1)
-        hk::launch_horner_layer<true, true, false>(hv, tab, halo, srcl, (const Spin<float>*)nullptr, mo,
-                                                   float2{1.f, 0.f}, hk::EpiNone{}, gr, st);
+        hk::launch_horner_layer<true, true>(hv, tab, lam, nullptr, mo, float2{1.f, 0.f}, st);
       else
-        hk::launch_horner_layer<true, false, false>(hv, tab, halo, srcl, (const Spin<float>*)mu[(t + 1) & 1], mo,
-                                                    float2{0.f, 0.f}, hk::EpiNone{}, gr, st);
+        hk::launch_horner_layer<true, false>(hv, tab, lam, mu[(t + 1) & 1], mo, float2{0.f, 0.f}, st);
       const Spin<float>* gp = t > 0 ? G[t - 1] : nullptr;
       if (NS == 6)
         hipLaunchKernelGGL(k_horner_grad<6>, dim3(nblk), dim3(256), 0, st, hv, tab, pv, mo, gp, int(t > 0), tm, red_);
       else
         hipLaunchKernelGGL(k_horner_grad<3>, dim3(nblk), dim3(256), 0, st, hv, tab, pv, mo, gp, int(t > 0), tm, red_);
-      QED3_HIP(hipGetLastError());
-      QED3_HIP(hipMemcpyAsync(part.data(), red_, part.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-      QED3_HIP(hipStreamSynchronize(st));
-      double q0[6] = {0, 0, 0, 0, 0, 0}, q1[6] = {0, 0, 0, 0, 0, 0};
-      for (unsigned k = 0; k < nblk; k++) {
-        // block k's spin row, decoded as tile_of does
-        int a;
-        if (tm.remap) {
-          const int per = tm.nxr_pad >> 3, j = int(k) >> 3;
-          a = j / per;
-        } else {
-          a = int(k) / tm.nxr_pad;
-        }
-        double* q = a == 0 ? q0 : q1;
-        for (int m = 0; m < 6; m++) q[m] += part[size_t(k) * 6 + m];
-      }
+      hipLaunchKernelGGL(k_grad_sum, dim3(kGradSums), dim3(256), 0, st, red_, nblk, ds + 2 + size_t(t) * kGradSums);
+    }
+    QED3_HIP(hipGetLastError());
+  }
+  std::vector<double> host(batch * per);
+  QED3_HIP(hipMemcpyAsync(host.data(), dscal, host.size() * sizeof(double), hipMemcpyDeviceToHost, st));
+  QED3_HIP(hipStreamSynchronize(st));
+  double loss = 0;
+  for (int b = 0; b < batch; b++) {
+    loss += host[b * per + 1];
+    for (int t = L - 1; t >= 0; t--) {
+      const double* q0 = host.data() + b * per + 2 + size_t(t) * kGradSums;
+      const double* q1 = q0 + 6;
       // step t used c[L-1-t]; gradients are 2 d loss / d conj(param)
       g[L - 1 - t] += 2.0 * cd(q0[0] + q1[0], q0[1] + q1[1]);
       if (t > 0) {
@@ -399,7 +413,6 @@ double Horner::loss_grad(const Spin<double>* v, const Spin<double>* e, int batch
         g[L + 3] += -2.0 * cd(q1[4], q1[5]);
       }
     }
-    loss += hl[1];
   }
   if (grad) *grad = g;
   return loss;

@@ -1,20 +1,11 @@
 // Device side of the time-exact Horner preconditioner (horner.hpp): one layer
 // g_out = T^{-1}(c v + S_th g_in) (or its adjoint form) per launch.
 //
-// Thread = site x; a block owns a range of R Hilbert-consecutive sites.  Under T the spin-up
-// row's recurrence runs forward in time and the spin-down row's backward (the other way
-// round under T^dagger).  A layer makes two passes over each site's time column:
-//   pass 1, s = 0 .. Lt-1: per slice the block stages g_in of its range and spatial halo in
-//     LDS (two alternating tiles, one barrier per slice), every thread forms the spatial
-//     transports of both rows from the same staged values and link phases, finishes the
-//     forward row's recurrence state = (y + kappa_t u^t state) / c_x and stores, at its
-//     output point, that row's result beside the other row's y (its recurrence input);
-//   pass 2, s = Lt-1 .. 0: every thread reads its own column back, runs the backward row's
-//     recurrence and stores both rows' results (no neighbours, no barriers).
-// So every neighbour, link phase and input load serves both rows.  Fields are FP32
-// spin-interleaved points (the checked apply and the training gradient, in any gauge); the
-// solver's binary16 layers are the parallel-in-time form further down.
-// The first layer of a network (FIRST) has no input field: no staging, no barrier.
+// Under T the spin-up row's recurrence runs forward in time and the spin-down row's backward
+// (the other way round under T^dagger).  Two forms:
+//   FP32 fields in any gauge (the checked apply and the training gradient): a transport pass
+//     y = c v + S_th g over all points, then the two rows' recurrences;
+//   binary16 fields in the temporal gauge (the solver): the parallel-in-time layer below.
 #pragma once
 #include <type_traits>
 
@@ -151,212 +142,187 @@ struct EpiNone {
   __device__ void operator()(double2) const {}
 };
 
-// LDS tile entry of the two-pass layer: an FP32 point
-__device__ __forceinline__ float4 to_tile(const Spin<float>& v) { return {v.a.x, v.a.y, v.b.x, v.b.y}; }
-
-template <int NS, typename F, typename P>
-struct SliceLoads {
-  F v;
-  P u[NS];
-  P ut;
-  F gc, gh0, gh1;
-};
-
-template <int NS, bool ADJ, bool FIRST, bool TG, typename F, class Src, class Epi, typename P>
-__global__ __launch_bounds__(256) void k_horner_layer(HornerView hv, DiracView<float, P> d, HaloView halo, Src src,
-                                                      const F* __restrict__ gin, F* __restrict__ gout, float2 cj,
-                                                      TileMap tm, Epi epi, GridReduce gr) {
-  static_assert(std::is_same<F, Spin<float>>::value, "the two-pass layer runs on FP32 fields");
-  using Tile = float4;
-  if (epi.skip()) return;  // uniform
-  extern __shared__ float4 hk_tile_raw[];
-  Tile* hk_tile = reinterpret_cast<Tile*>(hk_tile_raw);
+// ---- layers on FP32 fields -------------------------------------------------------------
+// The transport pass: y(s, x) = c_j v - sum_j u_j (m_same g_a + m_flip g_abar)(nb_j) for both spin
+// rows, a thread per site and tile of ts slices (the hop rows stay in registers).  It carries the
+// layer's gathers and has no order in time, so every point can be in flight: walking a site's
+// column with one thread, transports and recurrences together (the form before), left the GPU at
+// 80 blocks on dual n=32, Lt=32 and took 48 us a layer; this pass and the recurrences' take 9 + 9.
+// The roundings are spelled out (and contraction off), so that the FP32 results do not depend on
+// the code around them.
+constexpr int kTransportSlices = 4;
+__device__ __forceinline__ float2 cmul_coef(float2 h, float2 g) {  // h g
+#pragma clang fp contract(off)
+  return {__builtin_fmaf(g.x, h.x, -(g.y * h.y)), __builtin_fmaf(g.y, h.x, g.x * h.y)};
+}
+__device__ __forceinline__ float2 cmul_phase(float2 u, float2 c) {  // u c
+#pragma clang fp contract(off)
+  return {__builtin_fmaf(u.x, c.x, -(u.y * c.y)), __builtin_fmaf(u.x, c.y, u.y * c.x)};
+}
+template <int NS, bool ADJ>
+__global__ __launch_bounds__(256) void k_horner_transport(HornerView hv, DiracView<float> d,
+                                                          const Spin<float>* __restrict__ v,
+                                                          const Spin<float>* __restrict__ gin, Spin<float>* __restrict__ y,
+                                                          float2 cj, TileMap tm) {
+#pragma clang fp contract(off)
   int xr, st;
   tile_of(tm, blockIdx.x, xr, st);
-  (void)st;
-  const int V = hv.V, Lt = hv.Lt, R = blockDim.x;
-  const bool live = xr < tm.nxr;
-  const int x0 = xr * R;
-  const int x = live ? x0 + int(threadIdx.x) : V;
-  const bool act = x < V;
-  constexpr int rF = ADJ ? 1 : 0, rB = 1 - rF;  // rows whose recurrence runs forward / backward
-  const int h0 = (live && !FIRST) ? halo.halo_off[xr] : 0;
-  const int nh = (live && !FIRST) ? halo.halo_off[xr + 1] - h0 : 0;
-  const int hid0 = (int(threadIdx.x) < nh) ? halo.halo[h0 + threadIdx.x] : -1;
-  const int hid1 = (int(threadIdx.x) + R < nh) ? halo.halo[h0 + threadIdx.x + R] : -1;
+  const int V = hv.V;
+  const int x = xr < tm.nxr ? xr * int(blockDim.x) + int(threadIdx.x) : V;
+  if (x >= V) return;
+  constexpr int rF = ADJ ? 1 : 0, rB = 1 - rF;
   int nb[NS], lk[NS];
   float4 hrF[NS], hrB[NS];
-  float invc = 0.f, kt = 0.f;
-  if (act) {
-    if constexpr (!FIRST) {
-      const size_t mF = size_t((ADJ ? 2 : 0) + rF) * NS * V, mB = size_t((ADJ ? 2 : 0) + rB) * NS * V;
+  const size_t mF = size_t((ADJ ? 2 : 0) + rF) * NS * V, mB = size_t((ADJ ? 2 : 0) + rB) * NS * V;
 #pragma unroll
-      for (int j = 0; j < NS; j++) {
-        nb[j] = halo.nbl[j * V + x];
-        lk[j] = d.lnk[j * V + x];
-        hrF[j] = hv.hrow[mF + size_t(j) * V + x];
-        hrB[j] = hv.hrow[mB + size_t(j) * V + x];
-      }
-    }
-    invc = hv.invc[x];
-    kt = hv.kt[x];
+  for (int j = 0; j < NS; j++) {
+    nb[j] = d.nbr[size_t(j) * V + x];
+    lk[j] = d.lnk[size_t(j) * V + x];
+    hrF[j] = hv.hrow[mF + size_t(j) * V + x];
+    hrB[j] = hv.hrow[mB + size_t(j) * V + x];
   }
-  const auto in = src.bind();
-  // Loads of slice s: the injection, (original gauge) the temporal link s-1 -> s that the
-  // forward recurrence crosses, the link phases and the input field at the site and at its
-  // share of the halo.
-  auto load = [&](int s, SliceLoads<NS, F, P>& L) {
+  const int s1 = min(hv.Lt, (st + 1) * kTransportSlices);
+  for (int s = st * kTransportSlices; s < s1; s++) {
     const size_t sV = size_t(s) * V;
-    if (act) {
-      L.v = in.raw(sV + x);
-      if constexpr (!TG) {
-        if (s > 0) L.ut = d.uT[size_t(s - 1) * V + x];
-      }
-      if constexpr (!FIRST) {
-        const P* uS = d.uS + size_t(s) * d.E;
-#pragma unroll
-        for (int j = 0; j < NS; j++) L.u[j] = uS[lk[j] >= 0 ? lk[j] : ~lk[j]];
-        L.gc = gin[sV + x];
-      }
-    }
-    if constexpr (!FIRST) {
-      if (hid0 >= 0) L.gh0 = gin[sV + hid0];
-      if (hid1 >= 0) L.gh1 = gin[sV + hid1];
-    }
-  };
-  // sum_j u_j (m_same g_a + m_flip g_abar)(nb_j) for row a from the staged tile
-  auto transport = [&](const SliceLoads<NS, F, P>& L, const Tile* tb, const float4* hr, int a) -> float2 {
-    float2 t = {0.f, 0.f};
+    const float2* uS = d.uS + size_t(s) * d.E;
+    float2 u[NS];
+    Spin<float> g[NS];
 #pragma unroll
     for (int j = 0; j < NS; j++) {
-      float2 u = ldu(&L.u[j]);
-      if (lk[j] < 0) u.y = -u.y;
-      const float4 g = tb[nb[j]];
-      const float2 ga = a == 0 ? float2{g.x, g.y} : float2{g.z, g.w};
-      const float2 gb = a == 0 ? float2{g.z, g.w} : float2{g.x, g.y};
-      const float2 cm = cadd<float>(cmul<float>({hr[j].x, hr[j].y}, ga), cmul<float>({hr[j].z, hr[j].w}, gb));
-      t = cadd<float>(t, cmul<float>(u, cm));
+      u[j] = uS[lk[j] >= 0 ? lk[j] : ~lk[j]];
+      g[j] = gin[sV + nb[j]];
     }
-    return t;
-  };
-  float2 stF = {0.f, 0.f}, stB = {0.f, 0.f};
-  // S holds the time wrap (the link from Lt-1 to 0, which T leaves out): each recurrence
-  // starts from bc kappa_t w g(the far end of its walk), w the wrap link's phase,
-  // conjugated for the forward walk.
-  if constexpr (!FIRST) {
-    if (act) {
-      const cplx_t<float> w = TG ? ldu(d.uPoly + x) : ldu(d.uT + size_t(Lt - 1) * V + x);
-      const float2 gF = comp(gin[size_t(Lt - 1) * V + x], rF), gB = comp(gin[x], rB);
-      const float2 tF = cmul<float>({w.x, -w.y}, gF), tB = cmul<float>(w, gB);
-      stF = {d.bc * kt * tF.x, d.bc * kt * tF.y};
-      stB = {d.bc * kt * tB.x, d.bc * kt * tB.y};
-    }
+    auto transport = [&](const float4* hr, int a) -> float2 {
+      float2 t = {0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < NS; j++) {
+        float2 uj = u[j];
+        if (lk[j] < 0) uj.y = -uj.y;
+        const float2 cm = cadd<float>(cmul_coef({hr[j].x, hr[j].y}, comp(g[j], a)),
+                                      cmul_coef({hr[j].z, hr[j].w}, comp(g[j], 1 - a)));
+        t = cadd<float>(t, cmul_phase(uj, cm));
+      }
+      return t;
+    };
+    const Spin<float> vv = v[sV + x];
+    float2 yF = cmul_phase(cj, comp(vv, rF)), yB = cmul_phase(cj, comp(vv, rB));
+    const float2 tF = transport(hrF, rF), tB = transport(hrB, rB);
+    yF.x -= tF.x;
+    yF.y -= tF.y;
+    yB.x -= tB.x;
+    yB.y -= tB.y;
+    if constexpr (rF == 0)
+      put(y + sV + x, yF, yB);
+    else
+      put(y + sV + x, yB, yF);
   }
-  // ---- pass 1: forward in time --------------------------------------------------------
-  SliceLoads<NS, F, P> cur, nxt;
-  load(0, cur);
-  for (int s = 0; s < Lt; s++) {
-    if (s + 1 < Lt) load(s + 1, nxt);  // a slice ahead: in flight during this slice's work
-    Tile* tb = hk_tile + (s & 1) * (R + halo.hmax);
-    if constexpr (!FIRST) {
-      if (act) tb[threadIdx.x] = to_tile(cur.gc);
-      if (hid0 >= 0) tb[R + threadIdx.x] = to_tile(cur.gh0);
-      if (hid1 >= 0) tb[2 * R + threadIdx.x] = to_tile(cur.gh1);
-      for (int q = int(threadIdx.x) + 2 * R; q < nh; q += R)
-        tb[R + q] = to_tile(gin[size_t(s) * V + halo.halo[h0 + q]]);
-      __syncthreads();
+}
+
+// The recurrences, one thread per site and spin row: state = (y + kappa_t u^t state) / c_x walked
+// from the row's start to its end, each value written over its y.  The chain is arithmetic only:
+// the loads of the next kRecurDepth slices are issued while this group's are worked through.
+// FIRST (no input field): y = c_j v formed here, without a transport pass or a wrap term.
+constexpr int kRecurDepth = 8;
+template <bool FWD, bool FIRST>
+__device__ __forceinline__ void horner_recur_walk(const HornerView& hv, const DiracView<float>& d, const Spin<float>* in,
+                                                  const Spin<float>* __restrict__ gin, Spin<float>* out, float2 cj,
+                                                  int x, int row) {
+#pragma clang fp contract(off)  // the roundings are spelled out: FP32 results do not depend on the code around them
+  const int V = hv.V, Lt = hv.Lt;
+  const float invc = hv.invc[x], kt = hv.kt[x];
+  auto at = [&](int k) { return size_t(FWD ? k : Lt - 1 - k) * V + x; };
+  // component `row` of the point, as two floats
+  auto half = [&](const Spin<float>* p, size_t i) { return reinterpret_cast<const float2*>(p)[2 * i + row]; };
+  // a link's phase times v, conjugated for the forward walk
+  auto hop = [](float2 u, float2 v) {
+    if constexpr (FWD)
+      return float2{__builtin_fmaf(u.y, v.y, u.x * v.x), __builtin_fmaf(u.x, v.y, -(u.y * v.x))};
+    else
+      return float2{__builtin_fmaf(u.x, v.x, -(u.y * v.y)), __builtin_fmaf(v.x, u.y, v.y * u.x)};
+  };
+  float2 st = {0.f, 0.f};
+  if constexpr (!FIRST) {
+    // S holds the time wrap (the link from Lt-1 to 0, which T leaves out): each recurrence
+    // starts from bc kappa_t w g(the far end of its walk), w the wrap link's phase
+    const float2 w = d.uT[size_t(Lt - 1) * V + x], g = half(gin, at(Lt - 1));
+    float2 t = hop(w, g);
+    if constexpr (FWD) t.x = __builtin_fmaf(w.x, g.x, w.y * g.y);
+    st = {d.bc * kt * t.x, d.bc * kt * t.y};
+  }
+  struct Group {
+    float2 y[kRecurDepth], u[kRecurDepth];
+  };
+  auto load = [&](int k0, Group& G) {
+#pragma unroll
+    for (int j = 0; j < kRecurDepth; j++) {
+      const int k = min(k0 + j, Lt - 1);
+      G.y[j] = half(in, at(k));
+      G.u[j] = d.uT[at(FWD ? max(k - 1, 0) : k)];  // the link the walk crosses to reach slice at(k)
     }
-    if (act) {
-      float2 yF = cmul<float>(cj, comp(cur.v, rF)), yB = cmul<float>(cj, comp(cur.v, rB));
-      if constexpr (!FIRST) {
-        const float2 tF = transport(cur, tb, hrF, rF), tB = transport(cur, tb, hrB, rB);
-        yF.x -= tF.x;
-        yF.y -= tF.y;
-        yB.x -= tB.x;
-        yB.y -= tB.y;
-      }
-      if (s > 0) {
-        float2 t = stF;
-        if constexpr (!TG) {
-          const float2 ut = ldu(&cur.ut);
-          t = cmul<float>({ut.x, -ut.y}, stF);  // the link s-1 -> s, conjugated
+  };
+  Group cur, nxt;
+  load(0, cur);
+  for (int k0 = 0; k0 < Lt; k0 += kRecurDepth) {
+    if (k0 + kRecurDepth < Lt) load(k0 + kRecurDepth, nxt);
+#pragma unroll
+    for (int j = 0; j < kRecurDepth; j++) {
+      const int k = k0 + j;
+      if (k < Lt) {
+        float2 y = cur.y[j];
+        if constexpr (FIRST)
+          y = {__builtin_fmaf(cj.x, y.x, -(cj.y * y.y)), __builtin_fmaf(cj.y, y.x, cj.x * y.y)};
+        if (k > 0) {
+          const float2 t = hop(cur.u[j], st);
+          if constexpr (FWD && FIRST) {
+            y = {__builtin_fmaf(kt, t.x, y.x), __builtin_fmaf(kt, t.y, y.y)};
+          } else {
+            const float2 w = {kt * t.x, kt * t.y};
+            y = {y.x + w.x, y.y + w.y};
+          }
+        } else {
+          y.x += st.x;  // the wrap term, already weighted (0 in a first layer)
+          y.y += st.y;
         }
-        yF.x += kt * t.x;
-        yF.y += kt * t.y;
-      } else {
-        yF.x += stF.x;  // the wrap term, already weighted (0 in a first layer)
-        yF.y += stF.y;
+        st = {invc * y.x, invc * y.y};
+        reinterpret_cast<float2*>(out)[2 * at(k) + row] = st;
       }
-      stF = {invc * yF.x, invc * yF.y};
-      const size_t i = size_t(s) * V + x;
-      if constexpr (rF == 0)
-        put(gout + i, stF, yB);
-      else
-        put(gout + i, yB, stF);
     }
     cur = nxt;
   }
-  // ---- pass 2: backward in time over the thread's own column ------------------------
-  double2 acc = {0.0, 0.0};
-  if (act) {
-    F tcur = gout[size_t(Lt - 1) * V + x], tnxt = tcur;
-    P ucur{};
-    for (int s = Lt - 1; s >= 0; s--) {
-      const size_t i = size_t(s) * V + x;
-      if (s > 0) tnxt = gout[i - V];
-      if constexpr (!TG) {
-        if (s < Lt - 1) ucur = d.uT[i];  // the link s -> s+1 the backward recurrence crosses
-      }
-      const float2 gF = comp(tcur, rF);
-      float2 yB = comp(tcur, rB);
-      if (s < Lt - 1) {
-        float2 t = stB;
-        if constexpr (!TG) t = cmul<float>(ldu(&ucur), stB);
-        yB.x += kt * t.x;
-        yB.y += kt * t.y;
-      } else {
-        yB.x += stB.x;  // the wrap term
-        yB.y += stB.y;
-      }
-      stB = {invc * yB.x, invc * yB.y};
-      if constexpr (rF == 0) {
-        put(gout + i, gF, stB);
-        epi(i, stored(gout, gF, stB), acc);
-      } else {
-        put(gout + i, stB, gF);
-        epi(i, stored(gout, stB, gF), acc);
-      }
-      tcur = tnxt;
-    }
-  }
-  if constexpr (Epi::kReduce) store_partial(acc, gr.partials, blockIdx.x);
 }
 
-// Launch one layer over the lattice.  `tables` supplies the spatial link phases (and, without
-// TG, the temporal ones) of the gauge the fields live in.
-template <bool ADJ, bool FIRST, bool TG, typename F, class Src, class Epi, typename P>
-inline void launch_horner_layer(const HornerView& hv, const DiracView<float, P>& tables, const HaloView& halo,
-                                const Src& src, const F* gin, F* gout, float2 cj, const Epi& epi, GridReduce gr,
-                                hipStream_t st, const hipEvent_t* bracket = nullptr) {
-  constexpr int R = 256;
-  TileMap tm;
-  tm.nxr = (hv.V + R - 1) / R;
-  tm.nxr_pad = (tm.nxr + 7) / 8 * 8;
-  tm.nst = 1;
-  tm.remap = 1;
-  const unsigned nblk = unsigned(tm.nxr_pad);
-  if (Epi::kReduce && nblk > kReduceCapacity) throw std::invalid_argument("layer grid exceeds the reduction scratch");
-  const size_t smem = FIRST ? 0 : size_t(2) * (R + halo.hmax) * sizeof(float4);
-  if (bracket) QED3_HIP(hipEventRecord(bracket[0], st));
-  if (hv.nslot == 6)
-    hipLaunchKernelGGL((k_horner_layer<6, ADJ, FIRST, TG, F, Src, Epi, P>), dim3(nblk), dim3(R), smem, st, hv,
-                       tables, halo, src, gin, gout, cj, tm, epi, gr);
+template <bool ADJ, bool FIRST>
+__global__ __launch_bounds__(256) void k_horner_recur(HornerView hv, DiracView<float> d, const Spin<float>* in,
+                                                      const Spin<float>* __restrict__ gin, Spin<float>* out,
+                                                      float2 cj) {
+  const int nxb = (hv.V + 255) / 256;
+  const int row = int(blockIdx.x) / nxb;
+  const int x = (int(blockIdx.x) - row * nxb) * 256 + int(threadIdx.x);
+  if (x >= hv.V) return;
+  if (row == (ADJ ? 1 : 0))  // uniform: the row that runs forward in time
+    horner_recur_walk<true, FIRST>(hv, d, in, gin, out, cj, x, row);
   else
-    hipLaunchKernelGGL((k_horner_layer<3, ADJ, FIRST, TG, F, Src, Epi, P>), dim3(nblk), dim3(R), smem, st, hv,
-                       tables, halo, src, gin, gout, cj, tm, epi, gr);
-  if (bracket) QED3_HIP(hipEventRecord(bracket[1], st));
-  if constexpr (Epi::kReduce)
-    hipLaunchKernelGGL((k_finalize<Epi>), dim3(1), dim3(256), 0, st, gr.partials, nblk, epi);
+    horner_recur_walk<false, FIRST>(hv, d, in, gin, out, cj, x, row);
+}
+
+// One layer of K (ADJ: of K^dagger) on FP32 fields: gout = T^{-1}(c_j v + S_th gin)
+template <bool ADJ, bool FIRST>
+inline void launch_horner_layer(const HornerView& hv, const DiracView<float>& tables, const Spin<float>* v,
+                                const Spin<float>* gin, Spin<float>* gout, float2 cj, hipStream_t st) {
+  if constexpr (!FIRST) {
+    TileMap tm;
+    tm.nxr = (hv.V + 255) / 256;
+    tm.nxr_pad = (tm.nxr + 7) / 8 * 8;
+    tm.nst = (hv.Lt + kTransportSlices - 1) / kTransportSlices;
+    tm.remap = 1;
+    const dim3 grid(unsigned(tm.nxr_pad) * unsigned(tm.nst));
+    if (hv.nslot == 6)
+      hipLaunchKernelGGL((k_horner_transport<6, ADJ>), grid, dim3(256), 0, st, hv, tables, v, gin, gout, cj, tm);
+    else
+      hipLaunchKernelGGL((k_horner_transport<3, ADJ>), grid, dim3(256), 0, st, hv, tables, v, gin, gout, cj, tm);
+  }
+  hipLaunchKernelGGL((k_horner_recur<ADJ, FIRST>), dim3(2 * unsigned((hv.V + 255) / 256)), dim3(256), 0, st, hv, tables,
+                     FIRST ? v : gout, gin, gout, cj);
 }
 
 // ---- parallel-in-time layer (the solver's path: binary16 fields, temporal gauge) ------
