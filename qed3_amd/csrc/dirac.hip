@@ -14,16 +14,6 @@ namespace qed3 {
 namespace {
 constexpr size_t kReduceCap = kReduceCapacity;
 
-template <typename T>
-__global__ void k_phases(const double* __restrict__ ang, cplx_t<T>* __restrict__ u, size_t n) {
-  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) {
-    double sn, cs;
-    sincos(ang[i], &sn, &cs);
-    u[i] = {T(cs), T(sn)};
-  }
-}
-
 // 16-bit fixed-point angle in units of 2 pi / 65536, wrapped into [-pi, pi)
 __device__ __forceinline__ phase16_t angle16(double a) {
   const long long k = llrint(a * (65536.0 / (2.0 * M_PI)));
@@ -33,6 +23,32 @@ __device__ __forceinline__ phase16_t angle16(double a) {
 __global__ void k_phases_half(const double* __restrict__ ang, phase16_t* __restrict__ u, size_t n) {
   const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) u[i] = angle16(ang[i]);
+}
+
+// A gauge update: every angle (spatial [nS], then temporal) from the caller's arrays (srcS, srcT)
+// into the context's own, as complex phases in FP64 and FP32 and, where those tables are held
+// (hS), as 16-bit angles.  One pass and one FP64 sine and cosine per link: as two copies and four
+// to six kernels, each reading the angles again and the FP32 ones taking the FP64 sine anew, it
+// took 64 us at simplicial n=64, Lt=32 (5.2 M links), this takes 37.
+struct PhaseTables {
+  double *angS, *angT;
+  double2 *uS, *uT;
+  float2 *fS, *fT;
+  phase16_t *hS, *hT;
+};
+__global__ __launch_bounds__(256) void k_phases(const double* __restrict__ srcS, const double* __restrict__ srcT,
+                                                PhaseTables t, size_t nS, size_t n) {
+  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const bool sp = i < nS;
+  const size_t k = sp ? i : i - nS;
+  const double a = sp ? srcS[k] : srcT[k];
+  (sp ? t.angS : t.angT)[k] = a;
+  double sn, cs;
+  sincos(a, &sn, &cs);
+  (sp ? t.uS : t.uT)[k] = {cs, sn};
+  (sp ? t.fS : t.fT)[k] = {float(cs), float(sn)};
+  if (t.hS) (sp ? t.hS : t.hT)[k] = angle16(a);
 }
 
 // Temporal gauge, per site: phi_0 = 0, phi_{s+1} = phi_s + theta^t_s (FP64 and 16-bit), and
@@ -180,37 +196,156 @@ __device__ __forceinline__ double link_bilinear(const DiracView<double>& d, cons
   return sg * (tP.y - tM.y);
 }
 
-// Pseudofermion force, one thread per spatial link (s,l) followed by one per temporal
-// link (s,x):  F = -2 Re <w, dD/dtheta eta> with w = D eta  (dirac_pf.h:107-121).
-__global__ __launch_bounds__(256) void k_force(DiracView<double> d, const int4* __restrict__ ends,
-                                               const Spin<double>* __restrict__ eta,
-                                               const Spin<double>* __restrict__ w,
-                                               double* __restrict__ fs, double* __restrict__ ft) {
+// f_l (+)= c sum_k Re <u_k, dD/dtheta_l v_k> for every link, one thread per spatial link (s,l)
+// followed by one per temporal link (s,x); the second pair is skipped when F.u[1] is null, f is
+// overwritten when init.  The form for lattices whose fields stay in the caches (launch_force).
+__global__ __launch_bounds__(256) void k_force_links(DiracView<double> d, const int4* __restrict__ ends, ForcePairs F,
+                                                     double c, int init, double* __restrict__ fs,
+                                                     double* __restrict__ ft) {
   const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   const size_t nS = size_t(d.Lt) * d.E, nT = size_t(d.Lt) * d.V;
   if (i >= nS + nT) return;
-  const double f = -2.0 * link_bilinear(d, ends, i, w, eta);
-  if (i < nS)
-    fs[i] = f;
-  else
-    ft[i - nS] = f;
-}
-
-// f_i (+)= c (Re <u1, dD/dtheta_i v1> + Re <u2, dD/dtheta_i v2>) for every link; the second
-// pair is skipped when u2 is null, f is overwritten when init.
-__global__ __launch_bounds__(256) void k_force_acc(DiracView<double> d, const int4* __restrict__ ends,
-                                                   const Spin<double>* __restrict__ u1,
-                                                   const Spin<double>* __restrict__ v1,
-                                                   const Spin<double>* __restrict__ u2,
-                                                   const Spin<double>* __restrict__ v2, double c, int init,
-                                                   double* __restrict__ fs, double* __restrict__ ft) {
-  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const size_t nS = size_t(d.Lt) * d.E, nT = size_t(d.Lt) * d.V;
-  if (i >= nS + nT) return;
-  double t = link_bilinear(d, ends, i, u1, v1);
-  if (u2) t += link_bilinear(d, ends, i, u2, v2);
+  double t = link_bilinear(d, ends, i, F.u[0], F.v[0]);
+  if (F.u[1]) t += link_bilinear(d, ends, i, F.u[1], F.v[1]);
   double* f = i < nS ? fs + i : ft + (i - nS);
   *f = init ? c * t : *f + c * t;
+}
+
+// The same with NP pairs by sites, for lattices whose fields come from HBM.  A thread owns a site for a tile of ts slices and computes the links that start there: the
+// spatial ones stored in its orientation and the temporal one to the next slice.  With e^{i theta}
+// = u on the link x -> y,
+//   Re <w, dD/dtheta eta> = -Im <w_x, u H_xy eta_y> + Im <w_y, u^* H_yx eta_x>
+// and the second product is <u H_yx^dagger w_y, eta_x>, so both hops' coefficients are the site's
+// own (hop and hopd share C and S); the next slice's spinors serve the temporal link before they
+// become the site's.  A thread per link gathers four spinors, two hop rows and the link's ends;
+// here the block's sites and halo are staged in LDS, one slice at a time as the LDS stencil does,
+// so each spinor is requested once per block and the hop rows once per tile.  What is left are
+// the links' scattered phases and stores (8 and 16 B a lane per slot).
+template <int NS, int NP>
+__global__ __launch_bounds__(256) void k_force_sites(DiracView<double> d, ForcePairs F, double c, int init, int ts,
+                                                     TileMap tm, HaloView hv, double* __restrict__ fs,
+                                                     double* __restrict__ ft) {
+  using C = double2;
+  extern __shared__ unsigned char smem_raw[];
+  Spin<double>* tile = reinterpret_cast<Spin<double>*>(smem_raw);  // [2 NP][row]: u_k, then v_k
+  int xr, st;
+  tile_of(tm, blockIdx.x, xr, st);
+  const int V = d.V, Lt = d.Lt, R = blockDim.x, row = R + hv.hmax;
+  if (xr >= tm.nxr) return;  // uniform
+  const int x = xr * R + int(threadIdx.x);
+  const bool act = x < V;
+  const double r = d.r;
+  const int h0 = hv.halo_off[xr], nh = hv.halo_off[xr + 1] - h0;
+  int nb[NS], lk[NS];  // lk < 0: not this site's link
+  double hC[NS], hS[NS], hA[NS], hB[NS], gA[NS], gB[NS];
+#pragma unroll
+  for (int j = 0; j < NS; j++) {
+    lk[j] = -1;
+    if (act) {
+      nb[j] = hv.nbl[size_t(j) * V + x];
+      lk[j] = d.lnk[size_t(j) * V + x];
+      if (nb[j] == int(threadIdx.x)) lk[j] = -1;  // padding slot
+    }
+    if (lk[j] >= 0) {
+      const double4 h = d.hop[size_t(j) * V + x], g = d.hopd[size_t(j) * V + x];
+      hC[j] = r * h.x;
+      hS[j] = r * h.y;
+      hA[j] = h.z;
+      hB[j] = h.w;
+      gA[j] = g.z;
+      gB[j] = g.w;
+    }
+  }
+  // H = [[-r(C - iS), a - ib], [a + ib, -r(C + iS)]] times (p0, p1)
+  auto hmul = [](double rC, double rS, double A, double B, const C p0, const C p1, C& o0, C& o1) {
+    o0 = {-rC * p0.x - rS * p0.y + A * p1.x + B * p1.y, -rC * p0.y + rS * p0.x + A * p1.y - B * p1.x};
+    o1 = {A * p0.x - B * p0.y - rC * p1.x + rS * p1.y, A * p0.y + B * p0.x - rC * p1.y - rS * p1.x};
+  };
+  const double kh = act ? d.kth[x] : 0.0;
+  const double m0 = kh * (-r - 1.0), m1 = kh * (-r + 1.0);  // T- = diag(m0,m1), T+ = diag(m1,m0)
+  const int s0 = st * ts, s1 = min(Lt, s0 + ts);
+  Spin<double> w0[NP], e0[NP];
+  if (act) {
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
+      w0[k] = F.u[k][size_t(s0) * V + x];
+      e0[k] = F.v[k][size_t(s0) * V + x];
+    }
+  }
+  for (int s = s0; s < s1; s++) {
+    const size_t sV = size_t(s) * V;
+    // this slice's loads that do not go through LDS, in flight with the halo's
+    Spin<double> w1[NP], e1[NP];
+    C u[NS], ut{};
+    if (act) {
+      const size_t o1 = size_t(s == Lt - 1 ? 0 : s + 1) * V + x;
+#pragma unroll
+      for (int k = 0; k < NP; k++) {
+        w1[k] = F.u[k][o1];
+        e1[k] = F.v[k][o1];
+      }
+      ut = d.uT[sV + x];
+#pragma unroll
+      for (int j = 0; j < NS; j++)
+        if (lk[j] >= 0) u[j] = d.uS[size_t(s) * d.E + lk[j]];
+#pragma unroll
+      for (int k = 0; k < NP; k++) {
+        tile[k * row + threadIdx.x] = w0[k];
+        tile[(NP + k) * row + threadIdx.x] = e0[k];
+      }
+    }
+    for (int i = threadIdx.x; i < nh; i += R) {
+      const size_t o = sV + hv.halo[h0 + i];
+#pragma unroll
+      for (int k = 0; k < NP; k++) {
+        tile[k * row + R + i] = F.u[k][o];
+        tile[(NP + k) * row + R + i] = F.v[k][o];
+      }
+    }
+    __syncthreads();
+    if (act) {
+#pragma unroll
+      for (int j = 0; j < NS; j++) {
+        if (lk[j] < 0) continue;
+        double f = 0.0;
+#pragma unroll
+        for (int k = 0; k < NP; k++) {
+          const Spin<double> wy = tile[k * row + nb[j]], ey = tile[(NP + k) * row + nb[j]];
+          C a0, a1, b0, b1;
+          hmul(hC[j], hS[j], hA[j], hB[j], cmul<double>(u[j], ey.a), cmul<double>(u[j], ey.b), a0, a1);
+          hmul(hC[j], hS[j], gA[j], gB[j], cmul<double>(u[j], wy.a), cmul<double>(u[j], wy.b), b0, b1);
+          // Re <w, i v> = -Im <w, v>
+          const C t1 = cadd<double>(cconjmul<double>(w0[k].a, a0), cconjmul<double>(w0[k].b, a1));
+          const C t2 = cadd<double>(cconjmul<double>(b0, e0[k].a), cconjmul<double>(b1, e0[k].b));
+          f += t2.y - t1.y;
+        }
+        double* o = fs + (size_t(s) * d.E + lk[j]);
+        *o = init ? c * f : *o + c * f;
+      }
+      const double sg = (s == Lt - 1) ? double(d.bc) : 1.0;
+      const C uc = {ut.x, -ut.y};
+      double f = 0.0;
+      // dD[s+1 <- s] = -i sg T- e^{-i theta};  dD[s <- s+1] = +i sg T+ e^{+i theta}
+#pragma unroll
+      for (int k = 0; k < NP; k++) {
+        const C p0 = cmul<double>(uc, e0[k].a), p1 = cmul<double>(uc, e0[k].b);
+        const C q0 = cmul<double>(ut, e1[k].a), q1 = cmul<double>(ut, e1[k].b);
+        const C tP = cadd<double>(cconjmul<double>(w1[k].a, cscale<double>(m0, p0)),
+                                  cconjmul<double>(w1[k].b, cscale<double>(m1, p1)));
+        const C tM = cadd<double>(cconjmul<double>(w0[k].a, cscale<double>(m1, q0)),
+                                  cconjmul<double>(w0[k].b, cscale<double>(m0, q1)));
+        // Re<w, -i sg tP> = sg Im(tP);  Re<w, i sg tM> = -sg Im(tM)
+        f += sg * (tP.y - tM.y);
+      }
+      ft[sV + x] = init ? c * f : ft[sV + x] + c * f;
+#pragma unroll
+      for (int k = 0; k < NP; k++) {
+        w0[k] = w1[k];
+        e0[k] = e1[k];
+      }
+    }
+    __syncthreads();  // the tile has been read
+  }
 }
 
 template <typename T>
@@ -442,16 +577,15 @@ HaloView Dirac::halo(int R) {
 
 void Dirac::set_gauge(const double* spatial, const double* temporal, bool on_device) {
   const size_t nS = size_t(h_.Lt) * h_.E, nT = size_t(h_.Lt) * h_.V;
-  const hipMemcpyKind k = on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-  QED3_HIP(hipMemcpyAsync(angS_, spatial, nS * sizeof(double), k, stream_));
-  QED3_HIP(hipMemcpyAsync(angT_, temporal, nT * sizeof(double), k, stream_));
+  if (!on_device) {
+    QED3_HIP(hipMemcpyAsync(angS_, spatial, nS * sizeof(double), hipMemcpyHostToDevice, stream_));
+    QED3_HIP(hipMemcpyAsync(angT_, temporal, nT * sizeof(double), hipMemcpyHostToDevice, stream_));
+  }
+  const PhaseTables t{angS_, angT_, d64_.uS, d64_.uT, d32_.uS, d32_.uT, uSh_, uTh_};
   const int B = 256;
-  hipLaunchKernelGGL(k_phases<double>, dim3((nS + B - 1) / B), dim3(B), 0, stream_, angS_, d64_.uS, nS);
-  hipLaunchKernelGGL(k_phases<double>, dim3((nT + B - 1) / B), dim3(B), 0, stream_, angT_, d64_.uT, nT);
-  hipLaunchKernelGGL(k_phases<float>, dim3((nS + B - 1) / B), dim3(B), 0, stream_, angS_, d32_.uS, nS);
-  hipLaunchKernelGGL(k_phases<float>, dim3((nT + B - 1) / B), dim3(B), 0, stream_, angT_, d32_.uT, nT);
+  hipLaunchKernelGGL(k_phases, dim3(unsigned((nS + nT + B - 1) / B)), dim3(B), 0, stream_, on_device ? spatial : angS_,
+                     on_device ? temporal : angT_, t, nS, nS + nT);
   QED3_HIP(hipGetLastError());
-  if (uSh_) fill_half_phases();
   if (uStg_) fill_temporal_gauge();
   QED3_HIP(hipStreamSynchronize(stream_));
   has_gauge_ = true;
@@ -633,25 +767,64 @@ void Dirac::dot(const Spin<double>* x, const Spin<double>* y, double* re, double
   if (im) *im = h.y;
 }
 
+// Links or sites: with the spinors in the last-level cache (two FP64 fields of 2^21 points are 128
+// MB) the gathers of the form by links cost no more than the staging; beyond, each gathered
+// spinor is HBM traffic again.  By links / by sites: simplicial n=24, Lt=16 (0.09 M points) 8.8 /
+// 10.9 us, n=64, Lt=32 (1.3 M) 60 / 61; dual n=64, Lt=32 (2.6 M) 94 / 89; simplicial n=100, Lt=40
+// (4 M) 328 / 195.
+// By sites: slices per thread, the more the less often a site's hop rows are read (0.3 KB on six
+// slots), but at least four waves a SIMD; sites per block, the D stencil's range, whose halo
+// tables are there, or the largest whose tiles (two spinors a pair) fit in LDS.
+void Dirac::launch_force(const ForcePairs& F, int npairs, double c, bool init, double* fs, double* ft) {
+  if (points() < size_t(1) << 21) {
+    const size_t n = size_t(h_.Lt) * (h_.E + h_.V);
+    hipLaunchKernelGGL(k_force_links, dim3(unsigned((n + 255) / 256)), dim3(256), 0, stream_, view<double>(),
+                       reinterpret_cast<const int4*>(link_ends_), F, c, init ? 1 : 0, fs, ft);
+    QED3_HIP(hipGetLastError());
+    return;
+  }
+  int ts = std::min(16, h_.Lt);
+  while (ts > 1 && size_t(h_.V) * ((h_.Lt + ts - 1) / ts) < 4 * 64 * 1024) ts = (ts + 1) / 2;
+  const auto smem_of = [&](int R) { return size_t(2 * npairs) * (R + halo(R).hmax) * sizeof(Spin<double>); };
+  int R = tile<double>(false).lds ? tile<double>(false).block : 256;
+  while (R > 64 && smem_of(R) > 64 * 1024) R /= 2;  // at 64 it fits whatever the numbering
+  const HaloView hv = halo(R);
+  TileMap tm;
+  tm.nxr = (h_.V + R - 1) / R;
+  tm.nxr_pad = (tm.nxr + 7) / 8 * 8;
+  tm.nst = (h_.Lt + ts - 1) / ts;
+  tm.remap = 1;
+  const dim3 grid(unsigned(tm.nxr_pad) * unsigned(tm.nst));
+  const DiracView<double> v = view<double>();
+  auto go = [&](auto ns, auto np) {
+    hipLaunchKernelGGL((k_force_sites<decltype(ns)::value, decltype(np)::value>), grid, dim3(R), smem_of(R), stream_, v, F, c,
+                       init ? 1 : 0, ts, tm, hv, fs, ft);
+  };
+  auto go_ns = [&](auto ns) {
+    if (npairs == 2)
+      go(ns, std::integral_constant<int, 2>{});
+    else
+      go(ns, std::integral_constant<int, 1>{});
+  };
+  if (h_.max_nn == 6)
+    go_ns(std::integral_constant<int, 6>{});
+  else
+    go_ns(std::integral_constant<int, 3>{});
+  QED3_HIP(hipGetLastError());
+}
+
+// Pseudofermion force F = -2 Re <w, dD/dtheta eta>, w = D eta (dirac_pf.h:107-121)
 void Dirac::force(const Spin<double>* eta, double* fs, double* ft) {
   if (!tmp64_) tmp64_ = dalloc<Spin<double>>(points());
   apply<double>(false, tmp64_, eta, false);  // precalc: w = D eta
-  const size_t n = size_t(h_.Lt) * (h_.E + h_.V);
-  const int B = 256;
-  hipLaunchKernelGGL(k_force, dim3((n + B - 1) / B), dim3(B), 0, stream_, view<double>(),
-                     reinterpret_cast<const int4*>(link_ends_), eta, tmp64_, fs, ft);
-  QED3_HIP(hipGetLastError());
+  launch_force(ForcePairs{{tmp64_, nullptr}, {eta, nullptr}}, 1, -2.0, true, fs, ft);
   QED3_HIP(hipStreamSynchronize(stream_));
 }
 
 void Dirac::force_bilinear(const Spin<double>* u1, const Spin<double>* v1, const Spin<double>* u2,
                            const Spin<double>* v2, double c, bool init, double* fs, double* ft) {
   if ((u2 == nullptr) != (v2 == nullptr)) throw std::invalid_argument("force_bilinear: second pair incomplete");
-  const size_t n = size_t(h_.Lt) * (h_.E + h_.V);
-  const int B = 256;
-  hipLaunchKernelGGL(k_force_acc, dim3((n + B - 1) / B), dim3(B), 0, stream_, view<double>(),
-                     reinterpret_cast<const int4*>(link_ends_), u1, v1, u2, v2, c, init ? 1 : 0, fs, ft);
-  QED3_HIP(hipGetLastError());
+  launch_force(ForcePairs{{u1, u2}, {v1, v2}}, u2 ? 2 : 1, c, init, fs, ft);
 }
 
 double Dirac::time_apply(bool dag, int prec, int warmup, int reps) {

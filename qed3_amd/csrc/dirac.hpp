@@ -149,6 +149,12 @@ class GraphKey {
   }
 };
 
+// Pairs (u_k, v_k) whose derivative terms a force sums
+struct ForcePairs {
+  const Spin<double>* u[2];
+  const Spin<double>* v[2];
+};
+
 class Dirac {
  public:
   Dirac(const Geometry& g, int lattice, int Lt, int bc, double r, double M5, double at);
@@ -251,6 +257,8 @@ class Dirac {
   void upload_tables(DeviceTables<T>& d);
   template <typename T>
   void tune_one(bool dag);
+  // f (+)= c times the sum over npairs (1 or 2) pairs, for every link
+  void launch_force(const ForcePairs& F, int npairs, double c, bool init, double* fs, double* ft);
 
   HopTables h_;
   int bc_ = 0;
