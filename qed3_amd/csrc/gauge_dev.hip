@@ -44,11 +44,17 @@ __global__ __launch_bounds__(256) void k_plaq_grads(const double* __restrict__ u
   }
 }
 
-__global__ __launch_bounds__(256) void k_force_links(const double* __restrict__ gf, const double* __restrict__ gtp,
-                                                     const int* __restrict__ lf_face, const int* __restrict__ lf_sign,
-                                                     const int* __restrict__ st_off, const int* __restrict__ st_link,
-                                                     const int* __restrict__ st_sign, int Lt, int V, int E, int F,
-                                                     double* fs, double* ft) {
+// The gauge force F of every link from the plaquette gradients, its kick of the momenta and the
+// drift of the angles that follows: p += kick F, then angle += drift p (drift = 0: angles left).
+// A link's force reads no angle, so both updates ride on the force, which is never stored: a
+// leapfrog step is this kernel and k_plaq_grads, where the force's two arrays and four vector
+// updates made six launches of 2-5 us each on a small lattice.
+__global__ __launch_bounds__(256) void k_kick_drift(const double* __restrict__ gf, const double* __restrict__ gtp,
+                                                    const int* __restrict__ lf_face, const int* __restrict__ lf_sign,
+                                                    const int* __restrict__ st_off, const int* __restrict__ st_link,
+                                                    const int* __restrict__ st_sign, int Lt, int V, int E, int F,
+                                                    double kick, double drift, double* ps, double* pt, double* u,
+                                                    double* t) {
   const size_t ns = size_t(Lt) * E, nt = size_t(Lt) * V;
   for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < ns + nt; i += size_t(gridDim.x) * blockDim.x) {
     if (i < ns) {
@@ -60,13 +66,17 @@ __global__ __launch_bounds__(256) void k_force_links(const double* __restrict__ 
         if (f >= 0) v += lf_sign[2 * l + k] * gf[size_t(s) * F + f];
       }
       v += gtp[size_t(s) * E + l] - gtp[size_t(sm) * E + l];
-      fs[i] = v;
+      const double p = ps[i] + kick * v;
+      ps[i] = p;
+      if (drift != 0.0) u[i] += drift * p;
     } else {
       const size_t j = i - ns;
       const int s = int(j / V), x = int(j % V);
       double v = 0;
       for (int k = st_off[x]; k < st_off[x + 1]; k++) v += st_sign[k] * gtp[size_t(s) * E + st_link[k]];
-      ft[j] = v;
+      const double p = pt[j] + kick * v;
+      pt[j] = p;
+      if (drift != 0.0) t[j] += drift * p;
     }
   }
 }
@@ -173,12 +183,12 @@ DeviceGauge::~DeviceGauge() {
   if (hpart_) (void)hipHostFree(hpart_);
 }
 
-void DeviceGauge::force(const double* u, const double* t, double* fs, double* ft, hipStream_t st) {
+void DeviceGauge::kick_drift(double* u, double* t, double* ps, double* pt, double kick, double drift, hipStream_t st) {
   const size_t n1 = size_t(Lt_) * (F_ + E_), n2 = size_t(Lt_) * (E_ + V_);
   hipLaunchKernelGGL(k_plaq_grads, dim3(blocks_for(n1)), dim3(256), 0, st, u, t, fe_off_, fe_link_, fe_sign_,
                      ends_, beta_s_, beta_t_, compact_, Lt_, V_, E_, F_, gf_, gt_);
-  hipLaunchKernelGGL(k_force_links, dim3(blocks_for(n2)), dim3(256), 0, st, gf_, gt_, lf_face_, lf_sign_,
-                     st_off_, st_link_, st_sign_, Lt_, V_, E_, F_, fs, ft);
+  hipLaunchKernelGGL(k_kick_drift, dim3(blocks_for(n2)), dim3(256), 0, st, gf_, gt_, lf_face_, lf_sign_, st_off_,
+                     st_link_, st_sign_, Lt_, V_, E_, F_, kick, drift, ps, pt, u, t);
   QED3_HIP(hipGetLastError());
 }
 

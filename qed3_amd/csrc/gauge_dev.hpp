@@ -21,8 +21,10 @@ class DeviceGauge {
   ~DeviceGauge();
   DeviceGauge(const DeviceGauge&) = delete;
   DeviceGauge& operator=(const DeviceGauge&) = delete;
-  // fs[Lt][E], ft[Lt][V] = dS/d(angle) (device arrays)
-  void force(const double* u, const double* t, double* fs, double* ft, hipStream_t st);
+  // One leapfrog step of the gauge part, F = dS/d(angle) at (u, t): the momenta ps[Lt][E],
+  // pt[Lt][V] += kick F, then the angles u, t += drift times the new momenta (device arrays;
+  // drift = 0 leaves the angles)
+  void kick_drift(double* u, double* t, double* ps, double* pt, double kick, double drift, hipStream_t st);
   double action(const double* u, const double* t, hipStream_t st);  // FP64
   // sum of squares of n doubles (kinetic energy pieces), FP64
   double norm2(const double* a, size_t n, hipStream_t st);

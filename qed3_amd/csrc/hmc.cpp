@@ -141,8 +141,8 @@ HMC::HMC(Dirac& D, const HMCParams& p)
   dg_ = std::make_unique<DeviceGauge>(h, Sg_.beta_s(), Sg_.beta_t(), Sg_.face_edge_offsets(),
                                       Sg_.face_edge_links(), Sg_.face_edge_signs(), Sg_.compact());
   const size_t nS = size_t(h.Lt) * h.E, nT = size_t(h.Lt) * h.V;
-  for (double** p : {&du_, &dpu_, &dgs_}) QED3_HIP(hipMalloc(p, nS * sizeof(double)));
-  for (double** p : {&dt_, &dpt_, &dgt_}) QED3_HIP(hipMalloc(p, nT * sizeof(double)));
+  for (double** p : {&du_, &dpu_}) QED3_HIP(hipMalloc(p, nS * sizeof(double)));
+  for (double** p : {&dt_, &dpt_}) QED3_HIP(hipMalloc(p, nT * sizeof(double)));
 }
 
 HMC::~HMC() {
@@ -151,7 +151,7 @@ HMC::~HMC() {
   (void)hipFree(xi_);
   (void)hipFree(dfs_);
   (void)hipFree(dft_);
-  for (double* p : {du_, dt_, dpu_, dpt_, dgs_, dgt_}) (void)hipFree(p);
+  for (double* p : {du_, dt_, dpu_, dpt_}) (void)hipFree(p);
 }
 
 void HMC::update_eta(int k) {
@@ -268,7 +268,6 @@ HMCReport HMC::trajectory(double* u, double* t, bool no_reject) {
     daxpy(dpu_, fs, c, nS, st);
     daxpy(dpt_, ft, c, nT, st);
   };
-  auto gauge_force = [&] { dg_->force(du_, dt_, dgs_, dgt_, st); };
   ta = now();
   for (int k = 0; k < p_.npf; k++) {
     fermion_force(k);
@@ -277,13 +276,10 @@ HMCReport HMC::trajectory(double* u, double* t, bool no_reject) {
   t_fermion += since(ta);
   for (int n = 0; n < p_.nsteps; n++) {
     ta = now();
-    gauge_force();
-    kick(dgs_, dgt_, -0.5 * tau_in);
+    dg_->kick_drift(du_, dt_, dpu_, dpt_, -0.5 * tau_in, tau_in, st);
     for (int ni = 0; ni < p_.nsteps_inner; ni++) {
-      daxpy(du_, dpu_, tau_in, nS, st);
-      daxpy(dt_, dpt_, tau_in, nT, st);
-      gauge_force();
-      kick(dgs_, dgt_, (ni != p_.nsteps_inner - 1) ? -1.0 * tau_in : -0.5 * tau_in);
+      const bool last = ni == p_.nsteps_inner - 1;
+      dg_->kick_drift(du_, dt_, dpu_, dpt_, last ? -0.5 * tau_in : -1.0 * tau_in, last ? 0.0 : tau_in, st);
     }
     D_.set_gauge(du_, dt_, true);
     gauge_changed();

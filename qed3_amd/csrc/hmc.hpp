@@ -108,10 +108,9 @@ class HMC {
   double* dfs_ = nullptr;
   double* dft_ = nullptr;
   std::vector<double> pu_, pt_;  // host momenta (drawn from the host streams)
-  // device state of the integrator: angles, momenta, gauge force
+  // device state of the integrator: angles, momenta
   std::unique_ptr<DeviceGauge> dg_;
   double *du_ = nullptr, *dt_ = nullptr, *dpu_ = nullptr, *dpt_ = nullptr;
-  double *dgs_ = nullptr, *dgt_ = nullptr;
   HMCReport rep_;
   Overlap* ov_ = nullptr;
   bool ov_refresh_ = false;
