@@ -15,6 +15,9 @@ using namespace cgepi;
 
 constexpr int kBlock = 256;
 constexpr long kLargeBlocks = 256;  // one block per CU of a 256-CU part
+// Time of an iteration in us: of the batched launches over some systems, and of the same
+// systems' own launches (measured: see batch_cg)
+constexpr double kBatchBase = 80.0, kBatchPerMpoint = 100.0, kOwnPerSystem = 5.3;
 
 // One system of the batch: its operator views, LDS halo tables for ranges of kBlock
 // sites, its blocks in the stencil grids and the streaming grids, and its fields.
@@ -218,14 +221,14 @@ std::vector<CGResult> batch_launches(const std::vector<Dirac*>& Ds, const std::v
                                      const std::vector<const Spin<double>*>& bs, const CGOptions& o);
 }  // namespace
 
-// Systems whose own K1 grid covers the GPU (at least kLargeBlocks blocks of 256 at their
-// time tile) run the single-system kernels, which run at lower register pressure than the
-// batched kernels and in the temporal gauge, in rounds of one chunk per system on the
-// systems' own streams (cg_solve_half_many: no GPU idle time on host polls, and systems
-// that do not fill the GPU overlap); the others, too small for a launch of their own to
-// occupy the GPU, share the batched launches.  On the 64 systems of n in {32..128},
-// Lt in {16..64} the rounds were 12% faster than solving one system after another, the
-// batched launches 2% slower.
+// Every system runs the single-system kernels, a chunk of iterations at a time on its own stream
+// (cg_solve_half_many: they run at lower register pressure than the batched kernels, in the
+// temporal gauge, and overlap), except many small ones: the host and the hardware queues take
+// about kOwnPerSystem us an iteration for every system, the batched launches a base and a price
+// per point.  Batched / own launches: 64 of simplicial n=8, Lt=8: 13.2 / 25.7 ms; 32 of dual
+// n=10, Lt=12 and simplicial n=9, Lt=7: 12.4 / 20.1; 64 of simplicial n=16, Lt=16 (2.6 M points):
+// 38.2 / 36.7; 4 of n <= 30: 9.1 / 5.6; 8 of simplicial n=32, Lt=16: 16.4 / 8.6.  A system whose
+// own K1 grid covers the GPU (kLargeBlocks blocks of 256) is never batched.
 std::vector<CGResult> batch_cg(const std::vector<Dirac*>& Ds, const std::vector<Spin<double>*>& xs,
                                const std::vector<const Spin<double>*>& bs, const CGOptions& o) {
   const int ns = int(Ds.size());
@@ -240,6 +243,12 @@ std::vector<CGResult> batch_cg(const std::vector<Dirac*>& Ds, const std::vector<
     const int ts = std::max(1, std::min(D.tile<float>(false).ts, D.Lt()));
     const long blocks = long((D.V() + kBlock - 1) / kBlock) * ((D.Lt() + ts - 1) / ts);
     (blocks >= kLargeBlocks ? big : small).push_back(k);
+  }
+  double mpoints = 0;
+  for (int k : small) mpoints += 1e-6 * double(Ds[k]->points());
+  if (kOwnPerSystem * double(small.size()) <= kBatchBase + kBatchPerMpoint * mpoints) {
+    big.insert(big.end(), small.begin(), small.end());
+    small.clear();
   }
   std::vector<CGResult> out(ns);
   CGOptions os = o;
