@@ -431,8 +431,18 @@ Dirac::Dirac(const Geometry& g, int lattice, int Lt, int bc, double r, double M5
   dot_out_ = dalloc<double2>(1);
   QED3_HIP(hipMemsetAsync(counter_, 0, sizeof(unsigned int), stream_));
   QED3_HIP(hipStreamSynchronize(stream_));
+  // Launch shape until one is tuned or set.  With few points a thread's slices are a serial chain
+  // on a GPU that stands mostly empty.  FP64 CG / learned solve in us at block 256, 4 slices |
+  // 128, 2 | 64, 1: simplicial n=16, Lt=16 (0.04 M points) 3043 / 1148 | 1966 / 1020 | 1822 / 996;
+  // dual n=16, Lt=16 (0.08 M) 3708 / 1227 | 2725 / 1157 | 2616 / 1151; dual n=20, Lt=20 (0.16 M)
+  // 4213 / 1332 | 3602 / 1287 | 3926 / 1322; dual n=24, Lt=32 (0.37 M) 6239 / 1533 | 6162 / 1518 |
+  // 7329 / 1678; simplicial n=40, Lt=30 (0.48 M) 6339 / 1561 | 7253 / 1614 | 8493 / 1812.
+  const size_t pts = points();
+  const StencilTile t = pts < 90000    ? StencilTile{64, 1}
+                        : pts < 320000 ? StencilTile{128, std::min(2, h_.Lt)}
+                                       : StencilTile{256, std::min(4, h_.Lt)};
   for (auto& a : tile_)
-    for (auto& b : a) b = StencilTile{256, std::min(4, h_.Lt)};
+    for (auto& b : a) b = t;
 }
 
 template <typename T>
