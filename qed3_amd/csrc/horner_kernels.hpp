@@ -15,10 +15,14 @@
 namespace qed3 {
 namespace hk {
 
-// binary16 complex arithmetic on (re, im) pairs (packed FMAs)
+// binary16 complex arithmetic on (re, im) pairs: x y and acc + x y, in packed FMAs
 __device__ __forceinline__ half2_t cmul16(half2_t x, half2_t y) {
   const half2_t ys = {-y.y, y.x};
-  return x.xx * y + x.yy * ys;
+  return __builtin_elementwise_fma(x.yy, ys, x.xx * y);
+}
+__device__ __forceinline__ half2_t cfma16(half2_t x, half2_t y, half2_t acc) {
+  const half2_t ys = {-y.y, y.x};
+  return __builtin_elementwise_fma(x.yy, ys, __builtin_elementwise_fma(x.xx, y, acc));
 }
 
 // element idx of base through a 32-bit byte offset (idx * sizeof(T) < 2^32), so that the
@@ -47,10 +51,10 @@ __device__ __forceinline__ SpinH bload_h(const void* base, unsigned nbytes, unsi
 __device__ __forceinline__ unsigned bload_w(const void* base, unsigned nbytes, unsigned voff, unsigned soff) {
   return __builtin_bit_cast(unsigned, __builtin_amdgcn_raw_buffer_load_b32(buf_rsrc(base, nbytes), voff, soff, 0));
 }
-// e^{i theta} of the 10-bit angle in bits 10k..10k+9 of a packed word (theta = 2 pi a / 1024)
-// as a binary16 pair; the hardware sine and cosine take revolutions
-__device__ __forceinline__ half2_t angle_pair10(unsigned w, int k) {
-  const float rev = float((w >> (10 * k)) & 1023u) * (1.0f / 1024.0f);
+// e^{i theta} of a 10-bit angle (theta = 2 pi a / 1024) as a binary16 pair; the hardware sine
+// and cosine take revolutions
+__device__ __forceinline__ half2_t angle_pair10(unsigned a) {
+  const float rev = float(a) * (1.0f / 1024.0f);
   return half2_t{(_Float16)__builtin_amdgcn_cosf(rev), (_Float16)__builtin_amdgcn_sinf(rev)};
 }
 
@@ -342,10 +346,15 @@ inline void launch_horner_layer(const HornerView& hv, const DiracView<float>& ta
 // step the block stages the C slices its lanes are at, for its S sites and their halo (halo
 // tables of ranges of S sites).  The spatial link phases come per site as the view's uSite10:
 // the slots' angles (orientation applied) at 10 bits, three to a 32-bit word, so a thread
-// reads one word per slice on the trivalent lattice (a wave's loads consecutive), turned into
-// binary16 (cos, sin) pairs with the hardware sine and cosine.  The rounding (at most
-// pi/1024 rad) is of the order of the binary16 arithmetic's and only enters the
-// preconditioner.
+// reads one word per slice on the trivalent lattice (a wave's loads consecutive).  The rounding
+// (at most pi/1024 rad) is of the order of the binary16 arithmetic's and only enters the
+// preconditioner.  With six slots the kernel is bound by VALU issue, so each block looks the
+// 1,024 binary16 (cos, sin) pairs up in a 4 KB LDS table it fills once (a sine and a cosine,
+// quarter rate, and their conversions per slot and slice before), and the transports are chains
+// of packed FMAs into the rows' accumulators, 12 a slot instead of 16 packed operations: 25-29%
+// fewer vector instructions, learned solves of simplicial n=64, Lt=32: 2604 -> 2496 us, n=48,
+// Lt=45: 2530 -> 2392, n=128, Lt=64: 13300 -> 12780; with three slots 1-3% less up to n=64, and no
+// change at n=128, Lt=64, where the layer moves 5.4 TB/s.
 constexpr int kTcDepth = 2;    // steps whose loads are in flight ahead of the one computed
 // most threads per block (S sites x C lanes) with T slices per lane: the short chunks leave the
 // registers for twice the lanes
@@ -387,6 +396,7 @@ __global__ __launch_bounds__(tc_block(T), (NS == 3 ? 4 : 2)) void k_horner_layer
   const int row = S + halo.hmax;
   float2* carry = reinterpret_cast<float2*>(tile + (FIRST ? 0 : 2 * C * row));  // [2][blockDim]
   HopRow16* hqs = reinterpret_cast<HopRow16*>(carry + 2 * blockDim.x);  // [S][2 rows][NS], the sites' hop rows
+  half2_t* phase_tab = reinterpret_cast<half2_t*>(hqs + (FIRST ? 0 : S * 2 * NS));  // [1024] e^{i theta}
   int xr, st_;
   tile_of(tm, blockIdx.x, xr, st_);
   (void)st_;
@@ -486,16 +496,22 @@ __global__ __launch_bounds__(tc_block(T), (NS == 3 ? 4 : 2)) void k_horner_layer
       if constexpr (H2) Ld.gh1 = bload_h(gin, fbytes, vG + vh1, sG);
     }
   };
-  auto transport = [&](const Loads& Ld, const SpinH* tb, const HopRow16* hq, int r) -> float2 {
-    half2_t t16 = {(_Float16)0.f, (_Float16)0.f};
+  // both rows' transports sum_q u_q (s_q g_r + f_q g_(1-r)) of the staged neighbours
+  auto transport = [&](const Loads& Ld, const SpinH* tb, float2& tF, float2& tB) {
+    half2_t aF = {(_Float16)0.f, (_Float16)0.f}, aB = aF;
 #pragma unroll
     for (int q = 0; q < NS; q++) {
-      const half2_t u = angle_pair10(Ld.u[q / 3], q % 3);
+      const half2_t u = phase_tab[(Ld.u[q / 3] >> (10 * (q % 3))) & 1023u];
       const SpinH g = tb[nb[q]];
-      t16 += cmul16(u, cmul16(hq[q].s, comp16(g, r)) + cmul16(hq[q].f, comp16(g, 1 - r)));
+      const half2_t gF = comp16(g, rF), gB = comp16(g, rB);
+      aF = cfma16(u, cfma16(hqF[q].f, gB, cmul16(hqF[q].s, gF)), aF);
+      aB = cfma16(u, cfma16(hqB[q].f, gF, cmul16(hqB[q].s, gB)), aB);
     }
-    return {float(t16.x), float(t16.y)};
+    tF = {float(aF.x), float(aF.y)};
+    tB = {float(aB.x), float(aB.y)};
   };
+  if constexpr (!FIRST)
+    for (unsigned k = threadIdx.x; k < 1024u; k += blockDim.x) phase_tab[k] = angle_pair10(k);
   float2 zF[T];   // forward row: the chunk's states (FP32)
   half2_t zB[T];  // backward row: its recurrence inputs, then its states (binary16)
   float2 prevF = {0.f, 0.f};
@@ -534,7 +550,8 @@ __global__ __launch_bounds__(tc_block(T), (NS == 3 ? 4 : 2)) void k_horner_layer
       }
       float2 yF = cmul<float>(cjs, comp(cur.v, rF)), yB = cmul<float>(cjs, comp(cur.v, rB));
       if constexpr (!FIRST) {
-        const float2 tF = transport(cur, tb, hqF, rF), tB = transport(cur, tb, hqB, rB);
+        float2 tF, tB;
+        transport(cur, tb, tF, tB);
         yF.x -= tF.x;
         yF.y -= tF.y;
         yB.x -= tB.x;
@@ -698,7 +715,8 @@ inline int tc_sites(int Lt) {
 // LDS (halos of several times the range, as of randomly numbered tables).
 constexpr size_t kTcLds = 64 * 1024;
 inline size_t tc_smem(int C, int S, int nslot, bool first, int hmax) {
-  return (first ? 0 : size_t(2) * C * (S + hmax) * sizeof(SpinH) + size_t(S) * 2 * nslot * sizeof(HopRow16)) +
+  return (first ? 0 : size_t(2) * C * (S + hmax) * sizeof(SpinH) + size_t(S) * 2 * nslot * sizeof(HopRow16) +
+                          1024 * sizeof(half2_t)) +
          size_t(2) * C * S * sizeof(float2);
 }
 inline TcShape tc_shape(int V, int Lt, int nslot, bool first, int hmax) {
