@@ -138,18 +138,102 @@ __device__ __forceinline__ cplx_t<T> slot_phase(const DiracView<T, P>& d, int s,
   }
 }
 
-// Calls body(std::bool_constant<TG>) with TG = whether the view is in the temporal gauge,
-// decided once per block (a uniform branch on a kernel argument).  Only the 16-bit-angle
-// views of the half-storage solver have a temporal-gauge form.
+// Calls body(std::bool_constant<TG>, std::bool_constant<R1>) with TG = whether the view is in the
+// temporal gauge and R1 = whether the projector form of the hops is used (r = 1), decided once
+// per block (uniform branches on kernel arguments).  Only the 16-bit-angle views of the
+// half-storage solver have either form.
 template <typename T, typename P, class Body>
-__device__ __forceinline__ void with_gauge(const DiracView<T, P>& d, const Body& body) {
+__device__ __forceinline__ void with_form(const DiracView<T, P>& d, const Body& body) {
   if constexpr (std::is_same<P, phase16_t>::value) {
-    if (d.uPoly)
-      body(std::true_type{});
+    auto gauge = [&](auto r1) {
+      if (d.uPoly)
+        body(std::true_type{}, r1);
+      else
+        body(std::false_type{}, r1);
+    };
+    if (d.r == T(1))
+      gauge(std::true_type{});
     else
-      body(std::false_type{});
+      gauge(std::false_type{});
   } else {
-    body(std::false_type{});
+    body(std::false_type{}, std::false_type{});
+  }
+}
+
+// The hop to one neighbour, o += u H p, H = [[-r(C - iS), a - ib], [a + ib, -r(C + iS)]].
+// R1: for r = 1 the hop matrix is a projector times phases (C^2 + S^2 = a^2 + b^2), so its second
+// row is k times the first, k = (a + ib) / -(C - iS), and one product with the first row and the
+// link phase serves both: 18 multiply-adds a hop instead of 28 operations.  Used where the link
+// phases are 16-bit angles, whose rounding (5e-5) is far above that of k (2e-7); there the stencil
+// is bound by VALU issue on six slots: 234 -> 162 vector operations a point, K1 | K2 of the
+// half-storage CG at simplicial n=77, Lt=45 34 | 30 us -> 31 | 27, the solve 10.81 -> 10.08 ms.
+template <typename T, bool R1>
+struct Hop {
+  real4_t<T> h;
+  __device__ __forceinline__ void set(const real4_t<T>& t, T) { h = t; }
+  __device__ __forceinline__ void add(T r, const cplx_t<T>& u, const Spin<T>& p, cplx_t<T>& o0, cplx_t<T>& o1) const {
+    const cplx_t<T> p0 = cmul<T>(u, p.a), p1 = cmul<T>(u, p.b);
+    const T rC = r * h.x, rS = r * h.y, A = h.z, B = h.w;
+    o0.x += -rC * p0.x - rS * p0.y + A * p1.x + B * p1.y;
+    o0.y += -rC * p0.y + rS * p0.x + A * p1.y - B * p1.x;
+    o1.x += A * p0.x - B * p0.y - rC * p1.x + rS * p1.y;
+    o1.y += A * p0.y + B * p0.x - rC * p1.y - rS * p1.x;
+  }
+};
+template <>
+struct Hop<float, true> {
+  float4 h;  // the first row: -(C - iS), a - ib
+  float2 k;
+  __device__ __forceinline__ void set(const float4& t, float) {
+    h = {-t.x, t.y, t.z, -t.w};
+    const float n = t.x * t.x + t.y * t.y, q = n > 1e-37f ? __builtin_amdgcn_rcpf(n) : 0.f;  // padding slots: 0
+    // (a + ib) (-(C + iS)) / (C^2 + S^2)
+    k = {(t.w * t.y - t.z * t.x) * q, -(t.z * t.y + t.w * t.x) * q};
+  }
+  __device__ __forceinline__ void add(float, const float2& u, const Spin<float>& p, float2& o0, float2& o1) const {
+    const float tx = __builtin_fmaf(-h.w, p.b.y, __builtin_fmaf(h.z, p.b.x, __builtin_fmaf(-h.y, p.a.y, h.x * p.a.x)));
+    const float ty = __builtin_fmaf(h.w, p.b.x, __builtin_fmaf(h.z, p.b.y, __builtin_fmaf(h.y, p.a.x, h.x * p.a.y)));
+    const float wx = __builtin_fmaf(-u.y, ty, u.x * tx), wy = __builtin_fmaf(u.y, tx, u.x * ty);
+    o0.x += wx;
+    o0.y += wy;
+    o1.x = __builtin_fmaf(-k.y, wy, __builtin_fmaf(k.x, wx, o1.x));
+    o1.y = __builtin_fmaf(k.y, wx, __builtin_fmaf(k.x, wy, o1.y));
+  }
+};
+
+// The time hops of one point: o += sb T_b conj(ub) prev + sf T_f uf next, with T- = diag(m0, m1),
+// T+ = diag(m1, m0) and (T_b, T_f) = (T-, T+) for D, swapped for D^dagger.  R1: m1 = 0, each hop
+// moves one component.
+template <typename T, bool DAG, bool R1>
+__device__ __forceinline__ void time_hops(T m0, T m1, T sb, T sf, const cplx_t<T>& ub, const cplx_t<T>& uf,
+                                          const Spin<T>& prev, const Spin<T>& next, cplx_t<T>& o0, cplx_t<T>& o1) {
+  using C = cplx_t<T>;
+  if constexpr (R1) {
+    const C q = cconjmul<T>(ub, DAG ? prev.b : prev.a), f = cmul<T>(uf, DAG ? next.a : next.b);
+    const T cb = sb * m0, cf = sf * m0;
+    C& ob = DAG ? o1 : o0;
+    C& of = DAG ? o0 : o1;
+    ob.x += cb * q.x;
+    ob.y += cb * q.y;
+    of.x += cf * f.x;
+    of.y += cf * f.y;
+  } else {
+    const T bk0 = DAG ? m1 : m0, bk1 = DAG ? m0 : m1;
+    const T fw0 = DAG ? m0 : m1, fw1 = DAG ? m1 : m0;
+    {  // backward temporal hop from s-1 with phase exp(-i theta^t_{s-1})
+      const C q0 = cconjmul<T>(ub, prev.a), q1 = cconjmul<T>(ub, prev.b);
+      o0.x += sb * bk0 * q0.x;
+      o0.y += sb * bk0 * q0.y;
+      o1.x += sb * bk1 * q1.x;
+      o1.y += sb * bk1 * q1.y;
+    }
+    {  // forward temporal hop from s+1 with phase exp(+i theta^t_s)
+      const C q0 = cmul<T>(uf, next.a), q1 = cmul<T>(uf, next.b);
+      o0.x += sf * fw0 * q0.x;
+      o0.y += sf * fw0 * q0.y;
+      o1.x += sf * fw1 * q1.x;
+      o1.y += sf * fw1 * q1.y;
+    }
   }
 }
 
@@ -187,27 +271,24 @@ __device__ __forceinline__ void call_center(const Epi&, size_t, const Spin<T>&, 
 
 // The stencil for site x over the time slices [s0, s0+ts), handing every output point
 // to the epilogue (shared by the single-system and the batched kernels).
-template <typename T, int NS, bool DAG, bool TG, class Epi, class In, typename P>
+template <typename T, int NS, bool DAG, bool TG, bool R1, class Epi, class In, typename P>
 __device__ __forceinline__ void stencil_site_src(const DiracView<T, P>& d, const In& in,
                                                  const Epi& epi, int x, int s0, int ts, double2& acc) {
   using C = cplx_t<T>;
   const int V = d.V, Lt = d.Lt;
   if (x < V && s0 < Lt) {
     int nb[NS], lk[NS];
-    real4_t<T> hp[NS];
+    Hop<T, R1> hp[NS];
     const real4_t<T>* hop = DAG ? d.hopd : d.hop;
 #pragma unroll
     for (int j = 0; j < NS; j++) {
       nb[j] = d.nbr[j * V + x];
       lk[j] = d.lnk[j * V + x];
-      hp[j] = hop[j * V + x];
+      hp[j].set(hop[j * V + x], d.r);
     }
     const T c = d.diag[x];
     const T kh = d.kth[x];
     const T m0 = kh * (-d.r - T(1)), m1 = kh * (-d.r + T(1));
-    // T- = diag(m0, m1), T+ = diag(m1, m0); D uses (T- back, T+ fwd), D^dag swaps them.
-    const T bk0 = DAG ? m1 : m0, bk1 = DAG ? m0 : m1;
-    const T fw0 = DAG ? m0 : m1, fw1 = DAG ? m1 : m0;
     const int s1 = min(s0 + ts, Lt);
     const int sm = (s0 == 0) ? Lt - 1 : s0 - 1;
     Spin<T> prev = in(size_t(sm) * V + x);
@@ -225,31 +306,9 @@ __device__ __forceinline__ void stencil_site_src(const DiracView<T, P>& d, const
       for (int j = 0; j < NS; j++) {
         const C u = slot_phase<TG, NS>(d, s, x, j, lk[j]);
         const Spin<T> py = in(sV + nb[j]);
-        const C p0 = cmul<T>(u, py.a), p1 = cmul<T>(u, py.b);
-        const T Cc = hp[j].x, Ss = hp[j].y, A = hp[j].z, B = hp[j].w;
-        // H = [[-r(C - iS), a - ib], [a + ib, -r(C + iS)]]
-        const T rC = d.r * Cc, rS = d.r * Ss;
-        o0.x += -rC * p0.x - rS * p0.y + A * p1.x + B * p1.y;
-        o0.y += -rC * p0.y + rS * p0.x + A * p1.y - B * p1.x;
-        o1.x += A * p0.x - B * p0.y - rC * p1.x + rS * p1.y;
-        o1.y += A * p0.y + B * p0.x - rC * p1.y - rS * p1.x;
+        hp[j].add(d.r, u, py, o0, o1);
       }
-      {  // backward temporal hop from s-1 with phase exp(-i theta^t_{s-1})
-        const T sg = (s == 0) ? d.bc : T(1);
-        const C q0 = cconjmul<T>(uprev, prev.a), q1 = cconjmul<T>(uprev, prev.b);
-        o0.x += sg * bk0 * q0.x;
-        o0.y += sg * bk0 * q0.y;
-        o1.x += sg * bk1 * q1.x;
-        o1.y += sg * bk1 * q1.y;
-      }
-      {  // forward temporal hop from s+1 with phase exp(+i theta^t_s)
-        const T sg = (s == Lt - 1) ? d.bc : T(1);
-        const C q0 = cmul<T>(ucur, next.a), q1 = cmul<T>(ucur, next.b);
-        o0.x += sg * fw0 * q0.x;
-        o0.y += sg * fw0 * q0.y;
-        o1.x += sg * fw1 * q1.x;
-        o1.y += sg * fw1 * q1.y;
-      }
+      time_hops<T, DAG, R1>(m0, m1, s == 0 ? d.bc : T(1), s == Lt - 1 ? d.bc : T(1), uprev, ucur, prev, next, o0, o1);
       Spin<T> o;
       o.a = o0;
       o.b = o1;
@@ -272,8 +331,8 @@ __global__ __launch_bounds__(256) void k_stencil(DiracView<T, P> d, Src in, Epi 
   double2 acc = {0.0, 0.0};
   epi.begin();
   const auto bound = in.bind();
-  with_gauge(d, [&](auto tg) {
-    stencil_site_src<T, NS, DAG, decltype(tg)::value>(d, bound, epi, x, st * ts, ts, acc);
+  with_form(d, [&](auto tg, auto r1) {
+    stencil_site_src<T, NS, DAG, decltype(tg)::value, decltype(r1)::value>(d, bound, epi, x, st * ts, ts, acc);
   });
   if constexpr (Epi::kReduce) store_partial(acc, gr.partials, blockIdx.x);
 }
@@ -295,7 +354,7 @@ __host__ __device__ constexpr size_t lds_bytes(int block, int hmax) {
   return size_t(kLdsBuffers) * size_t(block + hmax) * sizeof(Spin<T>);
 }
 
-template <typename T, int NS, bool DAG, bool TG, class Epi, class In, typename P>
+template <typename T, int NS, bool DAG, bool TG, bool R1, class Epi, class In, typename P>
 __device__ __forceinline__ void stencil_lds_block(const DiracView<T, P>& d, const In& in, const Epi& epi,
                                                   int ts, int xr, int nxr, int st, const HaloView& hv,
                                                   Spin<T>* tileS, double2& acc) {
@@ -315,8 +374,8 @@ __device__ __forceinline__ void stencil_lds_block(const DiracView<T, P>& d, cons
   const int hid0 = (int(threadIdx.x) < nh) ? hv.halo[h0 + threadIdx.x] : -1;
   const int hid1 = (int(threadIdx.x) + R < nh) ? hv.halo[h0 + threadIdx.x + R] : -1;
   int nb[NS], lk[NS];
-  real4_t<T> hp[NS];
-  T c = 0, bk0 = 0, bk1 = 0, fw0 = 0, fw1 = 0;
+  Hop<T, R1> hp[NS];
+  T c = 0, m0 = 0, m1 = 0;
   Spin<T> prev, cur;
   C uprev;
   if (act && s0 < Lt) {
@@ -325,15 +384,12 @@ __device__ __forceinline__ void stencil_lds_block(const DiracView<T, P>& d, cons
     for (int j = 0; j < NS; j++) {
       nb[j] = hv.nbl[j * V + x];
       lk[j] = d.lnk[j * V + x];
-      hp[j] = hop[j * V + x];
+      hp[j].set(hop[j * V + x], d.r);
     }
     c = d.diag[x];
     const T kh = d.kth[x];
-    const T m0 = kh * (-d.r - T(1)), m1 = kh * (-d.r + T(1));
-    bk0 = DAG ? m1 : m0;
-    bk1 = DAG ? m0 : m1;
-    fw0 = DAG ? m0 : m1;
-    fw1 = DAG ? m1 : m0;
+    m0 = kh * (-d.r - T(1));
+    m1 = kh * (-d.r + T(1));
     const int sm = (s0 == 0) ? Lt - 1 : s0 - 1;
     prev = in(size_t(sm) * V + x);
     cur = in(size_t(s0) * V + x);
@@ -366,32 +422,9 @@ __device__ __forceinline__ void stencil_lds_block(const DiracView<T, P>& d, cons
       C o0 = cscale<T>(c, cur.a), o1 = cscale<T>(c, cur.b);
 #pragma unroll
       for (int j = 0; j < NS; j++) {
-        const C u = uu[j];
-        const Spin<T> py = tb[nb[j]];
-        const C p0 = cmul<T>(u, py.a), p1 = cmul<T>(u, py.b);
-        const T Cc = hp[j].x, Ss = hp[j].y, A = hp[j].z, B = hp[j].w;
-        const T rC = d.r * Cc, rS = d.r * Ss;
-        o0.x += -rC * p0.x - rS * p0.y + A * p1.x + B * p1.y;
-        o0.y += -rC * p0.y + rS * p0.x + A * p1.y - B * p1.x;
-        o1.x += A * p0.x - B * p0.y - rC * p1.x + rS * p1.y;
-        o1.y += A * p0.y + B * p0.x - rC * p1.y - rS * p1.x;
+        hp[j].add(d.r, uu[j], tb[nb[j]], o0, o1);
       }
-      {
-        const T sg = (s == 0) ? d.bc : T(1);
-        const C q0 = cconjmul<T>(uprev, prev.a), q1 = cconjmul<T>(uprev, prev.b);
-        o0.x += sg * bk0 * q0.x;
-        o0.y += sg * bk0 * q0.y;
-        o1.x += sg * bk1 * q1.x;
-        o1.y += sg * bk1 * q1.y;
-      }
-      {
-        const T sg = (s == Lt - 1) ? d.bc : T(1);
-        const C q0 = cmul<T>(ucur, next.a), q1 = cmul<T>(ucur, next.b);
-        o0.x += sg * fw0 * q0.x;
-        o0.y += sg * fw0 * q0.y;
-        o1.x += sg * fw1 * q1.x;
-        o1.y += sg * fw1 * q1.y;
-      }
+      time_hops<T, DAG, R1>(m0, m1, s == 0 ? d.bc : T(1), s == Lt - 1 ? d.bc : T(1), uprev, ucur, prev, next, o0, o1);
       Spin<T> o;
       o.a = o0;
       o.b = o1;
@@ -416,8 +449,9 @@ __global__ __launch_bounds__(256) void k_stencil_lds(DiracView<T, P> d, Src src,
   tile_of(tm, blockIdx.x, xr, st);
   double2 acc = {0.0, 0.0};
   epi.begin();
-  with_gauge(d, [&](auto tg) {
-    stencil_lds_block<T, NS, DAG, decltype(tg)::value>(d, in, epi, ts, xr, tm.nxr, st, hv, tileS, acc);
+  with_form(d, [&](auto tg, auto r1) {
+    stencil_lds_block<T, NS, DAG, decltype(tg)::value, decltype(r1)::value>(d, in, epi, ts, xr, tm.nxr, st, hv, tileS,
+                                                                            acc);
   });
   if constexpr (Epi::kReduce) store_partial(acc, gr.partials, blockIdx.x);
 }
