@@ -127,7 +127,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_stencil(const Sys* __restrict_
     auto run = [&](const auto v, const auto& in, auto tag) {
       using T = decltype(tag);
       Spin<T>* tile = reinterpret_cast<Spin<T>*>(smem_raw);
-      with_form(v, [&](auto tg, auto r1) {
+      with_form<EpiProjectorHops<std::decay_t<decltype(epi)>, NS>::value>(v, [&](auto tg, auto r1) {
         stencil_lds_block<T, NS, DAG, decltype(tg)::value, decltype(r1)::value>(v, in, epi, ts, xr, nxr, st, hv, tile,
                                                                                 acc);
       });

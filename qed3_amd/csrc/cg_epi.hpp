@@ -199,6 +199,9 @@ template <int POS>
 struct EpiK2H {
   static constexpr bool kReduce = true;
   static constexpr bool kUpdateX = POS == kXGroup - 1;
+  // the projector hops' two further registers a slot cost this position the fifth wave per SIMD
+  // on three slots (96 -> 98 VGPRs, see prefetch below), where VALU issue does not bound it
+  static constexpr bool kGeneralHops = kUpdateX;
   Spin<float>* x;
   SpinH* r;
   const SpinH* ring[kXGroup];  // ring[POS] is this iteration's p

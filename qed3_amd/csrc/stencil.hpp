@@ -141,8 +141,8 @@ __device__ __forceinline__ cplx_t<T> slot_phase(const DiracView<T, P>& d, int s,
 // Calls body(std::bool_constant<TG>, std::bool_constant<R1>) with TG = whether the view is in the
 // temporal gauge and R1 = whether the projector form of the hops is used (r = 1), decided once
 // per block (uniform branches on kernel arguments).  Only the 16-bit-angle views of the
-// half-storage solver have either form.
-template <typename T, typename P, class Body>
+// half-storage solver have either form; R1OK = false leaves out the projector's.
+template <bool R1OK, typename T, typename P, class Body>
 __device__ __forceinline__ void with_form(const DiracView<T, P>& d, const Body& body) {
   if constexpr (std::is_same<P, phase16_t>::value) {
     auto gauge = [&](auto r1) {
@@ -151,14 +151,20 @@ __device__ __forceinline__ void with_form(const DiracView<T, P>& d, const Body& 
       else
         body(std::false_type{}, r1);
     };
-    if (d.r == T(1))
-      gauge(std::true_type{});
-    else
-      gauge(std::false_type{});
+    if constexpr (R1OK) {
+      if (d.r == T(1)) return gauge(std::true_type{});
+    }
+    gauge(std::false_type{});
   } else {
     body(std::false_type{}, std::false_type{});
   }
 }
+
+// An epilogue that names kGeneralHops keeps the general hops on trivalent sites (its registers)
+template <class E, int NS, class = void>
+struct EpiProjectorHops : std::true_type {};
+template <class E>
+struct EpiProjectorHops<E, 3, std::void_t<decltype(E::kGeneralHops)>> : std::bool_constant<!E::kGeneralHops> {};
 
 // The hop to one neighbour, o += u H p, H = [[-r(C - iS), a - ib], [a + ib, -r(C + iS)]].
 // R1: for r = 1 the hop matrix is a projector times phases (C^2 + S^2 = a^2 + b^2), so its second
@@ -166,7 +172,8 @@ __device__ __forceinline__ void with_form(const DiracView<T, P>& d, const Body& 
 // link phase serves both: 18 multiply-adds a hop instead of 28 operations.  Used where the link
 // phases are 16-bit angles, whose rounding (5e-5) is far above that of k (2e-7); there the stencil
 // is bound by VALU issue on six slots: 234 -> 162 vector operations a point, K1 | K2 of the
-// half-storage CG at simplicial n=77, Lt=45 34 | 30 us -> 31 | 27, the solve 10.81 -> 10.08 ms.
+// half-storage CG at simplicial n=77, Lt=45 34 | 30 us -> 31 | 27, the solve 10.81 -> 10.08 ms; dual
+// n=128, Lt=64 178 | 152 -> 173 | 137, the solve 63.2 -> 60.7 ms.
 template <typename T, bool R1>
 struct Hop {
   real4_t<T> h;
@@ -331,7 +338,7 @@ __global__ __launch_bounds__(256) void k_stencil(DiracView<T, P> d, Src in, Epi 
   double2 acc = {0.0, 0.0};
   epi.begin();
   const auto bound = in.bind();
-  with_form(d, [&](auto tg, auto r1) {
+  with_form<EpiProjectorHops<Epi, NS>::value>(d, [&](auto tg, auto r1) {
     stencil_site_src<T, NS, DAG, decltype(tg)::value, decltype(r1)::value>(d, bound, epi, x, st * ts, ts, acc);
   });
   if constexpr (Epi::kReduce) store_partial(acc, gr.partials, blockIdx.x);
@@ -449,7 +456,7 @@ __global__ __launch_bounds__(256) void k_stencil_lds(DiracView<T, P> d, Src src,
   tile_of(tm, blockIdx.x, xr, st);
   double2 acc = {0.0, 0.0};
   epi.begin();
-  with_form(d, [&](auto tg, auto r1) {
+  with_form<EpiProjectorHops<Epi, NS>::value>(d, [&](auto tg, auto r1) {
     stencil_lds_block<T, NS, DAG, decltype(tg)::value, decltype(r1)::value>(d, in, epi, ts, xr, tm.nxr, st, hv, tileS,
                                                                             acc);
   });
