@@ -1,16 +1,17 @@
 // Device-driven CG on A = D^dagger D (the role of MatPoly::solve,
 // src/both_3d/matpoly.h:204-267).
 //
-// Each iteration is five kernels (plus the one-block reduction finalisers) whose control
-// flow lives on the device:
+// Each iteration is two kernels (plus the one-block reduction finalisers), each chunk of
+// iterations ends with a reliable update, and the control flow lives on the device:
 //   K1  p = r + beta p_old (formed while gathering), w = D p, gam = |w|^2
 //   K2  q = D^dag w,       alpha = mu/gam, x += alpha p, r -= alpha q, |r|^2
 //   U1  x64 += x_inner                           (only when a reliable update is due)
 //   U2  t = D x64                                (FP64, only when due)
 //   U3  r64 = b - D^dag t, r_inner = r64, |r64|^2 (FP64, only when due)
 // Kernels read the scalars (alpha, beta, flags) from device memory and exit at once
-// when the solve is finished or no update is due, so a chunk of iterations is
-// captured once in a hipGraph and replayed with one host poll per chunk.
+// when the solve is finished or no update is due (one that is due ends its chunk's
+// iterations), so a chunk is captured once in a hipGraph, kept with the context, and
+// replayed with one host poll per chunk.
 //
 // Inner precision float gives FP32 CG with FP64 reliable updates (Sleijpen & van der
 // Vorst 1996; Clark et al., CPC 181 (2010) 1517): the FP64 residual is recomputed

@@ -39,9 +39,6 @@ namespace qed3 {
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
-// Spinor fields of the preconditioner are stored spin-planar: plane a holds the spin
-// component a of every point (s, x) at [a * n + s * V + x], so the thread that walks the
-// time column of one spin row reads and writes contiguous values.
 struct HornerParams {
   int layers = 4;
   std::vector<std::complex<double>> c;  // [layers], c[j] multiplies the input at layer j

@@ -1,6 +1,6 @@
 """The learned method's parallel-in-time layers at every chunk length (4, 8 or 16 slices a lane
 by the lattice's size, 16 on split blocks beyond 64 slices): K, K^dagger and K K^dagger by the
-solver's kernels against the FP32 two-pass layers, which the oracle checks."""
+solver's kernels against the FP32 layers, which the oracle checks."""
 import numpy as np
 import pytest
 
