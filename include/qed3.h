@@ -286,7 +286,8 @@ int qed3_pcg_kernel_times(qed3_ctx* ctx, qed3_precond* pc, void* d_x, const void
  * chunks of iterations on its own stream, the next queued as soon as the stream has drained;
  * many systems too small to cover the GPU with one launch (< 256 blocks of 256) instead share
  * launches in which every CG phase runs over all of them (per-system scalars and convergence
- * masks, iterations captured in a hipGraph).  The reference runs one CG per right-hand side (PseudoFermion::update_eta,
+ * masks, iterations captured in a hipGraph).  A context may be listed several times, once per
+ * right-hand side.  The reference runs one CG per right-hand side (PseudoFermion::update_eta,
  * pseudofermion.h:51, looped in integrator.h:156-166).  reps[nsys] may be NULL. */
 int qed3_batch_cg(qed3_ctx* const* ctxs, int nsys, void* const* d_x, const void* const* d_b,
                   const qed3_cg_opts* opts, qed3_cg_report* reps);

@@ -3,6 +3,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstdlib>
+#include <map>
 
 #include "batch.hpp"
 #include "cg_epi.hpp"
@@ -238,46 +239,50 @@ std::vector<CGResult> batch_cg(const std::vector<Dirac*>& Ds, const std::vector<
   for (Dirac* D : Ds)
     if (!D->has_gauge()) throw std::invalid_argument("batch: a system has no gauge field");
   const auto t0 = std::chrono::steady_clock::now();
-  std::vector<int> big, small;
+  // A context's work fields, scalars and captured chunk hold one solve at a time: the systems of a
+  // context listed several times (several sources on one operator) share launches, whose fields are
+  // a system's own, or take turns on its stream.
+  std::map<const Dirac*, int> seen;
+  std::vector<int> small;
+  bool repeats = false;  // among the small ones
+  std::vector<std::vector<int>> big(1);  // per turn, no context twice in one
   for (int k = 0; k < ns; k++) {
     const Dirac& D = *Ds[k];
+    const size_t turn = size_t(seen[Ds[k]]++);
     const int ts = std::max(1, std::min(D.tile<float>(false).ts, D.Lt()));
     const long blocks = long((D.V() + kBlock - 1) / kBlock) * ((D.Lt() + ts - 1) / ts);
-    (blocks >= kLargeBlocks ? big : small).push_back(k);
+    if (big.size() <= turn) big.resize(turn + 1);
+    if (blocks >= kLargeBlocks) {
+      big[turn].push_back(k);
+    } else {
+      small.push_back(k);
+      repeats = repeats || turn > 0;
+    }
   }
   double mpoints = 0;
   for (int k : small) mpoints += 1e-6 * double(Ds[k]->points());
-  if (kOwnPerSystem * double(small.size()) <= kBatchBase + kBatchPerMpoint * mpoints) {
-    big.insert(big.end(), small.begin(), small.end());
+  if (!repeats && kOwnPerSystem * double(small.size()) <= kBatchBase + kBatchPerMpoint * mpoints) {
+    big[0].insert(big[0].end(), small.begin(), small.end());
     small.clear();
   }
   std::vector<CGResult> out(ns);
   CGOptions os = o;
   os.mixed = os.half = true;
-  if (!big.empty()) {
+  auto solve = [&](const std::vector<int>& which, bool shared) {
+    if (which.empty()) return;
     std::vector<Dirac*> d;
     std::vector<Spin<double>*> x;
     std::vector<const Spin<double>*> b;
-    for (int k : big) {
+    for (int k : which) {
       d.push_back(Ds[k]);
       x.push_back(xs[k]);
       b.push_back(bs[k]);
     }
-    const std::vector<CGResult> r = cg_solve_half_many(d, x, b, os);
-    for (size_t j = 0; j < big.size(); j++) out[big[j]] = r[j];
-  }
-  if (!small.empty()) {
-    std::vector<Dirac*> d;
-    std::vector<Spin<double>*> x;
-    std::vector<const Spin<double>*> b;
-    for (int k : small) {
-      d.push_back(Ds[k]);
-      x.push_back(xs[k]);
-      b.push_back(bs[k]);
-    }
-    const std::vector<CGResult> r = batch_launches(d, x, b, o);
-    for (size_t j = 0; j < small.size(); j++) out[small[j]] = r[j];
-  }
+    const std::vector<CGResult> r = shared ? batch_launches(d, x, b, o) : cg_solve_half_many(d, x, b, os);
+    for (size_t j = 0; j < which.size(); j++) out[which[j]] = r[j];
+  };
+  for (const auto& t : big) solve(t, false);
+  solve(small, true);
   const double secs = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   for (auto& r : out) r.seconds = secs;
   return out;

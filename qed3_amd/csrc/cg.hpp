@@ -72,8 +72,8 @@ double true_residual(Dirac& D, const Spin<double>* x, const Spin<double>* b);
 // graph, scalars read back into host stack memory, and the LDS stencil only where the
 // context already holds its halo tables (the plain stencil otherwise).
 size_t cg_workspace_bytes(size_t points);
-// Several systems by the half-storage solver (o.half implied), each on its own context's
-// stream: a chunk of iterations of every system is queued, and each system's next one as soon
+// Several systems by the half-storage solver (o.half implied), each on its own context (no context
+// twice) and its stream: a chunk of iterations of every system is queued, and each system's next one as soon
 // as its stream has drained, so the GPU runs the systems' chunks back to back and concurrently.
 std::vector<CGResult> cg_solve_half_many(const std::vector<Dirac*>& Ds, const std::vector<Spin<double>*>& xs,
                                          const std::vector<const Spin<double>*>& bs, const CGOptions& o);
