@@ -771,9 +771,16 @@ void Net::upload_params() {
   QED3_HIP(hipMemcpy(mixAH_, AH.data(), AH.size() * sizeof(bf16), hipMemcpyHostToDevice));
 }
 
+// Buffers for batches of up to capB_ pairs, with those of training if cap_train_.  Growing frees all
+// of them, so the flag says what this call allocates: an inference with a larger batch after a
+// training call takes no training buffers, and the next training call allocates them again.  The
+// capacity is zero until every allocation has succeeded.
 void Net::ensure(int B, bool training) {
   if (B <= capB_ && (!training || cap_train_)) return;
-  const size_t np = size_t(std::max(B, capB_)) * D_.points();
+  const int cap = std::max(B, capB_);
+  const size_t np = size_t(cap) * D_.points();
+  capB_ = 0;
+  cap_train_ = false;
   for (void* p : {act_, (void*)gfield_, (void*)gfield2_, (void*)out_, (void*)gout_,
                   (void*)partial_, (void*)red_})
     if (p) (void)hipFree(p);
@@ -788,14 +795,13 @@ void Net::ensure(int B, bool training) {
     gfield2_ = dmalloc<float>(np * 2 * RW);
     out_ = dmalloc<Spin<float>>(np);
     gout_ = dmalloc<Spin<float>>(np);
-    const size_t nB = std::max(B, capB_);
     partial_ = dmalloc<double>(std::max({sum_blocks(np, PTS) * size_t(2 * RW * KF),
                                          sum_blocks(np, 256) * size_t(2 * kHeadCols),
-                                         nB * 2 * sum_blocks(D_.points(), 256)}));
-    red_ = dmalloc<double>(2 * RW * KF + 2 * nB);
+                                         size_t(cap) * 2 * sum_blocks(D_.points(), 256)}));
+    red_ = dmalloc<double>(2 * RW * KF + 2 * size_t(cap));
   }
-  capB_ = std::max(B, capB_);
-  cap_train_ = cap_train_ || training;
+  capB_ = cap;
+  cap_train_ = training;
 }
 
 void Net::apply(Spin<float>* out, const Spin<float>* r, int B) {
