@@ -36,8 +36,8 @@ struct PhaseTables {
   float2 *fS, *fT;
   phase16_t *hS, *hT;
 };
-__global__ __launch_bounds__(256) void k_phases(const double* __restrict__ srcS, const double* __restrict__ srcT,
-                                                PhaseTables t, size_t nS, size_t n) {
+__global__ __launch_bounds__(256) void k_phases(const double* srcS, const double* srcT, PhaseTables t, size_t nS,
+                                                size_t n) {
   const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const bool sp = i < nS;
@@ -585,16 +585,39 @@ HaloView Dirac::halo(int R) {
   return v;
 }
 
+namespace {
+// Whether a kernel on the current device may read `bytes` at p in place: aligned memory of this
+// device, all of it inside its allocation.  Anything else (host memory, another device's, a short
+// or unknown range) is left to a copy, which finds out where it lies or reports the error; 0.6 us.
+bool kernel_can_read(const void* p, size_t bytes) {
+  hipPointerAttribute_t at{};
+  hipDeviceptr_t base{};
+  size_t size = 0;
+  int dev = -1;
+  const bool ok = reinterpret_cast<uintptr_t>(p) % alignof(double) == 0 && hipGetDevice(&dev) == hipSuccess &&
+                  hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeDevice && at.device == dev &&
+                  hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) == hipSuccess &&
+                  static_cast<const char*>(p) + bytes <= static_cast<const char*>(base) + size;
+  if (!ok) (void)hipGetLastError();  // an answer, not an error to be reported by the next launch
+  return ok;
+}
+}  // namespace
+
 void Dirac::set_gauge(const double* spatial, const double* temporal, bool on_device) {
   const size_t nS = size_t(h_.Lt) * h_.E, nT = size_t(h_.Lt) * h_.V;
-  if (!on_device) {
-    QED3_HIP(hipMemcpyAsync(angS_, spatial, nS * sizeof(double), hipMemcpyHostToDevice, stream_));
-    QED3_HIP(hipMemcpyAsync(angT_, temporal, nT * sizeof(double), hipMemcpyHostToDevice, stream_));
-  }
+  // the array the phases are made from: the caller's, or the context's after a copy
+  auto source = [&](const double* src, double* own, size_t n) -> const double* {
+    if (on_device && kernel_can_read(src, n * sizeof(double))) return src;
+    const hipError_t e = hipMemcpyAsync(own, src, n * sizeof(double),
+                                        on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, stream_);
+    if (e != hipSuccess) (void)hipGetLastError();
+    QED3_HIP(e);
+    return own;
+  };
+  const double *srcS = source(spatial, angS_, nS), *srcT = source(temporal, angT_, nT);
   const PhaseTables t{angS_, angT_, d64_.uS, d64_.uT, d32_.uS, d32_.uT, uSh_, uTh_};
   const int B = 256;
-  hipLaunchKernelGGL(k_phases, dim3(unsigned((nS + nT + B - 1) / B)), dim3(B), 0, stream_, on_device ? spatial : angS_,
-                     on_device ? temporal : angT_, t, nS, nS + nT);
+  hipLaunchKernelGGL(k_phases, dim3(unsigned((nS + nT + B - 1) / B)), dim3(B), 0, stream_, srcS, srcT, t, nS, nS + nT);
   QED3_HIP(hipGetLastError());
   if (uStg_) fill_temporal_gauge();
   QED3_HIP(hipStreamSynchronize(stream_));
