@@ -90,22 +90,11 @@ class ChunkLoop {
     if (o.use_graph && !o.times && std::getenv("QED3_NO_GRAPH") == nullptr) {
       GraphSlot& g = slot ? *slot : own_;
       key.add(chunk_);
-      if (!g.exec || g.key != key.words) {
-        g.clear();
-        QED3_HIP(hipStreamBeginCapture(st_, hipStreamCaptureModeThreadLocal));
-        try {
+      if (!g.exec || g.key != key.words)
+        g.capture(st_, key.words, [&] {
           for (int i = 0; i < chunk_; i++) one_iter_(i, -1);
           tail_();
-        } catch (...) {
-          hipGraph_t dead = nullptr;  // end the capture, or the stream stays in it
-          (void)hipStreamEndCapture(st_, &dead);
-          if (dead) (void)hipGraphDestroy(dead);
-          throw;
-        }
-        QED3_HIP(hipStreamEndCapture(st_, &g.graph));
-        QED3_HIP(hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0));
-        g.key = key.words;
-      }
+        });
       exec_ = g.exec;
     }
   }

@@ -116,6 +116,23 @@ struct GraphSlot {
     graph = nullptr;
     key.clear();
   }
+  // capture what body() queues on st; if it throws, the capture is ended and the slot left empty
+  template <class Body>
+  void capture(hipStream_t st, std::vector<unsigned long long> k, const Body& body) {
+    clear();
+    QED3_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+    try {
+      body();
+    } catch (...) {
+      hipGraph_t dead = nullptr;  // or the stream stays in it
+      (void)hipStreamEndCapture(st, &dead);
+      if (dead) (void)hipGraphDestroy(dead);
+      throw;
+    }
+    QED3_HIP(hipStreamEndCapture(st, &graph));
+    QED3_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
+    key = std::move(k);
+  }
   GraphSlot() = default;
   ~GraphSlot() { clear(); }
   GraphSlot(const GraphSlot&) = delete;

@@ -415,7 +415,14 @@ std::vector<CGResult> multishift_cg(Dirac& D, const std::vector<double>& shifts,
   const DiracView<double> v64 = D.view<double>();
   const int nn = D.tables().max_nn;
   const HaloView hvf = D.halo_for<double>(false), hvt = D.halo_for<double>(true);
-  const StencilTile tf = D.tile<double>(false), tt = D.tile<double>(true);
+  // the norms take one partial a block: more slices a thread where the set shape's grid has more
+  // blocks than the reduction scratch
+  auto fit = [&](StencilTile t) {
+    const size_t nxr = size_t((D.V() + t.block - 1) / t.block + 7) / 8 * 8;
+    while (t.ts < D.Lt() && nxr * size_t((D.Lt() + t.ts - 1) / t.ts) > kReduceCapacity) t.ts *= 2;
+    return t;
+  };
+  const StencilTile tf = fit(D.tile<double>(false)), tt = fit(D.tile<double>(true));
   // rows of the update pass: up to 2,048 blocks over the points and the shifts
   const unsigned rows = std::max(1u, std::min(unsigned(ns), 2048u / nb));
   auto one_iter = [&] {
@@ -433,14 +440,10 @@ std::vector<CGResult> multishift_cg(Dirac& D, const std::vector<double>& shifts,
     GraphKey key;
     key.add(v64).add(hvf).add(hvt).add(tf).add(tt).add(base).add(gr.partials).add(n).add(nn).add(ns).add(S.base);
     GraphSlot& g = D.graph_slot(3);
-    if (!g.exec || g.key != key.words) {
-      g.clear();
-      QED3_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-      for (int c = 0; c < chunk; c++) one_iter();
-      QED3_HIP(hipStreamEndCapture(st, &g.graph));
-      QED3_HIP(hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0));
-      g.key = key.words;
-    }
+    if (!g.exec || g.key != key.words)
+      g.capture(st, key.words, [&] {
+        for (int c = 0; c < chunk; c++) one_iter();
+      });
     exec = g.exec;
   }
   for (int c = 0; c <= o.maxiter / chunk + 1; c++) {
