@@ -208,40 +208,22 @@ struct Hop<float, true> {
   }
 };
 
-// The time hops of one point: o += sb T_b conj(ub) prev + sf T_f uf next, with T- = diag(m0, m1),
-// T+ = diag(m1, m0) and (T_b, T_f) = (T-, T+) for D, swapped for D^dagger.  R1: m1 = 0, each hop
-// moves one component.
-template <typename T, bool DAG, bool R1>
-__device__ __forceinline__ void time_hops(T m0, T m1, T sb, T sf, const cplx_t<T>& ub, const cplx_t<T>& uf,
-                                          const Spin<T>& prev, const Spin<T>& next, cplx_t<T>& o0, cplx_t<T>& o1) {
+// The time hops of one point for r = 1, where T- = diag(m0, 0) and T+ = diag(0, m0): each moves one
+// component.  o += sb T_b conj(ub) prev + sf T_f uf next with (T_b, T_f) = (T-, T+) for D, swapped
+// for D^dagger.  The general hops stand in the stencils themselves: inside a function shared with this
+// form the compiler fuses other products into the multiply-adds, and FP64 and FP32 results change.
+template <typename T, bool DAG>
+__device__ __forceinline__ void time_hops_r1(T m0, T sb, T sf, const cplx_t<T>& ub, const cplx_t<T>& uf,
+                                             const Spin<T>& prev, const Spin<T>& next, cplx_t<T>& o0, cplx_t<T>& o1) {
   using C = cplx_t<T>;
-  if constexpr (R1) {
-    const C q = cconjmul<T>(ub, DAG ? prev.b : prev.a), f = cmul<T>(uf, DAG ? next.a : next.b);
-    const T cb = sb * m0, cf = sf * m0;
-    C& ob = DAG ? o1 : o0;
-    C& of = DAG ? o0 : o1;
-    ob.x += cb * q.x;
-    ob.y += cb * q.y;
-    of.x += cf * f.x;
-    of.y += cf * f.y;
-  } else {
-    const T bk0 = DAG ? m1 : m0, bk1 = DAG ? m0 : m1;
-    const T fw0 = DAG ? m0 : m1, fw1 = DAG ? m1 : m0;
-    {  // backward temporal hop from s-1 with phase exp(-i theta^t_{s-1})
-      const C q0 = cconjmul<T>(ub, prev.a), q1 = cconjmul<T>(ub, prev.b);
-      o0.x += sb * bk0 * q0.x;
-      o0.y += sb * bk0 * q0.y;
-      o1.x += sb * bk1 * q1.x;
-      o1.y += sb * bk1 * q1.y;
-    }
-    {  // forward temporal hop from s+1 with phase exp(+i theta^t_s)
-      const C q0 = cmul<T>(uf, next.a), q1 = cmul<T>(uf, next.b);
-      o0.x += sf * fw0 * q0.x;
-      o0.y += sf * fw0 * q0.y;
-      o1.x += sf * fw1 * q1.x;
-      o1.y += sf * fw1 * q1.y;
-    }
-  }
+  const C q = cconjmul<T>(ub, DAG ? prev.b : prev.a), f = cmul<T>(uf, DAG ? next.a : next.b);
+  const T cb = sb * m0, cf = sf * m0;
+  C& ob = DAG ? o1 : o0;
+  C& of = DAG ? o0 : o1;
+  ob.x += cb * q.x;
+  ob.y += cb * q.y;
+  of.x += cf * f.x;
+  of.y += cf * f.y;
 }
 
 // Epilogues may load what they need at an output point early through pre = prefetch(i),
@@ -296,6 +278,9 @@ __device__ __forceinline__ void stencil_site_src(const DiracView<T, P>& d, const
     const T c = d.diag[x];
     const T kh = d.kth[x];
     const T m0 = kh * (-d.r - T(1)), m1 = kh * (-d.r + T(1));
+    // T- = diag(m0, m1), T+ = diag(m1, m0); D uses (T- back, T+ fwd), D^dag swaps them.
+    const T bk0 = DAG ? m1 : m0, bk1 = DAG ? m0 : m1;
+    const T fw0 = DAG ? m0 : m1, fw1 = DAG ? m1 : m0;
     const int s1 = min(s0 + ts, Lt);
     const int sm = (s0 == 0) ? Lt - 1 : s0 - 1;
     Spin<T> prev = in(size_t(sm) * V + x);
@@ -315,7 +300,26 @@ __device__ __forceinline__ void stencil_site_src(const DiracView<T, P>& d, const
         const Spin<T> py = in(sV + nb[j]);
         hp[j].add(d.r, u, py, o0, o1);
       }
-      time_hops<T, DAG, R1>(m0, m1, s == 0 ? d.bc : T(1), s == Lt - 1 ? d.bc : T(1), uprev, ucur, prev, next, o0, o1);
+      if constexpr (R1) {
+        time_hops_r1<T, DAG>(m0, s == 0 ? d.bc : T(1), s == Lt - 1 ? d.bc : T(1), uprev, ucur, prev, next, o0, o1);
+      } else {
+        {  // backward temporal hop from s-1 with phase exp(-i theta^t_{s-1})
+          const T sg = (s == 0) ? d.bc : T(1);
+          const C q0 = cconjmul<T>(uprev, prev.a), q1 = cconjmul<T>(uprev, prev.b);
+          o0.x += sg * bk0 * q0.x;
+          o0.y += sg * bk0 * q0.y;
+          o1.x += sg * bk1 * q1.x;
+          o1.y += sg * bk1 * q1.y;
+        }
+        {  // forward temporal hop from s+1 with phase exp(+i theta^t_s)
+          const T sg = (s == Lt - 1) ? d.bc : T(1);
+          const C q0 = cmul<T>(ucur, next.a), q1 = cmul<T>(ucur, next.b);
+          o0.x += sg * fw0 * q0.x;
+          o0.y += sg * fw0 * q0.y;
+          o1.x += sg * fw1 * q1.x;
+          o1.y += sg * fw1 * q1.y;
+        }
+      }
       Spin<T> o;
       o.a = o0;
       o.b = o1;
@@ -382,7 +386,7 @@ __device__ __forceinline__ void stencil_lds_block(const DiracView<T, P>& d, cons
   const int hid1 = (int(threadIdx.x) + R < nh) ? hv.halo[h0 + threadIdx.x + R] : -1;
   int nb[NS], lk[NS];
   Hop<T, R1> hp[NS];
-  T c = 0, m0 = 0, m1 = 0;
+  T c = 0, m0 = 0, bk0 = 0, bk1 = 0, fw0 = 0, fw1 = 0;
   Spin<T> prev, cur;
   C uprev;
   if (act && s0 < Lt) {
@@ -396,7 +400,11 @@ __device__ __forceinline__ void stencil_lds_block(const DiracView<T, P>& d, cons
     c = d.diag[x];
     const T kh = d.kth[x];
     m0 = kh * (-d.r - T(1));
-    m1 = kh * (-d.r + T(1));
+    const T m1 = kh * (-d.r + T(1));
+    bk0 = DAG ? m1 : m0;
+    bk1 = DAG ? m0 : m1;
+    fw0 = DAG ? m0 : m1;
+    fw1 = DAG ? m1 : m0;
     const int sm = (s0 == 0) ? Lt - 1 : s0 - 1;
     prev = in(size_t(sm) * V + x);
     cur = in(size_t(s0) * V + x);
@@ -431,7 +439,26 @@ __device__ __forceinline__ void stencil_lds_block(const DiracView<T, P>& d, cons
       for (int j = 0; j < NS; j++) {
         hp[j].add(d.r, uu[j], tb[nb[j]], o0, o1);
       }
-      time_hops<T, DAG, R1>(m0, m1, s == 0 ? d.bc : T(1), s == Lt - 1 ? d.bc : T(1), uprev, ucur, prev, next, o0, o1);
+      if constexpr (R1) {
+        time_hops_r1<T, DAG>(m0, s == 0 ? d.bc : T(1), s == Lt - 1 ? d.bc : T(1), uprev, ucur, prev, next, o0, o1);
+      } else {
+        {
+          const T sg = (s == 0) ? d.bc : T(1);
+          const C q0 = cconjmul<T>(uprev, prev.a), q1 = cconjmul<T>(uprev, prev.b);
+          o0.x += sg * bk0 * q0.x;
+          o0.y += sg * bk0 * q0.y;
+          o1.x += sg * bk1 * q1.x;
+          o1.y += sg * bk1 * q1.y;
+        }
+        {
+          const T sg = (s == Lt - 1) ? d.bc : T(1);
+          const C q0 = cmul<T>(ucur, next.a), q1 = cmul<T>(ucur, next.b);
+          o0.x += sg * fw0 * q0.x;
+          o0.y += sg * fw0 * q0.y;
+          o1.x += sg * fw1 * q1.x;
+          o1.y += sg * fw1 * q1.y;
+        }
+      }
       Spin<T> o;
       o.a = o0;
       o.b = o1;
