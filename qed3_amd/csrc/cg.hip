@@ -190,6 +190,12 @@ struct Work {
 };
 
 
+// Mixed solves with the update once per chunk / after every iteration, in us at delta = 0.2 | 0.3 |
+// 0.5 | 0.9 (one update every 8 | 6 | 4 | 1 iterations): dual n=16, Lt=16 3320 / 3410 | 3910 / 3460 |
+// 5720 / 3610 | 18930 / 4710; simplicial n=32, Lt=16 3670 / 3320 | 4090 / 3390 | 6230 / 3700 | 15680 /
+// 5040; simplicial n=64, Lt=32 8750 / 9360 | 9590 / 9870 | 11440 / 10970 | 26450 / 19990.
+constexpr double kLooseDelta = 0.25;
+
 template <typename T>
 CGResult run_cg(Dirac& D, Spin<double>* x, const Spin<double>* b, const CGOptions& o) {
   constexpr bool kMixed = std::is_same<T, float>::value;
@@ -238,9 +244,10 @@ CGResult run_cg(Dirac& D, Spin<double>* x, const Spin<double>* b, const CGOption
   // iteration that asks for it makes the rest of the chunk's iterations exit at once.  After
   // every iteration its three kernels and finaliser, idle but for one iteration of a solve
   // (FP64) or of some thirty (mixed), took a quarter of a small lattice's iteration.  With
-  // kernel timing, whose events must each bracket a real iteration, it follows each.
+  // kernel timing, whose events must each bracket a real iteration, it follows each; so it does
+  // where a loose delta asks for an update every few iterations, since the chunk's others then idle.
   EventTimer timer(o.times);
-  const bool ru_each = o.times != nullptr;
+  const bool ru_each = o.times != nullptr || (kMixed && o.delta > kLooseDelta);
   auto reliable_update = [&] {
     if (kMixed)
       hipLaunchKernelGGL(k_flush<T>, dim3(ngate), dim3(256), 0, st, W.xin, n, sc, 0);
@@ -271,7 +278,7 @@ CGResult run_cg(Dirac& D, Spin<double>* x, const Spin<double>* b, const CGOption
   GraphKey key;
   key.add(vin).add(v64).add(hvf).add(hvt).add(hv64f).add(hv64t).add(D.tile<T>(false)).add(D.tile<T>(true));
   key.add(D.tile<double>(false)).add(D.tile<double>(true)).add(W.r).add(W.p).add(W.p2).add(W.w).add(W.xin).add(W.t);
-  key.add(sc).add(gr.partials).add(n).add(nn);
+  key.add(sc).add(gr.partials).add(n).add(nn).add(int(ru_each));
   drive_chunks(one_iter, tail, o, n, st, sc, hsc, &D.graph_slot(kMixed ? 1 : 0), key);
   timer.finish(hsc->iter);
   if (o.times) o.times->ms[2] = o.times->ms[1], o.times->count[2] = o.times->count[1];
