@@ -283,12 +283,14 @@ int qed3_pcg_kernel_times(qed3_ctx* ctx, qed3_precond* pc, void* d_x, const void
  * masses, all on the current device) together, binary16-storage inner iteration (as
  * QED3_SOLVER_CG_HALF) with FP64 reliable updates and the true-residual stop (opts->solver
  * is ignored), time tiles from each context's autotuned shapes.  Each system runs hipGraph
- * chunks of iterations on its own stream, the next queued as soon as the stream has drained;
- * many systems too small to cover the GPU with one launch (< 256 blocks of 256) instead share
- * launches in which every CG phase runs over all of them (per-system scalars and convergence
- * masks, iterations captured in a hipGraph).  A context may be listed several times, once per
- * right-hand side.  The reference runs one CG per right-hand side (PseudoFermion::update_eta,
- * pseudofermion.h:51, looped in integrator.h:156-166).  reps[nsys] may be NULL. */
+ * chunks of iterations on its context's stream, the next queued as soon as the stream has
+ * drained; systems of up to 0.25 M points of six neighbours (0.5 M of three) share launches
+ * instead where that takes less time (many of them, or several on one stream), in which every
+ * CG phase runs over all of them (per-system scalars and convergence masks, iterations captured
+ * in a hipGraph).  A context may be listed several times, once per right-hand side.  Work
+ * queued on the contexts' streams before the call comes first.  The reference runs one CG per
+ * right-hand side (PseudoFermion::update_eta, pseudofermion.h:51, looped in
+ * integrator.h:156-166).  reps[nsys] may be NULL. */
 int qed3_batch_cg(qed3_ctx* const* ctxs, int nsys, void* const* d_x, const void* const* d_b,
                   const qed3_cg_opts* opts, qed3_cg_report* reps);
 

@@ -4,6 +4,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <map>
+#include <set>
 
 #include "batch.hpp"
 #include "cg_epi.hpp"
@@ -15,10 +16,15 @@ namespace {
 using namespace cgepi;
 
 constexpr int kBlock = 256;
-constexpr long kLargeBlocks = 256;  // one block per CU of a 256-CU part
-// Time of an iteration in us: of the batched launches over some systems, and of the same
-// systems' own launches (measured: see batch_cg)
-constexpr double kBatchBase = 80.0, kBatchPerMpoint = 100.0, kOwnPerSystem = 5.3;
+// Time of an iteration in us, from the points (in millions) times the neighbour slots of a system:
+// of its own launches alone on a stream, of its own launches beside two other systems' (about three
+// streams run at once), and its share of the batched launches, which have a base for the first and
+// for the second neighbour count among the systems.  Measured: see batch_cg.  From kLargeSlots on (0.25 M points of six slots) a
+// system's own launches are the faster ones however many share its stream.
+constexpr double kLargeSlots = 1.5;
+constexpr double kAloneBase = 18.0, kAlonePerSlot = 10.0;
+constexpr double kBesideBase = 21.0, kBesidePerSlot = 14.0, kStreamsAtOnce = 3.0;
+constexpr double kBatchBase = 22.0, kBatchBase2 = 34.0, kBatchPerSystem = 1.3, kBatchPerSlot = 20.5;
 
 // One system of the batch: its operator views, LDS halo tables for ranges of kBlock
 // sites, its blocks in the stencil grids and the streaming grids, and its fields.
@@ -223,14 +229,21 @@ std::vector<CGResult> batch_launches(const std::vector<Dirac*>& Ds, const std::v
                                      const std::vector<const Spin<double>*>& bs, const CGOptions& o);
 }  // namespace
 
-// Every system runs the single-system kernels, a chunk of iterations at a time on its own stream
-// (cg_solve_half_many: they run at lower register pressure than the batched kernels, in the
-// temporal gauge, and overlap), except many small ones: the host and the hardware queues take
-// about kOwnPerSystem us an iteration for every system, the batched launches a base and a price
-// per point.  Batched / own launches: 64 of simplicial n=8, Lt=8: 13.2 / 25.7 ms; 32 of dual
-// n=10, Lt=12 and simplicial n=9, Lt=7: 12.4 / 20.1; 64 of simplicial n=16, Lt=16 (2.6 M points):
-// 38.2 / 36.7; 4 of n <= 30: 9.1 / 5.6; 8 of simplicial n=32, Lt=16: 16.4 / 8.6.  A system whose
-// own K1 grid covers the GPU (kLargeBlocks blocks of 256) is never batched.
+// A large system runs the single-system kernels, a chunk of iterations at a time on its own stream
+// (cg_solve_half_many: they run at lower register pressure than the batched kernels, in the temporal
+// gauge, and overlap).  The others do so together, or share the batched launches, by the model above,
+// which does not ask for the launch shapes contexts happen to have: own launches cost a chain for the
+// systems of one stream (a context listed several times, contexts on one caller's stream) and a
+// third of the sum of all, whichever is longer.  Own | batched launches per iteration in us:
+//   4, 8, 24 contexts of simplicial n=8, Lt=8      37 | 34    56 | 41    140 | 76
+//   3, 8, 24 of simplicial n=16, Lt=16             30 | 40    79 | 73    198 | 174
+//   3, 8, 24 of dual n=20, Lt=20                   31 | 66    86 | 141   231 | 424
+//   4, 8 of simplicial n=32, Lt=16                 64 | 91    109 | 175
+//   2, 8 sources on one simplicial n=16, Lt=16     46 | 35    179 | 68
+//   2, 4 sources on one dual n=20, Lt=20           46 | 47    91 | 68
+//   8 contexts of simplicial n=16, Lt=16 on one stream  180 | 73
+// A loose delta's updates leave most of an own chunk idle (kLooseDelta: 4 of simplicial n=16, Lt=16
+// at 0.5 126 | 56), the batched launches update after every iteration.
 std::vector<CGResult> batch_cg(const std::vector<Dirac*>& Ds, const std::vector<Spin<double>*>& xs,
                                const std::vector<const Spin<double>*>& bs, const CGOptions& o) {
   const int ns = int(Ds.size());
@@ -239,32 +252,38 @@ std::vector<CGResult> batch_cg(const std::vector<Dirac*>& Ds, const std::vector<
   for (Dirac* D : Ds)
     if (!D->has_gauge()) throw std::invalid_argument("batch: a system has no gauge field");
   const auto t0 = std::chrono::steady_clock::now();
-  // A context's work fields, scalars and captured chunk hold one solve at a time: the systems of a
-  // context listed several times (several sources on one operator) share launches, whose fields are
-  // a system's own, or take turns on its stream.
-  std::map<const Dirac*, int> seen;
-  std::vector<int> small;
-  bool repeats = false;  // among the small ones
-  std::vector<std::vector<int>> big(1);  // per turn, no context twice in one
+  // A context's work fields, scalars and captured chunk hold one solve at a time, so the systems of
+  // a context listed several times (several sources on one operator) take turns on its stream,
+  // unless they share launches, whose fields are a system's own.
+  auto slots = [&](int k) { return 1e-6 * double(Ds[k]->points()) * Ds[k]->tables().max_nn; };
+  std::map<const Dirac*, size_t> seen;
+  std::vector<size_t> turn(ns);
+  std::vector<int> large, small;
   for (int k = 0; k < ns; k++) {
-    const Dirac& D = *Ds[k];
-    const size_t turn = size_t(seen[Ds[k]]++);
-    const int ts = std::max(1, std::min(D.tile<float>(false).ts, D.Lt()));
-    const long blocks = long((D.V() + kBlock - 1) / kBlock) * ((D.Lt() + ts - 1) / ts);
-    if (big.size() <= turn) big.resize(turn + 1);
-    if (blocks >= kLargeBlocks) {
-      big[turn].push_back(k);
-    } else {
-      small.push_back(k);
-      repeats = repeats || turn > 0;
+    turn[k] = seen[Ds[k]]++;
+    (slots(k) >= kLargeSlots ? large : small).push_back(k);
+  }
+  double longest = 0, beside = 0, batched = 0;
+  std::map<hipStream_t, double> chain;
+  std::set<int> groups;
+  for (int k : small) {
+    longest = std::max(longest, chain[Ds[k]->stream()] += kAloneBase + kAlonePerSlot * slots(k));
+    beside += kBesideBase + kBesidePerSlot * slots(k);
+    batched += kBatchPerSystem + kBatchPerSlot * slots(k);
+    groups.insert(Ds[k]->tables().max_nn);
+  }
+  batched += kBatchBase + (groups.size() > 1 ? kBatchBase2 : 0.0);
+  if (!small.empty()) beside *= std::ceil(double(small.size()) / kStreamsAtOnce) / double(small.size());
+  const bool share = !small.empty() && (o.delta > kLooseDelta || batched < std::max(longest, beside));
+  std::vector<std::vector<int>> own;  // per turn
+  auto on_own = [&](const std::vector<int>& which) {
+    for (int k : which) {
+      if (own.size() <= turn[k]) own.resize(turn[k] + 1);
+      own[turn[k]].push_back(k);
     }
-  }
-  double mpoints = 0;
-  for (int k : small) mpoints += 1e-6 * double(Ds[k]->points());
-  if (!repeats && kOwnPerSystem * double(small.size()) <= kBatchBase + kBatchPerMpoint * mpoints) {
-    big[0].insert(big[0].end(), small.begin(), small.end());
-    small.clear();
-  }
+  };
+  on_own(large);
+  if (!share) on_own(small);
   std::vector<CGResult> out(ns);
   CGOptions os = o;
   os.mixed = os.half = true;
@@ -281,8 +300,8 @@ std::vector<CGResult> batch_cg(const std::vector<Dirac*>& Ds, const std::vector<
     const std::vector<CGResult> r = shared ? batch_launches(d, x, b, o) : cg_solve_half_many(d, x, b, os);
     for (size_t j = 0; j < which.size(); j++) out[which[j]] = r[j];
   };
-  for (const auto& t : big) solve(t, false);
-  solve(small, true);
+  for (const auto& t : own) solve(t, false);
+  if (share) solve(small, true);
   const double secs = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   for (auto& r : out) r.seconds = secs;
   return out;
@@ -298,6 +317,8 @@ std::vector<CGResult> batch_launches(const std::vector<Dirac*>& Ds, const std::v
   for (Dirac* D : Ds)
     if (!D->has_gauge()) throw std::invalid_argument("batch: a system has no gauge field");
   hipStream_t st = Ds[0]->stream();
+  for (Dirac* D : Ds)  // what is queued on the other contexts' streams may write the sources
+    if (D->stream() != st) QED3_HIP(hipStreamSynchronize(D->stream()));
   // Systems are grouped by neighbour count (one kernel instantiation per group, so a
   // trivalent system does not run at the registers of the six-neighbour stencil) and,
   // within a group, ordered by descending time tile, so the longest blocks are dispatched

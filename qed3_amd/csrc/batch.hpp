@@ -1,6 +1,7 @@
 // Batched CG: many independent systems D_k^dag D_k x_k = b_k of different lattices
-// (simplicial/dual, refinement n, Lt) and masses advanced together, one launch per CG
-// phase for the whole batch.  The blocks of a launch are laid out system after system
+// (simplicial/dual, refinement n, Lt) and masses advanced together: the large ones, and small ones
+// where that is faster, each on its context's stream (cg_solve_half_many), the others with one
+// launch per CG phase for all of them.  The blocks of a launch are laid out system after system
 // (each system's count a multiple of 8, so the XCD-aware tile order holds per system);
 // each block finds its system, runs that system's LDS-staged stencil tile (time tile
 // from the system's autotuned shape) and reduces into that system's scalars, so systems

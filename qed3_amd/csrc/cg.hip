@@ -190,12 +190,6 @@ struct Work {
 };
 
 
-// Mixed solves with the update once per chunk / after every iteration, in us at delta = 0.2 | 0.3 |
-// 0.5 | 0.9 (one update every 8 | 6 | 4 | 1 iterations): dual n=16, Lt=16 3320 / 3410 | 3910 / 3460 |
-// 5720 / 3610 | 18930 / 4710; simplicial n=32, Lt=16 3670 / 3320 | 4090 / 3390 | 6230 / 3700 | 15680 /
-// 5040; simplicial n=64, Lt=32 8750 / 9360 | 9590 / 9870 | 11440 / 10970 | 26450 / 19990.
-constexpr double kLooseDelta = 0.25;
-
 template <typename T>
 CGResult run_cg(Dirac& D, Spin<double>* x, const Spin<double>* b, const CGOptions& o) {
   constexpr bool kMixed = std::is_same<T, float>::value;

@@ -67,6 +67,14 @@ CGResult cg_solve(Dirac& D, Spin<double>* x, const Spin<double>* b, const CGOpti
 // ||b - D^dag D x|| / ||b|| in FP64
 double true_residual(Dirac& D, const Spin<double>* x, const Spin<double>* b);
 
+// Above this delta an update is due every few iterations, and a chunk of iterations that waits for
+// its end to run one idles for the rest.
+// Mixed solves with the update once per chunk / after every iteration, in us at delta = 0.2 | 0.3 |
+// 0.5 | 0.9 (one update every 8 | 6 | 4 | 1 iterations): dual n=16, Lt=16 3320 / 3410 | 3910 / 3460 |
+// 5720 / 3610 | 18930 / 4710; simplicial n=32, Lt=16 3670 / 3320 | 4090 / 3390 | 6230 / 3700 | 15680 /
+// 5040; simplicial n=64, Lt=32 8750 / 9360 | 9590 / 9870 | 11440 / 10970 | 26450 / 19990.
+constexpr double kLooseDelta = 0.25;
+
 // The FP64 CG of cg_solve on work memory the caller provides (ws_bytes at ws, at least
 // cg_workspace_bytes(points)), allocating nothing: direct launches instead of a captured
 // graph, scalars read back into host stack memory, and the LDS stencil only where the

@@ -1,5 +1,5 @@
 """Several sources on one context in a batched solve: a context listed more than once, small and
-large (256 blocks of 256 at its time tile), alone and among others."""
+large (always on its own stream), alone and among others."""
 import numpy as np
 import pytest
 
@@ -7,14 +7,14 @@ import qed3_amd as q
 from conftest import rel
 
 TOL = 1e-10
-SMALL, SMALL6, LARGE = (1, 3, 5, 4), (0, 4, 6, 4), (1, 8, 64, 1)  # lattice, n, Lt, slices per block
+SMALL, SMALL6, LARGE = (1, 3, 5, 4), (0, 4, 6, 4), (1, 40, 16, 4)  # lattice, n, Lt, slices per block
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("listed", [
-    [SMALL] * 2, [SMALL6] * 3, [LARGE] * 2, [LARGE] * 3,
+    [SMALL] * 2, [SMALL6] * 3, [LARGE] * 2, [LARGE] * 3, [(1, 8, 64, 1)] * 2,
     [SMALL, LARGE, SMALL6, LARGE, SMALL, SMALL], [SMALL] * 20, [SMALL, SMALL6] * 12 + [LARGE] * 2,
-], ids=["small2", "small3", "large2", "large3", "mixed", "small20", "many"])
+], ids=["small2", "small3", "large2", "large3", "blocks2", "mixed", "small20", "many"])
 def test_each_source_gets_its_own_solution(gpu, listed):
     print("case", listed, flush=True)
     rng = np.random.default_rng(11)
