@@ -301,6 +301,7 @@ void run_layers(Horner& K, bool adj, const Spin<float>* in, Spin<float>* const* 
   Dirac& D = K.dirac();
   const HornerView hv = K.view();
   const DiracView<float> tab = D.view<float>();
+  const HaloView halo = hk::horner_halo(D);
   hipStream_t st = D.stream();
   const int L = K.layers();
   Spin<float>* prev = nullptr;
@@ -309,13 +310,13 @@ void run_layers(Horner& K, bool adj, const Spin<float>* in, Spin<float>* const* 
     const float2 cj = {float(c.real()), float(adj ? -c.imag() : c.imag())};
     Spin<float>* o = keep ? keep[t] : (t == L - 1 ? out : bufs[t & 1]);
     if (t == 0 && adj)
-      hk::launch_horner_layer<true, true>(hv, tab, in, nullptr, o, cj, st);
+      hk::launch_horner_layer<true, true>(hv, tab, halo, in, nullptr, o, cj, st);
     else if (t == 0)
-      hk::launch_horner_layer<false, true>(hv, tab, in, nullptr, o, cj, st);
+      hk::launch_horner_layer<false, true>(hv, tab, halo, in, nullptr, o, cj, st);
     else if (adj)
-      hk::launch_horner_layer<true, false>(hv, tab, in, prev, o, cj, st);
+      hk::launch_horner_layer<true, false>(hv, tab, halo, in, prev, o, cj, st);
     else
-      hk::launch_horner_layer<false, false>(hv, tab, in, prev, o, cj, st);
+      hk::launch_horner_layer<false, false>(hv, tab, halo, in, prev, o, cj, st);
     prev = o;
   }
   QED3_HIP(hipGetLastError());
@@ -368,6 +369,7 @@ double Horner::loss_grad(const Spin<double>* v, const Spin<double>* e, int batch
   const GridReduce gr = D_.reducer();
   const HornerView hv = view();
   const DiracView<float> tab = D_.view<float>();
+  const HaloView halo = hk::horner_halo(D_);
   std::vector<cd> g(p_.count(), cd(0, 0));
   const unsigned nbk = stream_grid(n);
   for (int b = 0; b < batch; b++) {
@@ -383,9 +385,9 @@ double Horner::loss_grad(const Spin<double>* v, const Spin<double>* e, int batch
     for (int t = L - 1; t >= 0; t--) {
       Spin<float>* mo = mu[t & 1];
       if (t == L - 1)
-        hk::launch_horner_layer<true, true>(hv, tab, lam, nullptr, mo, float2{1.f, 0.f}, st);
+        hk::launch_horner_layer<true, true>(hv, tab, halo, lam, nullptr, mo, float2{1.f, 0.f}, st);
       else
-        hk::launch_horner_layer<true, false>(hv, tab, lam, mu[(t + 1) & 1], mo, float2{0.f, 0.f}, st);
+        hk::launch_horner_layer<true, false>(hv, tab, halo, lam, mu[(t + 1) & 1], mo, float2{0.f, 0.f}, st);
       const Spin<float>* gp = t > 0 ? G[t - 1] : nullptr;
       if (NS == 6)
         hipLaunchKernelGGL(k_horner_grad<6>, dim3(nblk), dim3(256), 0, st, hv, tab, pv, mo, gp, int(t > 0), tm, red_);

@@ -4,7 +4,8 @@
 // Under T the spin-up row's recurrence runs forward in time and the spin-down row's backward
 // (the other way round under T^dagger).  Two forms:
 //   FP32 fields in any gauge (the checked apply and the training gradient): a transport pass
-//     y = c v + S_th g over all points, then the two rows' recurrences;
+//     y = c v + S_th g over all points, then the two rows' recurrences; with many sites, both
+//     together, a thread a column;
 //   binary16 fields in the temporal gauge (the solver): the parallel-in-time layer below.
 #pragma once
 #include <type_traits>
@@ -163,6 +164,23 @@ __device__ __forceinline__ float2 cmul_phase(float2 u, float2 c) {  // u c
 #pragma clang fp contract(off)
   return {__builtin_fmaf(u.x, c.x, -(u.y * c.y)), __builtin_fmaf(u.x, c.y, u.y * c.x)};
 }
+// sum_j u_j (m_same g_a + m_flip g_abar)(nb_j), lk < 0: the link is stored the other way round
+template <int NS, class G>
+__device__ __forceinline__ float2 transport_row(const float4 (&hr)[NS], const float2 (&u)[NS], const int (&lk)[NS], const G& g,
+                                                int a) {
+#pragma clang fp contract(off)
+  float2 t = {0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < NS; j++) {
+    float2 uj = u[j];
+    if (lk[j] < 0) uj.y = -uj.y;
+    const Spin<float> gj = g(j);
+    const float2 cm = cadd<float>(cmul_coef({hr[j].x, hr[j].y}, comp(gj, a)),
+                                  cmul_coef({hr[j].z, hr[j].w}, comp(gj, 1 - a)));
+    t = cadd<float>(t, cmul_phase(uj, cm));
+  }
+  return t;
+}
 template <int NS, bool ADJ>
 __global__ __launch_bounds__(256) void k_horner_transport(HornerView hv, DiracView<float> d,
                                                           const Spin<float>* __restrict__ v,
@@ -196,21 +214,10 @@ __global__ __launch_bounds__(256) void k_horner_transport(HornerView hv, DiracVi
       u[j] = uS[lk[j] >= 0 ? lk[j] : ~lk[j]];
       g[j] = gin[sV + nb[j]];
     }
-    auto transport = [&](const float4* hr, int a) -> float2 {
-      float2 t = {0.f, 0.f};
-#pragma unroll
-      for (int j = 0; j < NS; j++) {
-        float2 uj = u[j];
-        if (lk[j] < 0) uj.y = -uj.y;
-        const float2 cm = cadd<float>(cmul_coef({hr[j].x, hr[j].y}, comp(g[j], a)),
-                                      cmul_coef({hr[j].z, hr[j].w}, comp(g[j], 1 - a)));
-        t = cadd<float>(t, cmul_phase(uj, cm));
-      }
-      return t;
-    };
+    auto near = [&](int j) { return g[j]; };
     const Spin<float> vv = v[sV + x];
     float2 yF = cmul_phase(cj, comp(vv, rF)), yB = cmul_phase(cj, comp(vv, rB));
-    const float2 tF = transport(hrF, rF), tB = transport(hrB, rB);
+    const float2 tF = transport_row<NS>(hrF, u, lk, near, rF), tB = transport_row<NS>(hrB, u, lk, near, rB);
     yF.x -= tF.x;
     yF.y -= tF.y;
     yB.x -= tB.x;
@@ -222,37 +229,64 @@ __global__ __launch_bounds__(256) void k_horner_transport(HornerView hv, DiracVi
   }
 }
 
-// The recurrences, one thread per site and spin row: state = (y + kappa_t u^t state) / c_x walked
-// from the row's start to its end, each value written over its y.  The chain is arithmetic only:
-// the loads of the next kRecurDepth slices are issued while this group's are worked through.
-// FIRST (no input field): y = c_j v formed here, without a transport pass or a wrap term.
+// One row's recurrence, state = (y + kappa_t u^t state) / c_x, walked forward (FWD) or backward in
+// time.  A link's phase times v, conjugated for the forward walk:
+template <bool FWD>
+__device__ __forceinline__ float2 recur_hop(float2 u, float2 v) {
+#pragma clang fp contract(off)
+  if constexpr (FWD)
+    return {__builtin_fmaf(u.y, v.y, u.x * v.x), __builtin_fmaf(u.x, v.y, -(u.y * v.x))};
+  else
+    return {__builtin_fmaf(u.x, v.x, -(u.y * v.y)), __builtin_fmaf(v.x, u.y, v.y * u.x)};
+}
+// S holds the time wrap (the link from Lt-1 to 0, which T leaves out): a recurrence starts from
+// bc kappa_t w g(the far end of its walk), w the wrap link's phase
+template <bool FWD>
+__device__ __forceinline__ float2 recur_wrap(float bc, float kt, float2 w, float2 g) {
+#pragma clang fp contract(off)
+  float2 t = recur_hop<FWD>(w, g);
+  if constexpr (FWD) t.x = __builtin_fmaf(w.x, g.x, w.y * g.y);
+  return {bc * kt * t.x, bc * kt * t.y};
+}
+// y of a first layer (no input field)
+__device__ __forceinline__ float2 first_y(float2 cj, float2 v) {
+#pragma clang fp contract(off)
+  return {__builtin_fmaf(cj.x, v.x, -(cj.y * v.y)), __builtin_fmaf(cj.y, v.x, cj.x * v.y)};
+}
+// the state after one slice; at a walk's start (wrap) st is the wrap term, already weighted (0 in a
+// first layer), else the state before, across the link of phase u
+template <bool FWD, bool FIRST>
+__device__ __forceinline__ float2 recur_step(float2 y, float2 u, float2 st, bool wrap, float kt, float invc) {
+#pragma clang fp contract(off)
+  if (!wrap) {
+    const float2 t = recur_hop<FWD>(u, st);
+    if constexpr (FWD && FIRST) {
+      y = {__builtin_fmaf(kt, t.x, y.x), __builtin_fmaf(kt, t.y, y.y)};
+    } else {
+      const float2 w = {kt * t.x, kt * t.y};
+      y = {y.x + w.x, y.y + w.y};
+    }
+  } else {
+    y = {y.x + st.x, y.y + st.y};
+  }
+  return {invc * y.x, invc * y.y};
+}
+
+// The recurrences, one thread per site and spin row, each value written over its y.  The chain is
+// arithmetic only: the loads of the next kRecurDepth slices are issued while this group's are worked
+// through.  FIRST (no input field): y = c_j v formed here, without a transport pass or a wrap term.
 constexpr int kRecurDepth = 8;
 template <bool FWD, bool FIRST>
 __device__ __forceinline__ void horner_recur_walk(const HornerView& hv, const DiracView<float>& d, const Spin<float>* in,
                                                   const Spin<float>* __restrict__ gin, Spin<float>* out, float2 cj,
                                                   int x, int row) {
-#pragma clang fp contract(off)  // the roundings are spelled out: FP32 results do not depend on the code around them
   const int V = hv.V, Lt = hv.Lt;
   const float invc = hv.invc[x], kt = hv.kt[x];
   auto at = [&](int k) { return size_t(FWD ? k : Lt - 1 - k) * V + x; };
   // component `row` of the point, as two floats
   auto half = [&](const Spin<float>* p, size_t i) { return reinterpret_cast<const float2*>(p)[2 * i + row]; };
-  // a link's phase times v, conjugated for the forward walk
-  auto hop = [](float2 u, float2 v) {
-    if constexpr (FWD)
-      return float2{__builtin_fmaf(u.y, v.y, u.x * v.x), __builtin_fmaf(u.x, v.y, -(u.y * v.x))};
-    else
-      return float2{__builtin_fmaf(u.x, v.x, -(u.y * v.y)), __builtin_fmaf(v.x, u.y, v.y * u.x)};
-  };
   float2 st = {0.f, 0.f};
-  if constexpr (!FIRST) {
-    // S holds the time wrap (the link from Lt-1 to 0, which T leaves out): each recurrence
-    // starts from bc kappa_t w g(the far end of its walk), w the wrap link's phase
-    const float2 w = d.uT[size_t(Lt - 1) * V + x], g = half(gin, at(Lt - 1));
-    float2 t = hop(w, g);
-    if constexpr (FWD) t.x = __builtin_fmaf(w.x, g.x, w.y * g.y);
-    st = {d.bc * kt * t.x, d.bc * kt * t.y};
-  }
+  if constexpr (!FIRST) st = recur_wrap<FWD>(d.bc, kt, d.uT[size_t(Lt - 1) * V + x], half(gin, at(Lt - 1)));
   struct Group {
     float2 y[kRecurDepth], u[kRecurDepth];
   };
@@ -272,22 +306,8 @@ __device__ __forceinline__ void horner_recur_walk(const HornerView& hv, const Di
     for (int j = 0; j < kRecurDepth; j++) {
       const int k = k0 + j;
       if (k < Lt) {
-        float2 y = cur.y[j];
-        if constexpr (FIRST)
-          y = {__builtin_fmaf(cj.x, y.x, -(cj.y * y.y)), __builtin_fmaf(cj.y, y.x, cj.x * y.y)};
-        if (k > 0) {
-          const float2 t = hop(cur.u[j], st);
-          if constexpr (FWD && FIRST) {
-            y = {__builtin_fmaf(kt, t.x, y.x), __builtin_fmaf(kt, t.y, y.y)};
-          } else {
-            const float2 w = {kt * t.x, kt * t.y};
-            y = {y.x + w.x, y.y + w.y};
-          }
-        } else {
-          y.x += st.x;  // the wrap term, already weighted (0 in a first layer)
-          y.y += st.y;
-        }
-        st = {invc * y.x, invc * y.y};
+        const float2 y = FIRST ? first_y(cj, cur.y[j]) : cur.y[j];
+        st = recur_step<FWD, FIRST>(y, cur.u[j], st, k == 0, kt, invc);
         reinterpret_cast<float2*>(out)[2 * at(k) + row] = st;
       }
     }
@@ -309,16 +329,161 @@ __global__ __launch_bounds__(256) void k_horner_recur(HornerView hv, DiracView<f
     horner_recur_walk<false, FIRST>(hv, d, in, gin, out, cj, x, row);
 }
 
-// One layer of K (ADJ: of K^dagger) on FP32 fields: gout = T^{-1}(c_j v + S_th gin)
+// The layer with one thread a column: a block owns a range of sites.  Pass 1, forward in time: per
+// slice the block stages g_in of its range and halo in LDS (two tiles in turn, one barrier a slice),
+// every thread forms both rows' transports, steps the forward row and stores its state beside the
+// other row's y.  Pass 2, backward in time: every thread reads its own column back and steps the
+// other row.  Both passes move whole points, 120 B a point on three slots; the transport pass and the
+// recurrences by rows move 150 (half points, both rows' lines fetched twice), but over all points at
+// once.  So this form where the columns fill the GPU; the roundings are the same.
+template <int NS, bool ADJ, bool FIRST>
+__global__ __launch_bounds__(256) void k_horner_column(HornerView hv, DiracView<float> d, HaloView halo,
+                                                       const Spin<float>* __restrict__ v,
+                                                       const Spin<float>* __restrict__ gin,
+                                                       Spin<float>* __restrict__ gout, float2 cj, TileMap tm) {
+#pragma clang fp contract(off)
+  extern __shared__ unsigned char column_raw[];
+  float4* tile = reinterpret_cast<float4*>(column_raw);  // [2][R + hmax], points
+  int xr, st_;
+  tile_of(tm, blockIdx.x, xr, st_);
+  if (xr >= tm.nxr) return;  // uniform
+  const int V = hv.V, Lt = hv.Lt, R = blockDim.x;
+  const int x = xr * R + int(threadIdx.x);
+  const bool act = x < V;
+  constexpr int rF = ADJ ? 1 : 0, rB = 1 - rF;
+  const int h0 = FIRST ? 0 : halo.halo_off[xr], nh = FIRST ? 0 : halo.halo_off[xr + 1] - h0;
+  const int hid0 = int(threadIdx.x) < nh ? halo.halo[h0 + threadIdx.x] : -1;
+  const int hid1 = int(threadIdx.x) + R < nh ? halo.halo[h0 + threadIdx.x + R] : -1;
+  int nb[NS], lk[NS];
+  float4 hrF[NS], hrB[NS];
+  float invc = 0.f, kt = 0.f;
+  float2 stF = {0.f, 0.f}, stB = {0.f, 0.f};
+  if (act) {
+    invc = hv.invc[x];
+    kt = hv.kt[x];
+    if constexpr (!FIRST) {
+      const size_t mF = size_t((ADJ ? 2 : 0) + rF) * NS * V, mB = size_t((ADJ ? 2 : 0) + rB) * NS * V;
+#pragma unroll
+      for (int j = 0; j < NS; j++) {
+        nb[j] = halo.nbl[size_t(j) * V + x];
+        lk[j] = d.lnk[size_t(j) * V + x];
+        hrF[j] = hv.hrow[mF + size_t(j) * V + x];
+        hrB[j] = hv.hrow[mB + size_t(j) * V + x];
+      }
+      const size_t end = size_t(Lt - 1) * V + x;
+      const float2 w = d.uT[end];
+      stF = recur_wrap<true>(d.bc, kt, w, comp(gin[end], rF));
+      stB = recur_wrap<false>(d.bc, kt, w, comp(gin[x], rB));
+    }
+  }
+  struct Loads {
+    Spin<float> v, gc, gh0, gh1;
+    float2 u[NS], ut;  // ut: the temporal link s-1 -> s
+  };
+  auto load = [&](int s, Loads& L) {
+    const size_t sV = size_t(s) * V;
+    if (act) {
+      L.v = v[sV + x];
+      if (s > 0) L.ut = d.uT[sV - V + x];
+      if constexpr (!FIRST) {
+        const float2* uS = d.uS + size_t(s) * d.E;
+#pragma unroll
+        for (int j = 0; j < NS; j++) L.u[j] = uS[lk[j] >= 0 ? lk[j] : ~lk[j]];
+        L.gc = gin[sV + x];
+      }
+    }
+    if constexpr (!FIRST) {
+      if (hid0 >= 0) L.gh0 = gin[sV + hid0];
+      if (hid1 >= 0) L.gh1 = gin[sV + hid1];
+    }
+  };
+  Loads cur, nxt;
+  load(0, cur);
+  for (int s = 0; s < Lt; s++) {
+    if (s + 1 < Lt) load(s + 1, nxt);  // a slice ahead: in flight during this slice's work
+    float4* tb = tile + (s & 1) * (R + halo.hmax);
+    if constexpr (!FIRST) {
+      auto quad = [](const Spin<float>& p) { return float4{p.a.x, p.a.y, p.b.x, p.b.y}; };
+      if (act) tb[threadIdx.x] = quad(cur.gc);
+      if (hid0 >= 0) tb[R + threadIdx.x] = quad(cur.gh0);
+      if (hid1 >= 0) tb[2 * R + threadIdx.x] = quad(cur.gh1);
+      for (int k = int(threadIdx.x) + 2 * R; k < nh; k += R) tb[R + k] = quad(gin[size_t(s) * V + halo.halo[h0 + k]]);
+      __syncthreads();
+    }
+    if (act) {
+      float2 yF, yB;
+      if constexpr (FIRST) {
+        yF = first_y(cj, comp(cur.v, rF));
+        yB = first_y(cj, comp(cur.v, rB));
+      } else {
+        auto near = [&](int j) {
+          const float4 p = tb[nb[j]];
+          return Spin<float>{{p.x, p.y}, {p.z, p.w}};
+        };
+        yF = cmul_phase(cj, comp(cur.v, rF));
+        yB = cmul_phase(cj, comp(cur.v, rB));
+        const float2 tF = transport_row<NS>(hrF, cur.u, lk, near, rF), tB = transport_row<NS>(hrB, cur.u, lk, near, rB);
+        yF.x -= tF.x;
+        yF.y -= tF.y;
+        yB.x -= tB.x;
+        yB.y -= tB.y;
+      }
+      stF = recur_step<true, FIRST>(yF, cur.ut, stF, s == 0, kt, invc);
+      if constexpr (rF == 0)
+        put(gout + size_t(s) * V + x, stF, yB);
+      else
+        put(gout + size_t(s) * V + x, yB, stF);
+    }
+    cur = nxt;
+  }
+  if (!act) return;
+  Spin<float> t = gout[size_t(Lt - 1) * V + x], tn = t;
+  float2 u{};
+  for (int s = Lt - 1; s >= 0; s--) {
+    const size_t i = size_t(s) * V + x;
+    if (s > 0) tn = gout[i - V];
+    if (s < Lt - 1) u = d.uT[i];  // the link s -> s+1
+    const float2 gF = comp(t, rF);
+    stB = recur_step<false, FIRST>(comp(t, rB), u, stB, s == Lt - 1, kt, invc);
+    if constexpr (rF == 0)
+      put(gout + i, gF, stB);
+    else
+      put(gout + i, stB, gF);
+    t = tn;
+  }
+}
+
+// One layer of K (ADJ: of K^dagger) on FP32 fields: gout = T^{-1}(c_j v + S_th gin).  By columns from
+// kColumnSites sites on, where a thread a column is more than a wave per SIMD; halo: of ranges of 256
+// sites, needed there (horner_halo).  Application of four layers by rows / by columns in us, sites in
+// thousands: dual n=60, Lt=64 (72) 567 / 669; simplicial n=90, Lt=64 (81) 744 / 757; dual n=64, Lt=32
+// (82) 281 / 298; dual n=66, Lt=20 (87) 207 / 188; simplicial n=96, Lt=32 (92) 417 / 371; dual n=68,
+// Lt=64 (92) 702 / 744; simplicial n=128, Lt=64 (164) 1539 / 1172; dual n=128, Lt=64 (328) 2664 / 2175,
+// a training step there 6312 / 5353.
+constexpr int kColumnSites = 88000;
+inline HaloView horner_halo(Dirac& D) { return D.V() >= kColumnSites ? D.halo(256) : HaloView{}; }
 template <bool ADJ, bool FIRST>
-inline void launch_horner_layer(const HornerView& hv, const DiracView<float>& tables, const Spin<float>* v,
-                                const Spin<float>* gin, Spin<float>* gout, float2 cj, hipStream_t st) {
+inline void launch_horner_layer(const HornerView& hv, const DiracView<float>& tables, const HaloView& halo,
+                                const Spin<float>* v, const Spin<float>* gin, Spin<float>* gout, float2 cj,
+                                hipStream_t st) {
+  TileMap tm;
+  tm.nxr = (hv.V + 255) / 256;
+  tm.nxr_pad = (tm.nxr + 7) / 8 * 8;
+  tm.remap = 1;
+  if (hv.V >= kColumnSites) {
+    tm.nst = 1;
+    const dim3 grid{unsigned(tm.nxr_pad)};
+    const size_t smem = FIRST ? 0 : size_t(2) * (256 + halo.hmax) * sizeof(Spin<float>);
+    if (hv.nslot == 6)
+      hipLaunchKernelGGL((k_horner_column<6, ADJ, FIRST>), grid, dim3(256), smem, st, hv, tables, halo, v, gin, gout, cj,
+                         tm);
+    else
+      hipLaunchKernelGGL((k_horner_column<3, ADJ, FIRST>), grid, dim3(256), smem, st, hv, tables, halo, v, gin, gout, cj,
+                         tm);
+    return;
+  }
   if constexpr (!FIRST) {
-    TileMap tm;
-    tm.nxr = (hv.V + 255) / 256;
-    tm.nxr_pad = (tm.nxr + 7) / 8 * 8;
     tm.nst = (hv.Lt + kTransportSlices - 1) / kTransportSlices;
-    tm.remap = 1;
     const dim3 grid(unsigned(tm.nxr_pad) * unsigned(tm.nst));
     if (hv.nslot == 6)
       hipLaunchKernelGGL((k_horner_transport<6, ADJ>), grid, dim3(256), 0, st, hv, tables, v, gin, gout, cj, tm);
