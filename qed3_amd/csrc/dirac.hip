@@ -486,9 +486,10 @@ void* Dirac::scratch(int slot, size_t bytes) {
   return scratch_[slot];
 }
 
-void Dirac::release_scratch() {
+void Dirac::release_scratch(int slot) {
   QED3_HIP(hipStreamSynchronize(stream_));
   for (int i = 0; i < kScratchSlots; i++) {
+    if (slot >= 0 && i != slot) continue;
     if (scratch_[i]) QED3_HIP(hipFree(scratch_[i]));
     scratch_[i] = nullptr;
     scratch_bytes_[i] = 0;

@@ -244,7 +244,7 @@ class Dirac {
   // calls on one context are sequential.
   static constexpr int kScratchSlots = 15;
   void* scratch(int slot, size_t bytes);
-  void release_scratch();
+  void release_scratch(int slot = -1);  // of one slot, or all
   // the kept chunk graphs of the solvers on this context (0 FP64, 1 mixed, 2 half storage,
   // 3 multi-shift)
   static constexpr int kGraphSlots = 4;
