@@ -310,6 +310,13 @@ int qed3_pf_action(qed3_ctx* ctx, const void* d_phi, const void* d_eta, double* 
  * arrays in the gauge layout: d_fs[Lt][E], d_ft[Lt][V]. */
 int qed3_pf_force(qed3_ctx* ctx, const void* d_eta, double* d_fs, double* d_ft);
 
+/* f_l (+)= c (Re <u1, dD/dtheta_l v1> + Re <u2, dD/dtheta_l v2>) for every link, the building block
+ * of the pseudofermion and overlap forces (complex double fields; u2, v2 may both be NULL; f is
+ * overwritten if init).  form: 0 as the forces choose by the lattice's size, 1 a thread per link,
+ * 2 a thread per site (for checking the two kernels). */
+int qed3_force_bilinear(qed3_ctx* ctx, const void* d_u1, const void* d_v1, const void* d_u2, const void* d_v2,
+                        double c, int init, int form, double* d_fs, double* d_ft);
+
 /* ---- gauge action and HMC (host FP64 over the GPU fermion path) --------------------
  * U(1) plaquette action on the context's lattice with beta_s = at/(vol_f g^2) per face
  * and beta_t = 2 vol_l/(at ell_l^2 g^2) per temporal plaquette (action_ext.h:150-159):

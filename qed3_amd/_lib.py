@@ -110,6 +110,7 @@ SIGNATURES = {
     "qed3_fcg": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.POINTER(CGOpts),
                            C.POINTER(CGReport), c_int_p, c_int_p]),
     "qed3_pf_force": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
+    "qed3_force_bilinear": (C.c_int, [C.c_void_p] * 5 + [C.c_double, C.c_int, C.c_int, C.c_void_p, C.c_void_p]),
     "qed3_gauge_action": (C.c_int, [C.c_void_p, C.c_double, C.c_int, c_double_p, c_double_p,
                                     c_double_p, c_double_p, c_double_p]),
     "qed3_hmc_create": (C.c_int, [C.c_void_p, C.c_void_p, C.POINTER(C.c_void_p)]),

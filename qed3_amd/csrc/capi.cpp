@@ -820,6 +820,21 @@ int qed3_pf_force(qed3_ctx* ctx, const void* d_eta, double* d_fs, double* d_ft) 
   });
 }
 
+int qed3_force_bilinear(qed3_ctx* ctx, const void* d_u1, const void* d_v1, const void* d_u2, const void* d_v2,
+                        double c, int init, int form, double* d_fs, double* d_ft) {
+  if (!ctx || !d_u1 || !d_v1 || !d_fs || !d_ft) return fail(QED3_ERR_ARG, "null argument");
+  if (!d_u2 != !d_v2) return fail(QED3_ERR_ARG, "second pair incomplete");
+  if (form < 0 || form > 2) return fail(QED3_ERR_ARG, "form must be 0, 1 or 2");
+  if (!ctx->D->has_gauge()) return fail(QED3_ERR_STATE, "no gauge field set");
+  return guarded([&]() -> int {
+    using S = const qed3::Spin<double>*;
+    ctx->D->force_bilinear(static_cast<S>(d_u1), static_cast<S>(d_v1), static_cast<S>(d_u2), static_cast<S>(d_v2), c,
+                           init != 0, d_fs, d_ft, static_cast<qed3::ForceForm>(form));
+    QED3_HIP(hipStreamSynchronize(ctx->D->stream()));
+    return QED3_OK;
+  });
+}
+
 int qed3_gauge_action(qed3_ctx* ctx, double gsq, int compact, const double* spatial,
                       const double* temporal, double* S, double* fs, double* ft) {
   if (!ctx || !spatial || !temporal) return fail(QED3_ERR_ARG, "null argument");

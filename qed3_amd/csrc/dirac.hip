@@ -809,8 +809,9 @@ void Dirac::dot(const Spin<double>* x, const Spin<double>* y, double* re, double
 // By sites: slices per thread, the more the less often a site's hop rows are read (0.3 KB on six
 // slots), but at least four waves a SIMD; sites per block, the D stencil's range, whose halo
 // tables are there, or the largest whose tiles (two spinors a pair) fit in LDS.
-void Dirac::launch_force(const ForcePairs& F, int npairs, double c, bool init, double* fs, double* ft) {
-  if (points() < size_t(1) << 21) {
+void Dirac::launch_force(const ForcePairs& F, int npairs, double c, bool init, double* fs, double* ft,
+                         ForceForm form) {
+  if (form == ForceForm::kLinks || (form == ForceForm::kBySize && points() < size_t(1) << 21)) {
     const size_t n = size_t(h_.Lt) * (h_.E + h_.V);
     hipLaunchKernelGGL(k_force_links, dim3(unsigned((n + 255) / 256)), dim3(256), 0, stream_, view<double>(),
                        reinterpret_cast<const int4*>(link_ends_), F, c, init ? 1 : 0, fs, ft);
@@ -851,14 +852,14 @@ void Dirac::launch_force(const ForcePairs& F, int npairs, double c, bool init, d
 void Dirac::force(const Spin<double>* eta, double* fs, double* ft) {
   if (!tmp64_) tmp64_ = dalloc<Spin<double>>(points());
   apply<double>(false, tmp64_, eta, false);  // precalc: w = D eta
-  launch_force(ForcePairs{{tmp64_, nullptr}, {eta, nullptr}}, 1, -2.0, true, fs, ft);
+  launch_force(ForcePairs{{tmp64_, nullptr}, {eta, nullptr}}, 1, -2.0, true, fs, ft, ForceForm::kBySize);
   QED3_HIP(hipStreamSynchronize(stream_));
 }
 
 void Dirac::force_bilinear(const Spin<double>* u1, const Spin<double>* v1, const Spin<double>* u2,
-                           const Spin<double>* v2, double c, bool init, double* fs, double* ft) {
+                           const Spin<double>* v2, double c, bool init, double* fs, double* ft, ForceForm form) {
   if ((u2 == nullptr) != (v2 == nullptr)) throw std::invalid_argument("force_bilinear: second pair incomplete");
-  launch_force(ForcePairs{{u1, u2}, {v1, v2}}, u2 ? 2 : 1, c, init, fs, ft);
+  launch_force(ForcePairs{{u1, u2}, {v1, v2}}, u2 ? 2 : 1, c, init, fs, ft, form);
 }
 
 double Dirac::time_apply(bool dag, int prec, int warmup, int reps) {

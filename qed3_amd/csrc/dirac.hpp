@@ -166,6 +166,9 @@ class GraphKey {
   }
 };
 
+// Which force kernel runs: by the lattice's size, or one of the two (for checking them)
+enum class ForceForm { kBySize = 0, kLinks = 1, kSites = 2 };
+
 // Pairs (u_k, v_k) whose derivative terms a force sums
 struct ForcePairs {
   const Spin<double>* u[2];
@@ -231,7 +234,8 @@ class Dirac {
   // force layout (spatial [Lt][E], temporal [Lt][V]); (u2, v2) may both be null; f is
   // overwritten when init.  Asynchronous on the context's stream.
   void force_bilinear(const Spin<double>* u1, const Spin<double>* v1, const Spin<double>* u2,
-                      const Spin<double>* v2, double c, bool init, double* fs, double* ft);
+                      const Spin<double>* v2, double c, bool init, double* fs, double* ft,
+                      ForceForm form = ForceForm::kBySize);
 
   // ms per launch of one D or D^dag apply; prec 0 FP64, 1 FP32, 2 binary16 storage
   double time_apply(bool dag, int prec, int warmup, int reps);
@@ -275,7 +279,7 @@ class Dirac {
   template <typename T>
   void tune_one(bool dag);
   // f (+)= c times the sum over npairs (1 or 2) pairs, for every link
-  void launch_force(const ForcePairs& F, int npairs, double c, bool init, double* fs, double* ft);
+  void launch_force(const ForcePairs& F, int npairs, double c, bool init, double* fs, double* ft, ForceForm form);
 
   HopTables h_;
   int bc_ = 0;
