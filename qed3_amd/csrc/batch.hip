@@ -17,14 +17,28 @@ using namespace cgepi;
 
 constexpr int kBlock = 256;
 // Time of an iteration in us, from the points (in millions) times the neighbour slots of a system:
-// of its own launches alone on a stream, of its own launches beside two other systems' (about three
-// streams run at once), and its share of the batched launches, which have a base for the first and
-// for the second neighbour count among the systems.  Measured: see batch_cg.  From kLargeSlots on (0.25 M points of six slots) a
-// system's own launches are the faster ones however many share its stream.
+// of its own launches alone on a stream and beside two other systems' (about three streams run at
+// once).  The batched launches have a base for the first and for the second neighbour count among the
+// systems; a system adds to it by its slots, or by its points where its threads take four slices or
+// more.  Measured: see batch_cg.  From kLargeSlots on (0.25 M points of six slots) a system's own
+// launches are the faster ones however many share its stream.
 constexpr double kLargeSlots = 1.5;
 constexpr double kAloneBase = 18.0, kAlonePerSlot = 10.0;
 constexpr double kBesideBase = 21.0, kBesidePerSlot = 14.0, kStreamsAtOnce = 3.0;
-constexpr double kBatchBase = 22.0, kBatchBase2 = 34.0, kBatchPerSystem = 1.3, kBatchPerSlot = 20.5;
+constexpr double kBatchBase = 22.0, kBatchBase2 = 34.0;
+constexpr double kBatchPerSystem = 1.3, kBatchPerSlot = 20.5;
+constexpr double kBatchPerMpoint6 = 100.0, kBatchPerMpoint3 = 75.0;
+
+// Slices per thread of a system in the batched launches over `points` in all: its tuned shape's, or
+// by default one while the launches leave the GPU mostly empty, then four (the default shape suits a
+// context's own launches).  One | four slices, in ms: 8 of simplicial n=8, Lt=8 (0.04 M points) 3.3 |
+// 4.3, 24 (0.12 M) 6.3 | 6.4, 40 (0.2 M) 9.4 | 9.1; simplicial n=16, Lt=16: 4 (0.16 M) 4.0 | 4.6,
+// 8 (0.33 M) 6.6 | 5.7, 24 (1 M) 15.7 | 12.0.
+constexpr size_t kFewPoints = 200000;
+int batch_ts(const Dirac& D, bool f64, size_t points) {
+  const int ts = !D.tuned() ? (points < kFewPoints ? 1 : 4) : f64 ? D.tile<double>(false).ts : D.tile<float>(false).ts;
+  return std::max(1, std::min(ts, D.Lt()));
+}
 
 // One system of the batch: its operator views, LDS halo tables for ranges of kBlock
 // sites, its blocks in the stencil grids and the streaming grids, and its fields.
@@ -231,10 +245,10 @@ std::vector<CGResult> batch_launches(const std::vector<Dirac*>& Ds, const std::v
 
 // A large system runs the single-system kernels, a chunk of iterations at a time on its own stream
 // (cg_solve_half_many: they run at lower register pressure than the batched kernels, in the temporal
-// gauge, and overlap).  The others do so together, or share the batched launches, by the model above,
-// which does not ask for the launch shapes contexts happen to have: own launches cost a chain for the
-// systems of one stream (a context listed several times, contexts on one caller's stream) and a
-// third of the sum of all, whichever is longer.  Own | batched launches per iteration in us:
+// gauge, and overlap).  The others do so together, or share the batched launches, by the model above:
+// own launches cost a chain for the systems of one stream (a context listed several times, contexts
+// on one caller's stream) and a third of the sum of all, whichever is longer.  Own | batched launches
+// per iteration in us (tuned shapes, one or two slices a thread):
 //   4, 8, 24 contexts of simplicial n=8, Lt=8      37 | 34    56 | 41    140 | 76
 //   3, 8, 24 of simplicial n=16, Lt=16             30 | 40    79 | 73    198 | 174
 //   3, 8, 24 of dual n=20, Lt=20                   31 | 66    86 | 141   231 | 424
@@ -242,6 +256,10 @@ std::vector<CGResult> batch_launches(const std::vector<Dirac*>& Ds, const std::v
 //   2, 8 sources on one simplicial n=16, Lt=16     46 | 35    179 | 68
 //   2, 4 sources on one dual n=20, Lt=20           46 | 47    91 | 68
 //   8 contexts of simplicial n=16, Lt=16 on one stream  180 | 73
+// and with the default shape, four slices a thread:
+//   8, 24 contexts of simplicial n=16, Lt=16       81 | 64    206 | 134
+//   8, 24 of simplicial n=24, Lt=12                88 | 75    229 | 190
+//   8, 24 of dual n=20, Lt=20                      85 | 123   223 | 345
 // A loose delta's updates leave most of an own chunk idle (kLooseDelta: 4 of simplicial n=16, Lt=16
 // at 0.5 126 | 56), the batched launches update after every iteration.
 std::vector<CGResult> batch_cg(const std::vector<Dirac*>& Ds, const std::vector<Spin<double>*>& xs,
@@ -263,14 +281,19 @@ std::vector<CGResult> batch_cg(const std::vector<Dirac*>& Ds, const std::vector<
     turn[k] = seen[Ds[k]]++;
     (slots(k) >= kLargeSlots ? large : small).push_back(k);
   }
+  size_t points = 0;
+  for (int k : small) points += Ds[k]->points();
   double longest = 0, beside = 0, batched = 0;
   std::map<hipStream_t, double> chain;
   std::set<int> groups;
   for (int k : small) {
     longest = std::max(longest, chain[Ds[k]->stream()] += kAloneBase + kAlonePerSlot * slots(k));
     beside += kBesideBase + kBesidePerSlot * slots(k);
-    batched += kBatchPerSystem + kBatchPerSlot * slots(k);
-    groups.insert(Ds[k]->tables().max_nn);
+    const int nn = Ds[k]->tables().max_nn;
+    batched += batch_ts(*Ds[k], false, points) < 4
+                   ? kBatchPerSystem + kBatchPerSlot * slots(k)
+                   : (nn == 6 ? kBatchPerMpoint6 : kBatchPerMpoint3) * 1e-6 * double(Ds[k]->points());
+    groups.insert(nn);
   }
   batched += kBatchBase + (groups.size() > 1 ? kBatchBase2 : 0.0);
   if (!small.empty()) beside *= std::ceil(double(small.size()) / kStreamsAtOnce) / double(small.size());
@@ -323,9 +346,9 @@ std::vector<CGResult> batch_launches(const std::vector<Dirac*>& Ds, const std::v
   // trivalent system does not run at the registers of the six-neighbour stencil) and,
   // within a group, ordered by descending time tile, so the longest blocks are dispatched
   // first and the grid's tail is short.
-  auto ts_of = [](const Dirac& D, bool f64) {
-    return std::max(1, std::min(f64 ? D.tile<double>(false).ts : D.tile<float>(false).ts, D.Lt()));
-  };
+  size_t points = 0;
+  for (const Dirac* D : Ds) points += D->points();
+  auto ts_of = [&](const Dirac& D, bool f64) { return batch_ts(D, f64, points); };
   std::vector<int> order(ns);
   for (int k = 0; k < ns; k++) order[k] = k;
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) {

@@ -7,14 +7,14 @@ import qed3_amd as q
 from conftest import rel
 
 TOL = 1e-10
-SMALL, SMALL6, LARGE = (1, 3, 5, 4), (0, 4, 6, 4), (1, 40, 16, 4)  # lattice, n, Lt, slices per block
+SMALL, SMALL6, LARGE = (1, 3, 5, 4), (0, 4, 6, 4), (1, 40, 16, 4)  # lattice, n, Lt, slices per block (0: default shape)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("listed", [
-    [SMALL] * 2, [SMALL6] * 3, [LARGE] * 2, [LARGE] * 3, [(1, 8, 64, 1)] * 2,
+    [SMALL] * 2, [SMALL6] * 3, [LARGE] * 2, [LARGE] * 3, [(1, 8, 64, 1)] * 2, [(0, 16, 16, 0), (1, 15, 13, 0)] * 4,
     [SMALL, LARGE, SMALL6, LARGE, SMALL, SMALL], [SMALL] * 20, [SMALL, SMALL6] * 12 + [LARGE] * 2,
-], ids=["small2", "small3", "large2", "large3", "blocks2", "mixed", "small20", "many"])
+], ids=["small2", "small3", "large2", "large3", "blocks2", "default8", "mixed", "small20", "many"])
 def test_each_source_gets_its_own_solution(gpu, listed):
     print("case", listed, flush=True)
     rng = np.random.default_rng(11)
@@ -23,7 +23,8 @@ def test_each_source_gets_its_own_solution(gpu, listed):
         if (lat, n, Lt) not in ctx:
             D = ctx[lat, n, Lt] = q.WilsonDirac(lat, n, Lt, r=1.0, M5=0.1, at=0.3)
             D.update(rng.vonmises(0.0, 1.4, (Lt, D.E)), rng.vonmises(0.0, 1.4, (Lt, D.V)))
-            D.set_tile(256, ts, 1, 0)
+            if ts:
+                D.set_tile(256, ts, 1, 0)
     ops = [ctx[s[:3]] for s in listed]
     bs = [rng.normal(size=D.N) + 1j * rng.normal(size=D.N) for D in ops]
     d_b = [q.DeviceArray.from_numpy(b) for b in bs]
